@@ -94,6 +94,10 @@ KERNEL_BYTES = {
     # fewer bytes)
     "r4_momflux": (160, 16),
     "r5_nodes": (136, 124),
+    # the remap on the tiling (with the tile step): the face mass fluxes --
+    # ielnd, packed neighbours and faces 32, cnwt 32, rho 8; writes 32 | x, y,
+    # mesh velocity 32 -- and the rest of it (remap_tile, tile_bytes)
+    "remap_faces": (104, 32),
     # node relaxation sweeps: stencil table 32, x, y 16, writes 16 | the last
     # sweep also reads the Lagrangian x, y 16
     "relax_sweep": (0, 64),
@@ -143,11 +147,24 @@ FOLD_BYTES = {"f4_state": (0.125, 16)}
 #    cache: not counted.
 #  f1_seg (F1 of a fresh run call's first step): per entry 8 and per element
 #    ielnd 16, cs2 8, the at-rest byte written 1 | x, y, u, v 32.
-TILE_KERNELS = ("lag_tile", "f1_seg")
+#  remap_tile (after the tile step of an ALE step, which then also writes
+#    REMAP_F4_BYTES an element): per entry its element id and node slots 8,
+#    node ids 16, neighbour entries 4; per element once the packed neighbours
+#    16, face mass fluxes 32, corner masses 32, e, V, m 24, ielmat 4; m,
+#    corner masses, rho, e, p, cs2 and the at-rest byte written 73 | per node
+#    its list entry, entries and orders 12, x, y, u, v, mesh velocity 48,
+#    indtype 4; x, y, u, v written 32.  The far nodes of a direction with a
+#    flux come through the cache.
+TILE_KERNELS = ("lag_tile", "f1_seg", "remap_tile")
 
 
-def tile_bytes(k, nel, nnd, moving, zeroed, tiles):
+def tile_bytes(k, nel, nnd, moving, zeroed, tiles, remap):
     ntile, _, nent = tiles
+    if k == "remap_tile":
+        return 28 * nent + 181 * nel + 96 * nnd + 16 * ntile
+    if k == "lag_tile" and remap:
+        return (24 * nent + (97 + REMAP_F4_BYTES) * nel + 89 * nnd + 16 * ntile + 64 * moving +
+                72 * zeroed)
     if k == "lag_tile":
         # (per node: its entry's corner-mask byte; per tile: its bounds)
         return 24 * nent + 98 * nel + 89 * nnd + 16 * ntile + 64 * moving + 72 * zeroed
@@ -164,7 +181,7 @@ def kernel_bytes(k, nel, nnd, moving, zeroed, fold=False, tiles=None, remap=Fals
     per-step averages of bl_run_stats; tiles = (tiles, boundary elements,
     entries) of the tile step; remap: the step ends with the remap"""
     if k in TILE_KERNELS:
-        return tile_bytes(k, nel, nnd, moving, zeroed, tiles)
+        return tile_bytes(k, nel, nnd, moving, zeroed, tiles, remap)
     if k in ("f1_limiter", "e1_limiter"):
         return LIMITER_BYTES[0] * moving + LIMITER_BYTES[1] * nnd * min(1.0, moving / nel)
     be, bn = KERNEL_BYTES[k]
@@ -429,7 +446,7 @@ def main():
     fold = tiles is not None or (f1name in kern and "f4_state" in kern and
                                  kern[f1name]["launches"] < kern["f4_state"]["launches"])
     priced = set(KERNEL_BYTES) | (set(TILE_KERNELS) if tiles else set())
-    remap = "r1_volflux" in kern
+    remap = "r1_volflux" in kern or "remap_tile" in kern
     dom = max((k for k in kern if k in priced), key=lambda k: kern[k]["total_ms"],
               default=None)
     roof = None

@@ -71,6 +71,32 @@ __device__ __forceinline__ void fluxelvl_regs(int e, int id1, int id2, const int
   }
 }
 
+// fluxelvl_regs over both face pairs with the element's own corner basis cbo
+// and value rv in registers
+__device__ __forceinline__ void fluxelvl_own(const int nb[4], const int fc[4],
+                                             const double cbo[4], const double* __restrict__ cb,
+                                             const double fd4[4], double rv,
+                                             const double* __restrict__ var, double out[4]) {
+  // the neighbours' corners on the shared faces and their values: every
+  // load before the arithmetic
+  double c0[4], c1[4], vn[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    c0[i] = cb[4 * nb[i] + fc[i]];
+    c1[i] = cb[4 * nb[i] + ((fc[i] + 1) & 3)];
+    vn[i] = var[nb[i]];
+  }
+#pragma unroll
+  for (int i1 = 0; i1 < 2; ++i1) {
+    const int i2 = i1 + 2;
+    const double r3 = cbo[i2] + cbo[(i2 + 1) & 3];
+    const double w5 = r3 + c0[i2] + c1[i2];
+    const double r4 = cbo[i1] + cbo[i1 + 1];
+    const double w6 = r4 + c0[i1] + c1[i1];
+    fluxel_pair(r3, w5, r4, w6, rv, vn[i2], vn[i1], fd4[i1], fd4[i2], out[i1], out[i2]);
+  }
+}
+
 // ale_kn_sumflux for one element with its own face values and the matching
 // face values of its neighbours in registers (nbv[i]: the neighbour across
 // face i, ignored at a boundary face)

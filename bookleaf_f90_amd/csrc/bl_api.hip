@@ -676,7 +676,8 @@ int bl_destroy(bl_handle_t* h) {
                   h->d_diag_hist, h->d_diag_count, h->d_diag_part, h->d_ring, h->d_work, h->d_rest, h->d_vstats,
                   h->d_rlist, h->d_zlist, h->d_lflag, h->d_lmark, h->d_ld1, h->d_nbfc, h->d_cw[0], h->d_cw[1],
                   h->d_eoff, h->d_lboff, h->d_einst, h->d_ninst, h->d_inst, h->d_inst_dt, h->d_cnt,
-                  h->d_epart, h->d_eparti, h->d_ehist};
+                  h->d_epart, h->d_eparti, h->d_ehist, h->cm_other, h->mesh_w[0], h->mesh_w[1],
+                  h->d_cpe};
   for (void* p : bufs) if (p) hipFree(p);
   for (double* p : h->d_tmp) if (p) hipFree(p);
   for (double* p : h->cterm) if (p) hipFree(p);

@@ -132,6 +132,13 @@ struct FusedArgs {
   const uint8_t* tile_ncm;  // per tile node: bit jj, the node is corner jj of an element
   const int2* tile_el;
   const int4* tile_nd;  // the entry's four nodes (0-based), beside tile_el
+  // the tiled remap: of an own element's entry, the entries of its four face
+  // neighbours (one byte each); of a tile node, the entries around it by its
+  // corner in them (one byte each), and in y the corners in the order of the
+  // ALE sums (2 bits each), in element order (2 bits each from bit 8), and
+  // their count (from bit 16)
+  const int32_t* tile_nbr;
+  const int2* tile_ninc;
   const uint8_t* rest8;
   const uint8_t* rest8_prev;
   uint8_t* rest8_next;

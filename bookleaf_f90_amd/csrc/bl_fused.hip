@@ -31,7 +31,8 @@
 //                kernel per tile of elements and the ring around them
 //                (k_lag_tile, bl_tiles.hip)
 //   R1..R5     : the remap (ale_dr_*), after the Lagrangian step when ALE is
-//                active
+//                active; on a tiling the Lagrangian part is the tile step and
+//                the remap two kernels (k_remap_faces, k_remap_tile)
 //
 // Every FP64 expression is the same function of the same inputs as in the
 // per-driver path (bl_math.h), so the results are bit-identical to the
@@ -367,6 +368,15 @@ __host__ __device__ inline void step_end(DevTimestep* ts, const DtResult* res) {
     ts->err_step = ts->nstep;
     return;
   }
+  if (ts->ale_tile && !res->negvol2) {
+    // the remap put the step's state back into the set it started from
+    ts->cmflips = ts->cmflips + 1;
+    if (res->negvol3) {
+      ts->err = 1; ts->err_idx = -res->negvol3; ts->done = 1; ts->skip = 1;
+      ts->err_step = ts->nstep;
+    }
+    return;
+  }
   ts->flips = ts->flips + 1;
   if (res->negvol2) {
     ts->err = 1; ts->err_idx = -res->negvol2; ts->done = 1; ts->skip = 1;
@@ -388,7 +398,8 @@ k_f1_limiter(FusedArgs A, FusedNodes N, int nb1) {
   if (step_skipped(A, A.ts)) return;
   // the step before found a negative volume that F1b has not recorded yet:
   // this step does nothing (F1b makes it so)
-  if (A.end_in_f1b && (A.dtres->negvol || A.dtres->negvol2)) return;
+  // (one group of loads: tested one by one each would wait for the last)
+  if (A.end_in_f1b && (A.dtres->negvol | A.dtres->negvol2 | A.dtres->negvol3)) return;
   __shared__ int32_t list[kScanPer * kBlock];
   __shared__ uint32_t wave_n[kBlock / 64];
   double best = DBL_MAX, dv = -1.0;
@@ -493,8 +504,10 @@ __global__ void __launch_bounds__(kFinalBlock) k_f1b_select(FusedArgs A, int nb,
   if (threadIdx.x == 0) {
     if (skip) ts->done = 1;
     ts->skip = skip ? 1 : 0;
+    ts->bad = 0;
     A.dtres->negvol = 0;
     A.dtres->negvol2 = 0;
+    A.dtres->negvol3 = 0;
     if (A.end_in_f1b && !skip) ts->open = 1;
   }
   if (skip) return;
@@ -726,10 +739,12 @@ __device__ __forceinline__ bool ens_pending(const FusedArgs& A, const DevTimeste
 // force (kept in rcpscratch21/22 for F4), and the cell's corrector corner
 // force replaced by the frvolume average of the component forces.
 // Component energies are not saved and restored between predictor and
-// corrector (hydro_dr_set.f90 copies elenergy only).
+// corrector (hydro_dr_set.f90 copies elenergy only): they go to ce_out.  With
+// write false nothing is stored (a tile's ring copy of the cell).
 __device__ __forceinline__ void mix_f2(const FusedArgs& A, int imx, const Iso& g,
                                       const Iso& gh, const double u[4], const double v[4],
-                                      double h, double fx[4], double fy[4]) {
+                                      double h, double* ce_out, bool write, double fx[4],
+                                      double fy[4]) {
   const MixArgs& M = A.mx;
   int icp = M.imxfcp[imx] - 1;
   const int n = M.imxncp[imx];
@@ -741,15 +756,17 @@ __device__ __forceinline__ void mix_f2(const FusedArgs& A, int imx, const Iso& g
 #pragma unroll
     for (int j = 0; j < 4; ++j) { cu[j] = f * u[j]; cv[j] = f * v[j]; }
     const double ce = energy_update(M.cpenergy[icp], cm, cfx, cfy, cu, cv, h, A.zerocut);
-    M.cpenergy[icp] = ce;
+    if (write) ce_out[icp] = ce;
     const double crho = cm / (gh.vol * f);
     int cmat = M.icpmat[icp];
     cmat = cmat > 0 ? cmat : 0;
     const double cph = eos_pressure(A.eos_itype[cmat], A.eos_param + BL_NEOSPARAM * cmat, crho,
                                     ce, A.pcut);
     mix_force(M, icp, cph, gh.a1, gh.a3, gh.b1, gh.b3, cfx, cfy);
-    st4c(M.cpfx, icp, cfx);
-    st4c(M.cpfy, icp, cfy);
+    if (write) {
+      st4c(M.cpfx, icp, cfx);
+      st4c(M.cpfy, icp, cfy);
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) { w1[j] = w1[j] + f * cfx[j]; w2[j] = w2[j] + f * cfy[j]; }
   }
@@ -758,10 +775,11 @@ __device__ __forceinline__ void mix_f2(const FusedArgs& A, int imx, const Iso& g
 }
 
 // component terms of a mixed cell in F4: corrector geometry (the cell's iso
-// terms at x^{n+1}), volume, density, energy with cpu = frvolume*ubar
-// corners, EOS
+// terms at x^{n+1}), volume, density, energy (ce_in: after the predictor)
+// with cpu = frvolume*ubar corners, EOS
 __device__ __forceinline__ void mix_f4(const FusedArgs& A, int imx, const Iso& g,
-                                      const double ub[4], const double vb[4], double dt) {
+                                      const double ub[4], const double vb[4], double dt,
+                                      const double* ce_in) {
   const MixArgs& M = A.mx;
   int icp = M.imxfcp[imx] - 1;
   const int n = M.imxncp[imx];
@@ -777,7 +795,7 @@ __device__ __forceinline__ void mix_f4(const FusedArgs& A, int imx, const Iso& g
     for (int j = 0; j < 4; ++j) { cu[j] = f * ub[j]; cv[j] = f * vb[j]; }
     ld4c(M.cpfx, icp, cfx);
     ld4c(M.cpfy, icp, cfy);
-    const double ce = energy_update(M.cpenergy[icp], cm, cfx, cfy, cu, cv, dt, A.zerocut);
+    const double ce = energy_update(ce_in[icp], cm, cfx, cfy, cu, cv, dt, A.zerocut);
     M.cpenergy[icp] = ce;
     int cmat = M.icpmat[icp];
     cmat = cmat > 0 ? cmat : 0;
@@ -794,10 +812,11 @@ __device__ __forceinline__ void mix_f4(const FusedArgs& A, int imx, const Iso& g
 // does, then the component terms, whose frvolume average is the cell's
 // force.  Nothing else F2 reads or writes is touched, so the two run side by
 // side.
-__device__ __forceinline__ void f2_mix_cell(const FusedArgs& A, const FusedNodes& N,
-                                            const DevTimestep* ts, int imx) {
+__device__ __forceinline__ void f2_mix_force(const FusedArgs& A, const FusedNodes& N, double dt,
+                                             int imx, double* ce_out, bool write, double fx[4],
+                                             double fy[4]) {
   const int e = A.mx.imxel[imx] - 1;
-  const double h = 0.5 * ts->dt;
+  const double h = 0.5 * dt;
   int nd[4];
   load_nd(A.ielnd, e, nd);
   double x[4], y[4], u[4], v[4], xh[4], yh[4];
@@ -807,8 +826,13 @@ __device__ __forceinline__ void f2_mix_cell(const FusedArgs& A, const FusedNodes
   Iso g, gh;
   getiso(x, y, g);
   getiso(xh, yh, gh);
+  mix_f2(A, imx, g, gh, u, v, h, ce_out, write, fx, fy);
+}
+__device__ __forceinline__ void f2_mix_cell(const FusedArgs& A, const FusedNodes& N,
+                                            const DevTimestep* ts, int imx) {
+  const int e = A.mx.imxel[imx] - 1;
   double fx[4], fy[4];
-  mix_f2(A, imx, g, gh, u, v, h, fx, fy);
+  f2_mix_force(A, N, ts->dt, imx, A.mx.cpenergy, true, fx, fy);
   const int nel = A.nel;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -821,7 +845,8 @@ __device__ __forceinline__ void f2_mix_cell(const FusedArgs& A, const FusedNodes
 // corrector state of a mixed cell (F4 writes only the cell's own fields,
 // which this does not read)
 __device__ __forceinline__ void f4_mix_cell(const FusedArgs& A, const FusedNodes& O,
-                                            const DevTimestep* ts, int imx) {
+                                            const DevTimestep* ts, int imx,
+                                            const double* ce_in) {
   const int e = A.mx.imxel[imx] - 1;
   int nd[4];
   load_nd(A.ielnd, e, nd);
@@ -829,7 +854,7 @@ __device__ __forceinline__ void f4_mix_cell(const FusedArgs& A, const FusedNodes
   load4(O.x, nd, x); load4(O.y, nd, y); load4(A.ubar, nd, ub); load4(A.vbar, nd, vb);
   Iso g;
   getiso(x, y, g);
-  mix_f4(A, imx, g, ub, vb, ts->dt);
+  mix_f4(A, imx, g, ub, vb, ts->dt, ce_in);
 }
 
 // ---------------------------------------------------------------- F2
@@ -916,7 +941,10 @@ __device__ __forceinline__ void f2_element(const FusedArgs& A, const FusedNodes&
     wt[j] = gh.wt[j];
   }
   // last: no load of the element passes this atomic
-  if (check_volume && gh.vol < 0.0) atomicMax(&A.dtres->negvol, e + 1);
+  if (check_volume && gh.vol < 0.0) {
+    atomicMax(&A.dtres->negvol, e + 1);
+    A.ts->bad = 1;
+  }
 }
 
 // the zero viscosity of an element at rest now but not in the step before
@@ -1078,7 +1106,10 @@ __device__ __forceinline__ double f4_state_from(const FusedArgs& A, int e, doubl
     A.vol[e] = g.vol;
   }
   // last: no load of the element passes this atomic
-  if (g.vol < 0.0) atomicMax(&A.dtres->negvol2, e + 1);
+  if (g.vol < 0.0) {
+    atomicMax(&A.dtres->negvol2, e + 1);
+    A.ts->bad = 1;
+  }
   return c2;
 }
 __device__ __forceinline__ double f4_state_of(const FusedArgs& A, int e, double dt,
@@ -1211,7 +1242,11 @@ __device__ __forceinline__ void seg_collect(const FusedArgs& A, int seg, int nse
                        A.parti + 2 * nseg + seg);
 }
 
+// ALE: a remap follows (k_remap_tile), which does the next step's F1 terms;
+// the corner weights and the volume at x^{n+1} are written for it.  MIX: mixed
+// cells take their components' force.
 // (three waves per SIMD: at most 168 VGPRs; LDS allows three workgroups)
+template <bool ALE, bool MIX>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3)))
 k_lag_tile(FusedArgs A, FusedNodes N, FusedNodesOut O, EnsArgs E) {
   // slot-fastest, so that a wave's lanes of one (quantity, corner) are
@@ -1273,6 +1308,22 @@ k_lag_tile(FusedArgs A, FusedNodes N, FusedNodesOut O, EnsArgs E) {
         acc[3][j][sl] = fy[j];
       }
     }
+    if (MIX) {
+      // a mixed cell's force: its components' (after the pure cells' terms
+      // are in LDS, which frees their registers)
+      const int im = A.ielmat[e];
+      if (im < 0) {
+        f2_mix_force(A, N, dt, -im - 1, A.mx.cpe, writer, fx, fy);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t sl = (slots >> (8 * j)) & 0xFFu;
+          if (sl != kNoSlot) {
+            acc[2][j][sl] = fx[j];
+            acc[3][j][sl] = fy[j];
+          }
+        }
+      }
+    }
     if (writer) {
       // the batch's last step leaves the corner forces in rscratch23/24
       // (lagstep cnfx/cnfy)
@@ -1306,7 +1357,8 @@ k_lag_tile(FusedArgs A, FusedNodes N, FusedNodesOut O, EnsArgs E) {
   // the EOS and region tables of those (their loads overlap F3; the index
   // loads arrive with the node values F3 waits for)
   el_eos(A, emat, ein);
-  const CflIn cin = cfl_of_region(A, ereg - 1);
+  CflIn cin{0, 0};
+  if (!ALE) cin = cfl_of_region(A, ereg - 1);
   // --- F3: the tile's nodes, their corners in jj order
   if (own) {
     double m = 0.0, a = 0.0, fu = 0.0, fv = 0.0;
@@ -1350,9 +1402,12 @@ k_lag_tile(FusedArgs A, FusedNodes N, FusedNodesOut O, EnsArgs E) {
     Iso g;
     const double c2 =
         f4_state_from(A, e, dt, ein.m, ein.en, ein.et, ein.p, x, y, ub, vb, fx, fy, g);
-    f1_terms(A, e, x, y, u, v, g, c2, cin, moving, cflv, divv);
-    A.rest8_next[e] = moving ? 0 : 1;
+    if (!ALE) {
+      f1_terms(A, e, x, y, u, v, g, c2, cin, moving, cflv, divv);
+      A.rest8_next[e] = moving ? 0 : 1;
+    }
   }
+  if (ALE) return;
   // an ensemble's next-step limiter reads its instance's worklist
   if (A.einst) ens_list(A, E, inst, tid & 63, interior && moving, e);
   seg_collect(A, t, A.nseg, interior, e, cflv, divv);
@@ -1595,7 +1650,7 @@ __global__ void __launch_bounds__(kBlock) k_r4(AleArgs B, FusedArgs A, FusedNode
     if (A.ts->skip) return;
     const int imx = (int)blockIdx.x * kBlock + threadIdx.x;
     if (imx >= A.mx.nmx) return;
-    f4_mix_cell(A, O, A.ts, imx);
+    f4_mix_cell(A, O, A.ts, imx, A.mx.cpenergy);
     if (fold7 && A.ts->ale_on && !A.dtres->negvol) {
       int nd[4];
       load_nd(A.ielnd, A.mx.imxel[imx] - 1, nd);
@@ -1682,6 +1737,308 @@ __global__ void __launch_bounds__(kBlock) k_r5(AleArgs B, DevTimestep* tsw) {
   B.v[n] = v;
 }
 
+// -------------------------------------------------- the remap on the tiles
+// With a tiling (bl_tiles.hip) an ALE step is F1L, F1b, the tile step, the
+// mesh motion (node relaxation only), k_remap_faces and k_remap_tile.  The
+// face mass fluxes need the neighbours' state at x^{n+1} and everything
+// after them the neighbours' fluxes, so the remap takes two passes: the
+// fluxes of every element, then per tile all the rest (R2 to R5 and the next
+// step's F1 terms) over the tile's own elements and the ring around their
+// nodes, whose corner terms stay in LDS.  The tile step's node and element
+// sets alternate inside the step: the remap reads the sets the tile step
+// wrote and writes back to the sets the step started from; the corner masses
+// (read by the tiles around an element while its own tile rewrites them)
+// alternate between two arrays from step to step.  The arithmetic is R1's to
+// R5's, in their order.
+//
+// Against F1 to F4 and R1 to R5 in eleven kernels, per step: two-material
+// Eulerian Sod 2048x256 with mixed cells 240 -> 146 us, Eulerian Sedov 401^2
+// 105 -> 64 us, Eulerian Sod 100x25 58 -> 37 us, EQUI relaxation 1024x512
+// 309 -> 203 us: the corner terms, fluxes and corner masses that went through
+// HBM between the kernels (about 900 B an element) stay in LDS, and F1 needs
+// no pass of its own.  Bound by latency: three workgroups a CU (45 KB of LDS,
+// at most 168 VGPRs) of dependent gathers and divisions.  A tiling is used
+// wherever the mesh has one; the eleven kernels remain for meshes without.
+
+#define REMAP_TILE_GATE(T) \
+  if ((T)->skip || (T)->bad) return
+
+// R1's face mass fluxes (and a negative volume of the moved mesh, which R3
+// finds in the five-kernel form)
+__global__ void __launch_bounds__(kBlock) k_remap_faces(AleArgs B) {
+  REMAP_TILE_GATE(B.ts);
+  if (!B.ts->ale_on) return;
+  const int e = xcd_index();
+  if (e >= B.nel) return;
+  int nd[4];
+  load_nd(B.ielnd, e, nd);
+  const NbFc c = load_nbfc_packed(e, B.nbfc);
+  double cw[4];
+  ld4(B.cnwt, e, cw);
+  const double rho = B.rho[e];
+  double ax[4], ay[4], bx[4], by[4], own[4], nbv[4];
+  remap_faces(B, nd, B.ts->dt, ax, ay, bx, by, own, nbv);
+  double f[4];
+  fluxelvl_own(c.nb, c.fc, cw, B.cnwt, own, rho, B.rho, f);
+  st4(B.fcdm, e, f);
+  Iso g;
+  getiso(bx, by, g);
+  if (g.vol < 0.0) atomicMax(&B.dtres->negvol3, e + 1);
+}
+
+// The corner momentum fluxes of one element for u and v (fluxndvl_uv) from
+// its corner masses cm, its corner mass flux cd of each direction and the
+// outer-node table: the neighbour's corner beyond the shared face is the
+// limiter's far node (the tables agree on the meshes that have one).  A
+// direction without flux reads nothing.
+__device__ __forceinline__ void fluxndvl_outer(const FusedArgs& A, const FusedNodes& H, int e,
+                                               const int nd[4], const NbFc& c,
+                                               const double* __restrict__ cb,
+                                               const double cm[4], const double cd[2],
+                                               double ou[4], double ov[4]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) { ou[j] = 0.0; ov[j] = 0.0; }
+  const bool any = cd[0] > 0.0 || cd[0] < 0.0 || cd[1] > 0.0 || cd[1] < 0.0;
+  if (!any) return;
+  double u[4], v[4];
+  load4(H.u, nd, u);
+  load4(H.v, nd, v);
+  const int4* o4 = reinterpret_cast<const int4*>(A.outer);
+#pragma unroll
+  for (int l = 0; l < 2; ++l) {
+    const int lr = l + 2;
+    const bool left = cd[l] > 0.0, right = cd[l] < 0.0;
+    double du[2] = {0.0, 0.0}, dv[2] = {0.0, 0.0};
+    if (left || right) {
+      const int4 o = o4[2 * e + l];
+      const int f = left ? c.fc[l] : c.fc[lr], nb = left ? c.nb[l] : c.nb[lr];
+      const int n0 = (left ? o.x : o.z) - 1, n1 = (left ? o.y : o.w) - 1;
+      const double un[2] = {H.u[n0], H.u[n1]}, vn[2] = {H.v[n0], H.v[n1]};
+      const double b0 = cb[4 * nb + f], b1 = cb[4 * nb + ((f + 1) & 3)],
+                   b2 = cb[4 * nb + ((f + 2) & 3)], b3 = cb[4 * nb + ((f + 3) & 3)];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {  // icn = k + 1
+        const int jl = l + k, jr = (lr + 1 - k) & 3;  // the two corners along the direction
+        const double w5 = cm[jl] + cm[jr];
+        if (left) {
+          const double rd = cm[jl] - 0.5 * cd[l];
+          const double w6 = k == 0 ? b2 + b1 : b3 + b0;
+          du[k] = fluxnd_left(cd[l], rd, w5, w6, u[jl], un[k], u[jr]);
+          dv[k] = fluxnd_left(cd[l], rd, w5, w6, v[jl], vn[k], v[jr]);
+        } else {
+          const double rd = cm[jr] + 0.5 * cd[l];
+          const double w6 = k == 0 ? b0 + b3 : b1 + b2;
+          du[k] = fluxnd_right(cd[l], rd, w5, w6, u[jr], u[jl], un[k]);
+          dv[k] = fluxnd_right(cd[l], rd, w5, w6, v[jr], v[jl], vn[k]);
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int jl = l + k, jr = (lr + 1 - k) & 3;
+      ou[jl] = ou[jl] - du[k];
+      ou[jr] = ou[jr] + du[k];
+      ov[jl] = ov[jl] - dv[k];
+      ov[jr] = ov[jr] + dv[k];
+    }
+  }
+}
+
+// R2 to R5 and the next step's F1 terms, one workgroup per tile.  Phase A,
+// one thread per own or ring element: the face energy fluxes, the corner mass
+// flux and the corner momentum fluxes, to LDS by (corner, entry).  Phase B,
+// one thread per tile node: the node sums in the reference's two orders
+// (A.tile_ninc), the remapped velocity and position, to LDS and, by the one
+// tile that writes the node, to the home node set W.  Phase C, one thread per
+// own element: mass, energy, corner masses, then the hydro update on the
+// moved mesh, the components of a mixed cell and F1's terms.  H: the node set
+// the tile step wrote.  A step outside the ALE time window copies the tile
+// step's state to the home sets and does F1's terms.
+template <bool MIX>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3)))
+k_remap_tile(AleArgs B, FusedArgs A, FusedNodes H, FusedNodesOut W, double* cm_out) {
+  __shared__ double s_cm[4][kTileEls], s_fu[4][kTileEls], s_fv[4][kTileEls], s_ef[4][kTileEls];
+  __shared__ double s_v0[kTileEls], s_fl[kTileEls];
+  __shared__ double nout[4][kTileNodes + 1];  // x, y, u, v after the remap
+  const int t = xcd_block();
+  const int tid = threadIdx.x;
+  const int4 tb = A.tile_bounds[t];
+  const int eb = tb.x, ne = tb.y - tb.x;
+  const int nb0 = tb.z, nn = tb.w - tb.z;
+  const bool node = tid < nn, active = tid < ne;
+  const uint32_t nv = (uint32_t)A.tile_nodes[nb0 + min(tid, nn - 1)];
+  const int2 inc = A.tile_ninc[nb0 + min(tid, nn - 1)];
+  const int2 ent = A.tile_el[eb + min(tid, ne - 1)];
+  const int4 q = A.tile_nd[eb + min(tid, ne - 1)];
+  const uint32_t nbr = (uint32_t)A.tile_nbr[eb + min(tid, ne - 1)];
+  const DevTimestep* ts = A.ts;
+  if (ts->skip) return;
+  const int e = ent.x & 0x3fffffff;
+  const bool own = active && (((uint32_t)ent.x >> 30) & kTileOwn);
+  const uint32_t slots = (uint32_t)ent.y;
+  if (ts->bad) {
+    // a negative volume of the corrector leaves the components after the
+    // predictor (of the predictor: before it)
+    if (MIX && own && !A.dtres->negvol && A.ielmat[e] < 0) {
+      const int imx = -A.ielmat[e] - 1;
+      for (int k = 0, icp = A.mx.imxfcp[imx] - 1; k < A.mx.imxncp[imx]; ++k, ++icp)
+        A.mx.cpenergy[icp] = A.mx.cpe[icp];
+    }
+    return;
+  }
+  const bool on = ts->ale_on != 0;
+  const double dt = ts->dt;
+  const int nd[4] = {q.x, q.y, q.z, q.w};
+  const NbFc c = load_nbfc_packed(e, B.nbfc);
+  // (every thread's entry names an element of the tile)
+  double cm[4], ef[4];
+  ld4(B.cnmass, e, cm);
+  const double en0 = B.en[e], v0 = B.vol[e];
+  double totm = 0.0, fl = 0.0;
+  if (on) {
+    double fm[4], wn[4];
+    ld4(B.fcdm, e, fm);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wn[i] = B.fcdm[4 * c.nb[i] + c.fc[i]];
+    fluxelvl_own(c.nb, c.fc, cm, B.cnmass, fm, en0, B.en, ef);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (c.nb[i] == e) wn[i] = 0.0;
+    double cd[2];
+#pragma unroll
+    for (int i1 = 0; i1 < 2; ++i1) {
+      const int i2 = i1 + 2;
+      totm = totm - fm[i1] - fm[i2] + wn[i1] + wn[i2];
+      const double w1 = wn[i1] - fm[i1];
+      const double w2 = wn[i2] - fm[i2];
+      cd[i1] = 0.25 * (w1 - w2);
+      fl = fl + 0.25 * (w1 + w2);
+    }
+    double ou[4], ov[4];
+    fluxndvl_outer(A, H, e, nd, c, B.cnmass, cm, cd, ou, ov);
+    if (active) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        s_cm[j][tid] = cm[j];
+        s_fu[j][tid] = ou[j];
+        s_fv[j][tid] = ov[j];
+        s_ef[j][tid] = ef[j];
+      }
+      s_v0[tid] = v0;
+      s_fl[tid] = fl;
+    }
+  }
+  // the node's values, and phase C's element inputs, before the barrier
+  const int n = (int)(nv & 0x7fffffffu);
+  const double x0 = H.x[n], y0 = H.y[n], u0 = H.u[n], v0n = H.v[n];
+  double wu = B.ubar[n], wv = B.vbar[n];
+  const int ntype = A.indtype[n];
+  const double m0 = B.mass[e];
+  const int mat = A.ielmat[e];
+  __syncthreads();
+  if (node) {
+    double x1 = x0, y1 = y0, u1 = u0, v1 = v0n;
+    if (on) {
+      // the entries around the node by corner; the two orders of its corners,
+      // 2 bits a place, then the count
+      double nv0 = 0.0, nm0 = 0.0, nm1, su = 0.0, sv = 0.0;
+      const uint32_t by = (uint32_t)inc.x, ord = (uint32_t)inc.y;
+      const int cnt = (int)(ord >> 16);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (k < cnt) {
+          const int j = (int)(ord >> (2 * k)) & 3, en = (int)(by >> (8 * j)) & 0xff;
+          nv0 = nv0 + 0.25 * s_v0[en];
+          nm0 = nm0 + s_cm[j][en];
+        }
+      nm1 = nm0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (k < cnt) {
+          const int j = (int)(ord >> (2 * k)) & 3, en = (int)(by >> (8 * j)) & 0xff;
+          nm1 = nm1 + s_fl[en];
+          const int je = (int)(ord >> (8 + 2 * k)) & 3, ee = (int)(by >> (8 * je)) & 0xff;
+          su = su + s_fu[je][ee];
+          sv = sv + s_fv[je][ee];
+        }
+      const double cutm = B.dencut * nv0;
+      if (ntype != -1 && ntype != -3 && nm1 > cutm) u1 = (u0 * nm0 + su) / nm1;
+      if (ntype != -2 && ntype != -3 && nm1 > cutm) v1 = (v0n * nm0 + sv) / nm1;
+      if (B.zeul) { wu = -wu; wv = -wv; }
+      x1 = x0 + dt * wu;
+      y1 = y0 + dt * wv;
+    }
+    if (nv >> 31) {
+      W.x[n] = x1;
+      W.y[n] = y1;
+      W.u[n] = u1;
+      W.v[n] = v1;
+    }
+    nout[0][tid] = x1;
+    nout[1][tid] = y1;
+    nout[2][tid] = u1;
+    nout[3][tid] = v1;
+  }
+  __syncthreads();
+  double cflv = DBL_MAX, divv = -1.0;
+  bool moving = false;
+  if (own) {
+    double x[4], y[4], u[4], v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t sl = (slots >> (8 * j)) & 0xFFu;
+      x[j] = nout[0][sl];
+      y[j] = nout[1][sl];
+      u[j] = nout[2][sl];
+      v[j] = nout[3][sl];
+    }
+    Iso g;
+    getiso(x, y, g);
+    double c2;
+    if (on) {
+      double s = 0.0;
+#pragma unroll
+      for (int i1 = 0; i1 < 2; ++i1) {
+        const int i2 = i1 + 2;
+        double w1 = s_ef[c.fc[i1]][(nbr >> (8 * i1)) & 0xffu];
+        double w2 = s_ef[c.fc[i2]][(nbr >> (8 * i2)) & 0xffu];
+        if (c.nb[i1] == e) w1 = 0.0;
+        if (c.nb[i2] == e) w2 = 0.0;
+        s = s - ef[i1] - ef[i2] + w1 + w2;
+      }
+      const double m1 = m0 + totm;
+      double en = en0;
+      if (m1 > v0 * B.dencut) en = (en * m0 + s) / m1;
+      B.mass[e] = m1;
+      const double cm1[4] = {cm[0] + fl, cm[1] + fl, cm[2] + fl, cm[3] + fl};
+      st4(cm_out, e, cm1);
+      const double r = m1 / g.vol;
+      ElIn ei;
+      el_eos(A, mat, ei);
+      A.en_o[e] = en;
+      A.rho_o[e] = r;
+      A.pre_o[e] = eos_pressure(ei.et, ei.p, r, en, B.pcut);
+      c2 = eos_cs2(ei.et, ei.p, r, en, B.pcut, B.ccut);
+      A.cs2_o[e] = c2;
+    } else {
+      st4(cm_out, e, cm);
+      A.en_o[e] = en0;
+      A.rho_o[e] = A.rho[e];
+      A.pre_o[e] = A.pre[e];
+      c2 = A.cs2[e];
+      A.cs2_o[e] = c2;
+    }
+    if (MIX && mat < 0) {
+      f4_mix_cell(A, H, ts, -mat - 1, A.mx.cpe);
+      if (on && !A.dtres->negvol3)
+        mix_hydroupdate_iso(A.mx, -mat - 1, g, A.eos_itype, A.eos_param, A.pcut, A.ccut);
+    }
+    f1_terms(A, e, x, y, u, v, g, c2, moving, cflv, divv);
+    A.rest8_next[e] = moving ? 0 : 1;
+  }
+  seg_collect(A, t, A.nseg, own, e, cflv, divv);
+}
+
 // negative volume found by F2 (F3/F4 did not run) or F4 (F3 did): stop the
 // batch at this step; the ALE kernels that follow are gated by skip.
 // Workgroups from 1 on are F4m, one thread per mixed cell: they run when
@@ -1694,7 +2051,7 @@ __global__ void __launch_bounds__(kBlock) k_f5_end(FusedArgs A, FusedNodes O) {
   if (blockIdx.x > 0) {
     if (ts->skip || res->negvol || res->negvol2) return;
     const int imx = ((int)blockIdx.x - 1) * kBlock + threadIdx.x;
-    if (imx < A.mx.nmx) f4_mix_cell(A, O, ts, imx);
+    if (imx < A.mx.nmx) f4_mix_cell(A, O, ts, imx, A.mx.cpenergy);
     return;
   }
   if (threadIdx.x != 0 || ts->skip) return;
@@ -1744,6 +2101,13 @@ __global__ void __launch_bounds__(kBlock) k_f7_aleend(FusedArgs A, const double*
 using namespace bl;
 
 namespace {
+
+// The end of a batch whose last step left its end open (no F1b after it),
+// on the device, so that the host reads the timestep once after all the
+// call's work
+__global__ void k_batch_end(DevTimestep* ts, const DtResult* res) {
+  if (threadIdx.x == 0) step_end(ts, res);
+}
 
 FusedArgs make_args(bl_handle_t* h) {
   FusedArgs A{};
@@ -1845,15 +2209,31 @@ bool use_tiles(const bl_handle_t* h) {
   return fold_f1(h) && h->tiles_on && h->tile_state == 1;
 }
 
+// an ALE step that can run on the tiling: unsplit advection with a mesh
+// motion of its own
+bool ale_on_tiles(const bl_handle_t* h) {
+  return h->cfg.zexist && h->cfg.adv_type == 1 && h->ens_n == 0 &&
+         (h->cfg.zeul || h->relax_type != BL_RELAX_OFF);
+}
+
+// and does: the tile step, then k_remap_faces and k_remap_tile
+bool ale_tiles(const bl_handle_t* h) {
+  return ale_on_tiles(h) && h->tiles_on && h->tile_state == 1 && h->d_tile_nbr;
+}
+
+// the next step's F1 terms come from the step before: a run call starts with
+// one F1 pass
+bool folded(const bl_handle_t* h) { return fold_f1(h) || ale_tiles(h); }
+
 // an ensemble's step on the tiling (tiles within instances): F5 still ends
 // each step, and E1's terms go to the tiles' slots and the worklists
 bool ens_tiles(const bl_handle_t* h) {
   return h->ens_n > 0 && h->tiles_on && h->tile_state == 1;
 }
 
-// the tile step's arguments for a step from node and element set p: it
-// reads element set p and writes set 1 - p
-void tile_args(bl_handle_t* h, FusedArgs& A, int p) {
+// the tile step's arguments for a step of parity p (its at-rest bytes) from
+// element set s: it reads element set s and writes set 1 - s
+void tile_args(bl_handle_t* h, FusedArgs& A, int p, int s) {
   const int nel = h->sz.nel;
   A.ntile = h->ntile;
   A.nseg = h->ntile;
@@ -1864,9 +2244,11 @@ void tile_args(bl_handle_t* h, FusedArgs& A, int p) {
   A.tile_ncm = h->d_tile_ncm;
   A.tile_el = h->d_tile_el;
   A.tile_nd = h->d_tile_nd;
-  A.rho = h->elset[p][0]; A.en = h->elset[p][1]; A.pre = h->elset[p][2]; A.cs2 = h->elset[p][3];
-  A.rho_o = h->elset[1 - p][0]; A.en_o = h->elset[1 - p][1];
-  A.pre_o = h->elset[1 - p][2]; A.cs2_o = h->elset[1 - p][3];
+  A.tile_nbr = h->d_tile_nbr;
+  A.tile_ninc = h->d_tile_ninc;
+  A.rho = h->elset[s][0]; A.en = h->elset[s][1]; A.pre = h->elset[s][2]; A.cs2 = h->elset[s][3];
+  A.rho_o = h->elset[1 - s][0]; A.en_o = h->elset[1 - s][1];
+  A.pre_o = h->elset[1 - s][2]; A.cs2_o = h->elset[1 - s][3];
   A.rest8 = h->d_rest8 + (size_t)p * nel;
   A.rest8_prev = h->d_rest8 + (size_t)(1 - p) * nel;
   A.rest8_next = h->d_rest8 + (size_t)(1 - p) * nel;
@@ -1881,15 +2263,17 @@ void rest_masks(bl_handle_t* h, uint64_t* m[2]) {
   m[1] = h->d_rest + 4 * (size_t)nblocks(std::max(h->sz.nel, 1));
 }
 
-// the first F1 of a folded run call, on node set p, outside the step graphs
+// the first F1 of a folded run call, on the current node set (p: the parity
+// of its first step), outside the step graphs
 int launch_f1_prologue(bl_handle_t* h, int p, int stop_at_time_end) {
   FusedArgs A = make_args(h);
   A.stop_at_time_end = stop_at_time_end;
   A.time_end = h->cfg.time_end;
-  if (use_tiles(h)) {
-    tile_args(h, A, p);
+  if (use_tiles(h) || ale_tiles(h)) {
+    const int s = h->cur_set;
+    tile_args(h, A, p, s);
     A.rest8_next = h->d_rest8 + (size_t)p * h->sz.nel;  // the first step's own bytes
-    FusedNodes N{h->nodeset[p][0], h->nodeset[p][1], h->nodeset[p][2], h->nodeset[p][3]};
+    FusedNodes N{h->nodeset[s][0], h->nodeset[s][1], h->nodeset[s][2], h->nodeset[s][3]};
     BL_LAUNCH(h, "f1_seg", k_f1_seg, (unsigned)h->ntile, kBlock, A, N, EnsArgs{});
     return BL_SUCCESS;
   }
@@ -1902,8 +2286,62 @@ int launch_f1_prologue(bl_handle_t* h, int p, int stop_at_time_end) {
   return BL_SUCCESS;
 }
 
+// one ALE step on the tiling (parity p: its at-rest bytes, and corner masses
+// p -> 1 - p; the node and element sets start and end at the current one)
+int launch_ale_step(bl_handle_t* h, int p, int stop_at_time_end) {
+  FusedArgs A = make_args(h);
+  A.stop_at_time_end = stop_at_time_end;
+  A.time_end = h->cfg.time_end;
+  const int s = h->cur_set;
+  double* const cm[2] = {h->R(BL_CNMASS), h->cm_other};
+  FusedNodes N{h->nodeset[s][0], h->nodeset[s][1], h->nodeset[s][2], h->nodeset[s][3]};
+  FusedNodesOut O{h->nodeset[1 - s][0], h->nodeset[1 - s][1], h->nodeset[1 - s][2],
+                  h->nodeset[1 - s][3]};
+  tile_args(h, A, p, s);
+  A.cnmass = cm[p];
+  const unsigned nseg = (unsigned)A.nseg;
+  const unsigned nbl = std::min(nseg, (unsigned)h->tune_lim_grid);
+  BL_LAUNCH(h, "f1_limiter", k_f1_limiter, nbl, (unsigned)h->tune_lim_block, A, N, (int)nseg);
+  BL_LAUNCH(h, "f1b_select", k_f1b_select, 1, kF1bThreads, A, (int)nseg, (int)nbl);
+  if (A.mx.ncp > 0)
+    BL_LAUNCH(h, "lag_tile", (k_lag_tile<true, true>), (unsigned)h->ntile, kBlock, A, N, O,
+              EnsArgs{});
+  else
+    BL_LAUNCH(h, "lag_tile", (k_lag_tile<true, false>), (unsigned)h->ntile, kBlock, A, N, O,
+              EnsArgs{});
+  AleArgs B = make_ale(h, O);
+  // node relaxation: the mesh velocity in buffers of its own (the components'
+  // energies read the step's ubar after it)
+  if (!h->cfg.zeul) {
+    if (mesh_motion(h, O.x, O.y, h->mesh_w[0], h->mesh_w[1], 0.0, h->d_ts)) return BL_FAILURE;
+    B.ubar = h->mesh_w[0];
+    B.vbar = h->mesh_w[1];
+  }
+  // the remap reads the sets the tile step wrote and writes the start's
+  FusedArgs R = A;
+  R.rho = A.rho_o; R.en = A.en_o; R.pre = A.pre_o; R.cs2 = A.cs2_o;
+  R.rho_o = A.rho; R.en_o = A.en; R.pre_o = A.pre; R.cs2_o = A.cs2;
+  B.rho = R.rho;
+  B.en = R.en;
+  B.cnmass = cm[p];
+  FusedNodes H{O.x, O.y, O.u, O.v};
+  FusedNodesOut W{h->nodeset[s][0], h->nodeset[s][1], h->nodeset[s][2], h->nodeset[s][3]};
+  BL_LAUNCH(h, "remap_faces", k_remap_faces, nblocks(h->sz.nel), kBlock, B);
+  if (A.mx.ncp > 0)
+    BL_LAUNCH(h, "remap_tile", k_remap_tile<true>, (unsigned)h->ntile, kBlock, B, R, H, W,
+              cm[1 - p]);
+  else
+    BL_LAUNCH(h, "remap_tile", k_remap_tile<false>, (unsigned)h->ntile, kBlock, B, R, H, W,
+              cm[1 - p]);
+  if (!h->diag_on) return BL_SUCCESS;
+  // per-step diagnostics need the step's end first
+  BL_LAUNCH(h, "batch_end", k_batch_end, 1, 64, h->d_ts, (const DtResult*)h->d_dtres);
+  return launch_diag(h, W.x, W.y, W.u, W.v, R.rho_o, R.en_o, R.pre_o);
+}
+
 // one step (parity p: node set p -> node set 1-p), launched on h->stream
 int launch_step(bl_handle_t* h, int p, int stop_at_time_end) {
+  if (ale_tiles(h)) return launch_ale_step(h, p, stop_at_time_end);
   FusedArgs A = make_args(h);
   A.stop_at_time_end = stop_at_time_end;
   A.time_end = h->cfg.time_end;
@@ -1914,13 +2352,13 @@ int launch_step(bl_handle_t* h, int p, int stop_at_time_end) {
                   h->nodeset[1 - p][3]};
   FusedNodes Oc{O.x, O.y, O.u, O.v};
   if (use_tiles(h)) {
-    tile_args(h, A, p);
+    tile_args(h, A, p, p);
     A.end_in_f1b = end_in_f1b(h) ? 1 : 0;  // with per-step diagnostics F5 ends the step
     const unsigned nseg = (unsigned)A.nseg;
     const unsigned nbl = std::min(nseg, (unsigned)h->tune_lim_grid);
     BL_LAUNCH(h, "f1_limiter", k_f1_limiter, nbl, (unsigned)h->tune_lim_block, A, N, (int)nseg);
     BL_LAUNCH(h, "f1b_select", k_f1b_select, 1, kF1bThreads, A, (int)nseg, (int)nbl);
-    BL_LAUNCH(h, "lag_tile", k_lag_tile, (unsigned)h->ntile, kBlock, A, N, O, EnsArgs{});
+    BL_LAUNCH(h, "lag_tile", (k_lag_tile<false, false>), (unsigned)h->ntile, kBlock, A, N, O, EnsArgs{});
     if (end_in_f1b(h)) return BL_SUCCESS;
     // per-step diagnostics: F5 records the step's end, then the record of
     // the node and element sets the step wrote
@@ -1998,13 +2436,6 @@ int ensure_nodesets(bl_handle_t* h) {
     BL_HIP(hipMemset(h->d_rest, 0, sizeof(uint64_t) * words));
     BL_HIP(hipMemset(h->d_vstats, 0, sizeof(unsigned long long) * kStatWords));
   }
-  if (!h->cterm[0])
-    for (int k = 0; k < 4; ++k)
-      BL_HIP(hipMalloc(&h->cterm[k], sizeof(double) * 4 * std::max(h->sz.nel, 1)));
-  if (h->cfg.zexist && !h->ale_tmp[0])
-    for (int k = 0; k < 11; ++k)
-      BL_HIP(hipMalloc(&h->ale_tmp[k], sizeof(double) * ((k < 7 || k == 10) ? 4 : 1) *
-                                           std::max(h->sz.nel, 1)));
   if (h->nodeset[1][0]) return BL_SUCCESS;
   const int ids[4] = {BL_NDX, BL_NDY, BL_NDU, BL_NDV};
   for (int k = 0; k < 4; ++k) {
@@ -2012,6 +2443,32 @@ int ensure_nodesets(bl_handle_t* h) {
     BL_HIP(hipMalloc(&h->nodeset[1][k], sizeof(double) * std::max(h->sz.nnd2, 1)));
   }
   h->cur_set = 0;
+  return BL_SUCCESS;
+}
+
+// what the steps of the form a run call takes work in: the tiled remap's
+// second corner masses, mesh velocity, component energies and face fluxes;
+// or the other forms' corner terms and remap temporaries.  After
+// prepare_tiles, outside any capture.
+int ensure_step_buffers(bl_handle_t* h) {
+  const size_t nel = (size_t)std::max(h->sz.nel, 1), nnd = (size_t)std::max(h->sz.nnd, 1);
+  auto alloc = [](double** p, size_t n) {
+    if (*p) return hipSuccess;
+    return hipMalloc(p, sizeof(double) * n);
+  };
+  if (ale_tiles(h)) {
+    BL_HIP(alloc(&h->ale_tmp[0], 4 * nel));
+    BL_HIP(alloc(&h->cm_other, 4 * nel));
+    if (!h->cfg.zeul)
+      for (int k = 0; k < 2; ++k) BL_HIP(alloc(&h->mesh_w[k], nnd));
+    if (h->sz.ncp > 0) BL_HIP(alloc(&h->d_cpe, (size_t)std::max(h->sz.mcp, 1)));
+    return BL_SUCCESS;
+  }
+  if (use_tiles(h) || ens_tiles(h)) return BL_SUCCESS;
+  for (int k = 0; k < 4; ++k) BL_HIP(alloc(&h->cterm[k], 4 * nel));
+  if (h->cfg.zexist)
+    for (int k = 0; k < 11; ++k)
+      BL_HIP(alloc(&h->ale_tmp[k], ((k < 7 || k == 10) ? 4 : 1) * nel));
   return BL_SUCCESS;
 }
 
@@ -2082,12 +2539,23 @@ void point_elements_at(bl_handle_t* h, int s) {
 // (a batch of another step kind moved the node sets but kept the elements
 // in place).  Outside any capture.
 int prepare_tiles(bl_handle_t* h) {
-  if (!h->tiles_on || !(fold_f1(h) || h->ens_n > 0)) return BL_SUCCESS;
+  const bool ale = ale_on_tiles(h);
+  if (!h->tiles_on || !(fold_f1(h) || h->ens_n > 0 || ale)) return BL_SUCCESS;
   if (h->tile_state == 0) {
     if (build_tiles(h)) return BL_FAILURE;
     invalidate_graph(h);
   }
   if (h->tile_state != 1) return BL_SUCCESS;
+  // the remap's tables follow the neighbours (ielel, ielfc) too
+  if (ale && (!h->ale_tables || h->nbfc_stale)) {
+    if (build_ale_tiles(h)) return BL_FAILURE;
+    invalidate_graph(h);
+  }
+  if (ale && !h->d_tile_nbr) return BL_SUCCESS;  // a mesh it cannot run on
+  if (ale && h->ale_home != h->cur_set) {
+    invalidate_graph(h);
+    h->ale_home = h->cur_set;
+  }
   if (h->el_cur != h->cur_set) {
     for (int k = 0; k < 4; ++k) std::swap(h->elset[0][k], h->elset[1][k]);
     h->el_cur = h->cur_set;
@@ -2176,13 +2644,6 @@ std::vector<int> graph_plan(int nsteps, int p) {
   return plan;
 }
 
-// The end of a batch whose last step left its end open (no F1b after it),
-// on the device, so that the host reads the timestep once after all the
-// call's work
-__global__ void k_batch_end(DevTimestep* ts, const DtResult* res) {
-  if (threadIdx.x == 0) step_end(ts, res);
-}
-
 // The registry's geometry fields after a Lagrangian batch: F4 keeps them in
 // registers, so they are rebuilt once from the final coordinates; the last
 // step's corrector corner forces go back to the element-major rscratch23/24
@@ -2201,9 +2662,17 @@ __global__ void k_materialize(int nel, const int32_t* __restrict__ ielnd,
                               double* __restrict__ b2, double* __restrict__ b3,
                               double* __restrict__ cnwt, double* __restrict__ vol,
                               const double* __restrict__ fxT, const double* __restrict__ fyT,
-                              double* __restrict__ cnfx, double* __restrict__ cnfy) {
+                              double* __restrict__ cnfx, double* __restrict__ cnfy,
+                              double* __restrict__ cm, const double* __restrict__ cm_other) {
   int e = xcd_index();
   if (e >= nel) return;
+  // after an odd number of tiled remaps the corner masses are in the other
+  // array: back into the registry's
+  if (cm_other && (ts->cmflips & 1)) {
+    double c[4];
+    ld4(cm_other, e, c);
+    st4(cm, e, c);
+  }
   const bool other = ((ts ? ts->set0 + ts->flips : cur) & 1) != 0;
   const double* __restrict__ ndx = other ? x1 : x0;
   const double* __restrict__ ndy = other ? y1 : y0;
@@ -2249,17 +2718,19 @@ __global__ void k_publish(const DevTimestep* __restrict__ ts, const double* __re
 // ts null; the tile step's last step wrote rscratch23/24 itself), then the
 // results for the host
 int launch_batch_end(bl_handle_t* h, const DevTimestep* d_ts, int cur) {
-  if (end_in_f1b(h))
+  const bool ale = ale_tiles(h);
+  if (end_in_f1b(h) || ale)
     BL_LAUNCH(h, "batch_end", k_batch_end, 1, 64, h->d_ts, (const DtResult*)h->d_dtres);
   const int nel = h->sz.nel;
-  const bool tiles = use_tiles(h);
+  const bool tiles = use_tiles(h) || ale;
   BL_LAUNCH(h, "materialize", k_materialize, nblocks(nel), kBlock, nel, h->I(BL_IELND),
             h->nodeset[0][0], h->nodeset[0][1], h->nodeset[1][0], h->nodeset[1][1], d_ts, cur,
             h->R(BL_CNX), h->R(BL_CNY), h->R(BL_A1), h->R(BL_A2), h->R(BL_A3), h->R(BL_B1),
             h->R(BL_B2), h->R(BL_B3), h->R(BL_CNWT), h->R(BL_ELVOLUME),
             tiles ? nullptr : (const double*)h->cterm[0],
             tiles ? nullptr : (const double*)h->cterm[1], h->R(BL_RSCRATCH23),
-            h->R(BL_RSCRATCH24));
+            h->R(BL_RSCRATCH24), h->R(BL_CNMASS),
+            ale ? (const double*)h->cm_other : nullptr);
   BL_LAUNCH(h, "publish", k_publish, 1, kBlock, (const DevTimestep*)h->d_ts,
             (const double*)h->d_hist, h->h_pub_ts, h->h_pub_hist, (int)h->hist_cap);
   return BL_SUCCESS;
@@ -2317,12 +2788,12 @@ int launch_ensemble_step(bl_handle_t* h, int p) {
   if (ens_tiles(h)) {
     // E1 ran in the previous step's tile step (or in the run call's
     // prologue); the tile step reads element set p and writes 1 - p
-    tile_args(h, A, p);
+    tile_args(h, A, p, p);
     A.end_in_f1b = 0;  // F5 ends each step
     BL_LAUNCH(h, "e1_limiter", k_e1_limiter, (unsigned)h->ens_lblocks,
               (unsigned)h->tune_lim_block, A, N, E);
     BL_LAUNCH(h, "e1b_select", k_e1b_select, (unsigned)h->ens_n, kBlock, A, E, (int)h->ntile);
-    BL_LAUNCH(h, "lag_tile", k_lag_tile, (unsigned)h->ntile, kBlock, A, N, O, E);
+    BL_LAUNCH(h, "lag_tile", (k_lag_tile<false, false>), (unsigned)h->ntile, kBlock, A, N, O, E);
     BL_LAUNCH(h, "f5_end", k_f5_end, 1, kBlock, A, Oc);
     return BL_SUCCESS;
   }
@@ -2384,7 +2855,8 @@ int bl_ensemble_run(bl_handle_t* h, int32_t nsteps, double* dt_hist, int32_t* id
   }
   fill_err(err, BL_SUCCESS, 0, "");
   if (nsteps <= 0) { if (steps_taken) *steps_taken = 0; return BL_SUCCESS; }
-  if (ensure_nodesets(h) || prepare_tiles(h) || clear_rest(h)) return BL_FAILURE;
+  if (ensure_nodesets(h) || prepare_tiles(h) || ensure_step_buffers(h) || clear_rest(h))
+    return BL_FAILURE;
   if (h->ehist_cap < nsteps) {
     // as bl_run_graph: room for runs of up to 1024 steps without re-capture
     const int cap = std::max(nsteps, 1024);
@@ -2422,7 +2894,7 @@ int bl_ensemble_run(bl_handle_t* h, int32_t nsteps, double* dt_hist, int32_t* id
     const EnsArgs E = make_ens(h);
     FusedNodes N{h->nodeset[p][0], h->nodeset[p][1], h->nodeset[p][2], h->nodeset[p][3]};
     if (ens_tiles(h)) {
-      tile_args(h, A, p);
+      tile_args(h, A, p, p);
       A.rest8_next = h->d_rest8 + (size_t)p * h->sz.nel;  // the first step's own bytes
       BL_LAUNCH(h, "f1_seg", k_f1_seg, (unsigned)h->ntile, kBlock, A, N, E);
     } else {
@@ -2458,7 +2930,7 @@ int bl_ensemble_run(bl_handle_t* h, int32_t nsteps, double* dt_hist, int32_t* id
               h->R(BL_A2), h->R(BL_A3), h->R(BL_B1), h->R(BL_B2), h->R(BL_B3), h->R(BL_CNWT),
               h->R(BL_ELVOLUME), tiles ? nullptr : (const double*)h->cterm[0],
               tiles ? nullptr : (const double*)h->cterm[1], h->R(BL_RSCRATCH23),
-              h->R(BL_RSCRATCH24));
+              h->R(BL_RSCRATCH24), (double*)nullptr, (const double*)nullptr);
   }
   if (taken > 0 && (dt_hist || idt_hist || ctl_hist)) {
     const size_t n = (size_t)taken * h->ens_n;
@@ -2723,7 +3195,8 @@ int bl_get_tiling(bl_handle_t* h, int32_t* on, int32_t* ntile, int32_t* nboundar
     return BL_FAILURE;
   }
   const bool built = h->tile_state == 1;
-  if (on) *on = (h->tiles_on && built && (fold_f1(h) || h->ens_n > 0)) ? 1 : 0;
+  if (on)
+    *on = (h->tiles_on && built && (fold_f1(h) || h->ens_n > 0 || ale_tiles(h))) ? 1 : 0;
   if (ntile) *ntile = built ? h->ntile : 0;
   if (nboundary) *nboundary = 0;  // every element completes in its own tile
   if (nentries) *nentries = built ? h->nentries : 0;
@@ -2772,7 +3245,7 @@ int bl_run_graph(bl_handle_t* h, int32_t nsteps, int32_t stop_at_time_end, bl_ti
     return bl_run(h, nsteps, stop_at_time_end, ts, dt_hist, idt_hist, ctl_hist, steps_taken,
                   err);
   fill_err(err, BL_SUCCESS, 0, "");
-  if (ensure_nodesets(h) || prepare_tiles(h)) return BL_FAILURE;
+  if (ensure_nodesets(h) || prepare_tiles(h) || ensure_step_buffers(h)) return BL_FAILURE;
   if (h->hist_cap < nsteps || !h->h_pub_hist) {
     // the graphs bake in the history's capacity: size it generously so that
     // runs of different lengths do not re-capture
@@ -2795,7 +3268,9 @@ int bl_run_graph(bl_handle_t* h, int32_t nsteps, int32_t stop_at_time_end, bl_ti
   if (h->cfg.zexist && (h->nbfc_stale || !h->d_nbfc) && build_nbfc(h)) return BL_FAILURE;
   // (all of them at once, so that a later call of another length finds
   // its graphs: a capture costs about 0.1 ms)
-  const std::vector<int> plan = graph_plan(h->timing ? 0 : nsteps, h->cur_set);
+  const bool ale = ale_tiles(h);
+  const int p0 = ale ? 0 : h->cur_set;  // the first step's parity
+  const std::vector<int> plan = graph_plan(h->timing ? 0 : nsteps, p0);
   bool missing = false;
   for (int q : plan) missing = missing || !h->graph_exec[q];
   for (int q = 0; missing && q < kGraphs; ++q)
@@ -2808,12 +3283,13 @@ int bl_run_graph(bl_handle_t* h, int32_t nsteps, int32_t stop_at_time_end, bl_ti
   d->nstep = ts->nstep; d->idtel = ts->idtel; d->sdt = ts->sdt;
   d->last_step = ts->nstep + nsteps;
   d->set0 = h->cur_set;
+  d->ale_tile = ale ? 1 : 0;
   if (clear_rest(h, d, resume)) return BL_FAILURE;
-  const bool tiles = use_tiles(h);
-  int p = h->cur_set;
+  const bool tiles = use_tiles(h) || ale;
+  int p = p0;
   // F1 of the first step: on a resumed call the last call's last step left
   // its terms, its at-rest mask and the zeros it stands for
-  if (fold_f1(h) && !resume && launch_f1_prologue(h, p, stop_at_time_end)) return BL_FAILURE;
+  if (folded(h) && !resume && launch_f1_prologue(h, p, stop_at_time_end)) return BL_FAILURE;
   // with kernel timing on, the same step kernels are launched directly so
   // each launch can be bracketed by HIP events on this stream
   if (h->timing)

@@ -38,6 +38,7 @@ struct DtResult {
   int32_t div_idx;  // 1-based, 0 if none exceeds TINY
   int32_t negvol;   // largest 1-based index with V < 0 (0 if none)
   int32_t negvol2;  // the same for the corrector geometry of the fused step
+  int32_t negvol3;  // the same for the moved mesh of the tiled remap
 };
 
 // device-resident timestep state of the fused step (bl_run_graph): the
@@ -70,6 +71,14 @@ struct DevTimestep {
   int32_t open;
   // the node set the batch started from (the final one is set0 + flips)
   int32_t set0;
+  // the step running found a negative volume before its remap: the kernels
+  // after the tile step do nothing (cleared by F1b)
+  int32_t bad;
+  // the batch's steps end with the tiled remap, which puts each step's state
+  // back into the node and element set the step started from; and the steps
+  // whose remap ran (they alternate the two corner-mass arrays)
+  int32_t ale_tile;
+  int32_t cmflips;
 };
 constexpr int32_t kNoPending = 0x7fffffff;
 
@@ -211,6 +220,18 @@ struct Handle {
   double* elset[2][4] = {};
   int el_cur = 0;
   float* d_ld1 = nullptr;         // (nnd, 2): one-sweep displacement of the node
+  // the tiled remap (zexist): per tile entry the entries of its four face
+  // neighbours (one byte each, of the tile's own elements), per tile node the
+  // entries around it by corner and their two summation orders; the second
+  // corner-mass array (the first is the registry's); the mesh velocity of
+  // the node relaxation; the component energies after the predictor
+  int32_t* d_tile_nbr = nullptr;
+  int2* d_tile_ninc = nullptr;
+  double* cm_other = nullptr;
+  double* mesh_w[2] = {};
+  double* d_cpe = nullptr;
+  bool ale_tables = false;        // built, or found that the mesh has none (both null)
+  int ale_home = -1;              // the node set the captured remap steps start from
   // per-step diagnostics of the fused step: region table + Sod L1 records
   bool diag_on = false;
   double diag_x0 = 0.0, diag_scale = 1.0;

@@ -40,6 +40,7 @@ struct MixArgs {
   double* cpb3;
   double* cpfx;  // rcpscratch21 (lagstep cpfx), (4, mcp)
   double* cpfy;  // rcpscratch22
+  double* cpe;   // tile step: cpenergy after the predictor (null otherwise)
 };
 
 MixArgs make_mix(Handle* h);

@@ -193,6 +193,7 @@ MixArgs make_mix(Handle* h) {
   M.cpvisc = h->R(BL_CPVISC); M.cpviscx = h->R(BL_CPVISCX); M.cpviscy = h->R(BL_CPVISCY);
   M.cpa1 = h->R(BL_CPA1); M.cpa3 = h->R(BL_CPA3); M.cpb1 = h->R(BL_CPB1); M.cpb3 = h->R(BL_CPB3);
   M.cpfx = h->R(BL_RCPSCRATCH21); M.cpfy = h->R(BL_RCPSCRATCH22);
+  M.cpe = h->d_cpe;
   return M;
 }
 

@@ -18,6 +18,11 @@ constexpr uint32_t kTileOwn = 1;
 // mesh has a node that is the same corner of two elements (h->tile_state
 // -1, no tiling); ielnd and the node positions come from the registry.
 int build_tiles(Handle* h);
+// The tiled remap's tables on a built tiling, from ielel, ielfc and ielsort2
+// (h->ale_tables; d_tile_nbr stays null on a mesh it cannot run on: a face
+// neighbour outside the tile's entries, or a boundary face whose ielfc is not
+// the opposite face).
+int build_ale_tiles(Handle* h);
 void free_tiles(Handle* h);
 
 }  // namespace bl

@@ -110,7 +110,7 @@ int upload_vec(T** d, const std::vector<T>& v) {
 
 void free_tiles(Handle* h) {
   void* bufs[] = {h->d_tile_eptr, h->d_tile_nptr, h->d_tile_bounds, h->d_tile_nodes, h->d_tile_ncm, h->d_tile_el,
-                  h->d_tile_nd, h->d_rest8, h->d_ens_toff};
+                  h->d_tile_nd, h->d_rest8, h->d_ens_toff, h->d_tile_nbr, h->d_tile_ninc};
   for (void* p : bufs)
     if (p) hipFree(p);
   h->d_tile_eptr = h->d_tile_nptr = h->d_tile_nodes = nullptr;
@@ -119,6 +119,9 @@ void free_tiles(Handle* h) {
   h->d_tile_el = nullptr;
   h->d_tile_nd = nullptr;
   h->d_ens_toff = nullptr;
+  h->d_tile_nbr = nullptr;
+  h->d_tile_ninc = nullptr;
+  h->ale_tables = false;
   h->d_rest8 = nullptr;
   h->ntile = h->nentries = 0;
   h->tile_state = 0;
@@ -285,6 +288,87 @@ int build_tiles(Handle* h) {
     h->el_cur = h->cur_set;
   }
   h->tile_state = 1;
+  return BL_SUCCESS;
+}
+
+int build_ale_tiles(Handle* h) {
+  if (h->d_tile_nbr) hipFree(h->d_tile_nbr);
+  if (h->d_tile_ninc) hipFree(h->d_tile_ninc);
+  h->d_tile_nbr = nullptr;
+  h->d_tile_ninc = nullptr;
+  h->ale_tables = true;
+  const int nel = h->sz.nel, ntile = h->ntile;
+  bl_handle_t* hh = static_cast<bl_handle_t*>(h);
+  std::vector<int32_t> el(4 * (size_t)nel), fc(4 * (size_t)nel), sort2(nel), pos2(nel);
+  std::vector<int32_t> eptr(ntile + 1), nptr(ntile + 1);
+  if (bl_download(hh, BL_IELEL, el.data(), 4 * (int64_t)nel) ||
+      bl_download(hh, BL_IELFC, fc.data(), 4 * (int64_t)nel) ||
+      bl_download(hh, BL_IELSORT2, sort2.data(), nel))
+    return BL_FAILURE;
+  BL_HIP(hipMemcpy(eptr.data(), h->d_tile_eptr, sizeof(int32_t) * (ntile + 1),
+                   hipMemcpyDeviceToHost));
+  BL_HIP(hipMemcpy(nptr.data(), h->d_tile_nptr, sizeof(int32_t) * (ntile + 1),
+                   hipMemcpyDeviceToHost));
+  std::vector<int2> ents(eptr[ntile]);
+  BL_HIP(hipMemcpy(ents.data(), h->d_tile_el, sizeof(int2) * ents.size(),
+                   hipMemcpyDeviceToHost));
+  // the place of each element in the ALE sums (unset ielsort2: identity)
+  for (int k = 0; k < nel; ++k) pos2[k] = k;
+  for (int k = 0; k < nel; ++k) {
+    const int e = (sort2[k] < 1 || sort2[k] > nel) ? k : sort2[k] - 1;
+    pos2[e] = k;
+  }
+  std::vector<int32_t> nbr(ents.size(), 0), local(nel, -1), stamp(nel, -1);
+  std::vector<int2> ninc(nptr[ntile], make_int2(0, 0));
+  struct Inc { int32_t e, j; };
+  std::vector<Inc> inc(4 * (kTileNodes + 1));
+  std::vector<int> cnt(kTileNodes + 1);
+  for (int t = 0; t < ntile; ++t) {
+    const int eb = eptr[t], ne = eptr[t + 1] - eb, nb = nptr[t], nn = nptr[t + 1] - nb;
+    std::fill(cnt.begin(), cnt.begin() + nn, 0);
+    for (int k = 0; k < ne; ++k) {
+      const int e = ents[eb + k].x & 0x3fffffff;
+      local[e] = k;
+      stamp[e] = t;
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t sl = ((uint32_t)ents[eb + k].y >> (8 * j)) & 0xFFu;
+        if (sl == kNoSlot) continue;
+        // (at most four: no node is corner jj of two elements)
+        int2& q = ninc[nb + sl];
+        q.x = (int)((uint32_t)q.x | ((uint32_t)k << (8 * j)));
+        inc[4 * sl + cnt[sl]++] = Inc{e, j};
+      }
+    }
+    for (int k = 0; k < ne; ++k) {
+      const uint32_t w = (uint32_t)ents[eb + k].x;
+      if (!((w >> 30) & kTileOwn)) continue;
+      const int e = (int)(w & 0x3fffffffu);
+      uint32_t bytes = 0;
+      for (int i = 0; i < 4; ++i) {
+        const int b = el[4 * (size_t)e + i] - 1, g = fc[4 * (size_t)e + i] - 1;
+        if (b < 0 || b >= nel || g < 0 || g > 3 || stamp[b] != t ||
+            (b == e && g != ((i + 2) & 3)))
+          return BL_SUCCESS;  // not a mesh the tiled remap runs on
+        bytes |= (uint32_t)local[b] << (8 * i);
+      }
+      nbr[eb + k] = (int32_t)bytes;
+    }
+    for (int v = 0; v < nn; ++v) {
+      Inc* q = &inc[4 * (size_t)v];
+      const int n = cnt[v];
+      uint32_t code = (uint32_t)n << 16;
+      std::sort(q, q + n, [&](const Inc& a, const Inc& b) {
+        return a.e != b.e ? pos2[a.e] < pos2[b.e] : a.j < b.j;
+      });
+      for (int k = 0; k < n; ++k) code |= (uint32_t)q[k].j << (2 * k);
+      std::sort(q, q + n, [](const Inc& a, const Inc& b) {
+        return a.e != b.e ? a.e < b.e : a.j < b.j;
+      });
+      for (int k = 0; k < n; ++k) code |= (uint32_t)q[k].j << (8 + 2 * k);
+      ninc[nb + v].y = (int)code;
+    }
+  }
+  if (upload_vec(&h->d_tile_ninc, ninc) || upload_vec(&h->d_tile_nbr, nbr)) return BL_FAILURE;
   return BL_SUCCESS;
 }
 
