@@ -18,7 +18,7 @@
 // each wave runs its 64 nodes through the three layers on the matrix cores
 // (v_mfma_f32_16x16x16_bf16: BF16 weights and activations, FP32
 // accumulation), 16 nodes per pass, weights and activations in registers.
-// Training is one thread per sample in FP32 with the forward pass rounding
+// Training is a lane per sample in FP32 with the forward pass rounding
 // weights and activations to BF16 as the matrix cores see them
 // (straight-through gradients); per-workgroup gradients are summed in a
 // fixed order, so training is reproducible run to run; Adam updates FP32
@@ -602,147 +602,273 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
   return z ^ (z >> 31);
 }
 
-// one workgroup of kTrainBlock samples, a thread per sample: forward with
+// One workgroup of 512 threads per kTrainBlock samples: forward with
 // BF16-rounded weights, inputs and hidden activations and FP32 sums;
 // backward; this workgroup's gradient of the mean squared error over the
 // batch (each parameter summed over the samples in order) into
-// part[blockIdx][param], its loss sum into lpart[blockIdx].  Samples come
-// from idx (explicit) or are drawn from npairs by (seed, it).  Per-sample
-// vectors live in LDS rows padded to an odd stride (no bank conflicts).
-constexpr int kInP = kIn + 1, kHidP = kHid + 1;
+// part[blockIdx][param], its loss sum into lpart[blockIdx].  Sample s is pair
+// s (drawn = 0), or drawn from npairs by (seed, it).
+//
+// Lane l of every wave holds sample l; wave w computes hidden units 8w to
+// 8w+7 of it, so that a weight is one value for the whole wave (a scalar
+// operand, from wr, the weights rounded to BF16 beforehand) and 8 sums run
+// side by side.  The weight gradients are blocks of 4 x 2 (4 x 1 for the
+// first layer) parameters a thread, read from LDS four rows at a time.  Every sum keeps one order: k ascending in the layers, samples
+// ascending in the gradients.  At batch 8192 (128 workgroups) a launch takes 22
+// us where one thread a sample (a wave a workgroup, serial chains) took 128;
+// 256 threads took 35 (with the k loops unrolled), 1024 threads as long as
+// 512.  Bound by latency: a workgroup's phases wait for one another.
+constexpr int kTrainThreads = 512;
+constexpr int kUnits = kHid / (kTrainThreads / 64);  // hidden units a wave
+// LDS rows: multiples of 16 bytes, and consecutive rows 4 banks apart
+constexpr int kInP = kIn + 2, kHidP = kHid + 4;
+static_assert(kTrainBlock == 64, "a lane per sample");
+// columns of a thread's block of the weight gradients (four rows)
+constexpr int kCols2 = kHid * kHid / (4 * kTrainThreads), kCols1 = kTrainThreads > 256 ? 1 : 2;
+static_assert(kTrainThreads >= (kHid / 4) * (kIn / kCols1) && kCols2 >= 1,
+              "a gradient block per thread");
+// W consecutive floats of a row of LDS (W of 1, 2 or 4, aligned)
+template <int W>
+__device__ __forceinline__ void row_load(const float* p, float v[W]) {
+  typedef float vec __attribute__((ext_vector_type(W)));
+  const vec x = *reinterpret_cast<const vec*>(p);
+#pragma unroll
+  for (int c = 0; c < W; ++c) v[c] = x[c];
+}
+template <>
+__device__ __forceinline__ void row_load<1>(const float* p, float v[1]) { v[0] = *p; }
+// g[r][c] = sum over the samples q of fmaf(d[q][r], b[q][c], .), q ascending
+template <int W, int SD, int SB>
+__device__ __forceinline__ void grad_block(const float* d, const float* b, float g[4][W]) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int c = 0; c < W; ++c) g[r][c] = 0.0f;
+#pragma unroll 8
+  for (int q = 0; q < kTrainBlock; ++q) {
+    float dd[4], bb[W];
+    row_load<4>(d + q * SD, dd);
+    row_load<W>(b + q * SB, bb);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int c = 0; c < W; ++c) g[r][c] = fmaf(dd[r], bb[c], g[r][c]);
+  }
+}
 
-__global__ void __launch_bounds__(kTrainBlock)
-k_mlp_train(const float* __restrict__ w, const float* __restrict__ norm,
-            const float* __restrict__ feat,
-            const float* __restrict__ targ, const int32_t* __restrict__ idx, int npairs,
+// out[u] = sum over k < K of fmaf(w[u * su + k * sk], a[k], .), k ascending:
+// a rolled loop of four k at a time (a launch runs this code once, so
+// unrolled it is bound by the instruction fetch)
+template <int K>
+__device__ __forceinline__ void train_dot(const float* __restrict__ w, int su, int sk,
+                                          const float* a, float out[kUnits]) {
+#pragma unroll
+  for (int u = 0; u < kUnits; ++u) out[u] = 0.0f;
+  constexpr int kStep = 4;
+#pragma unroll 2
+  for (int k0 = 0; k0 + kStep <= K; k0 += kStep) {
+    float x[kStep];
+    row_load<kStep>(a + k0, x);
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u)
+#pragma unroll
+      for (int k = 0; k < kStep; ++k) out[u] = fmaf(w[u * su + (k0 + k) * sk], x[k], out[u]);
+  }
+#pragma unroll
+  for (int k = K / kStep * kStep; k < K; ++k)
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) out[u] = fmaf(w[u * su + k * sk], a[k], out[u]);
+}
+
+__global__ void __launch_bounds__(kTrainThreads)
+k_mlp_train(const float* __restrict__ wr, const float* __restrict__ norm,
+            const float* __restrict__ feat, const float* __restrict__ targ, int drawn, int npairs,
             int batch, uint64_t seed, int it, float* __restrict__ part,
             float* __restrict__ lpart) {
-  __shared__ float sw[kNParam];
-  __shared__ float sx[kTrainBlock][kInP];
-  __shared__ float sa1[kTrainBlock][kHidP];   // r(z1) in BF16
-  __shared__ float sa2[kTrainBlock][kHidP];   // r(z2) in BF16
-  __shared__ float sd1[kTrainBlock][kHidP];   // z1, then dL/dz1
-  __shared__ float sd2[kTrainBlock][kHidP];   // z2, then dL/dz2
-  __shared__ float sd3[kTrainBlock][kOut];    // dL/dy
+  __shared__ __align__(16) float sx[kTrainBlock][kInP];
+  __shared__ __align__(16) float sa1[kTrainBlock][kHidP];  // r(z1) in BF16
+  __shared__ __align__(16) float sa2[kTrainBlock][kHidP];  // r(z2) in BF16
+  __shared__ __align__(16) float sd1[kTrainBlock][kHidP];  // dL/dz1
+  __shared__ __align__(16) float sd2[kTrainBlock][kHidP];  // dL/dz2
+  __shared__ float sd3[kTrainBlock][kOut];                 // dL/dy
   __shared__ float sloss[kTrainBlock];
-  const int t = threadIdx.x;
-  for (int p = t; p < kNParam; p += kTrainBlock) {
-    const bool is_w = (p < kOffB1) || (p >= kOffW2 && p < kOffB2) || (p >= kOffW3 && p < kOffB3);
-    sw[p] = is_w ? bfr(w[p]) : w[p];
-  }
-  const int s = blockIdx.x * kTrainBlock + t;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), u0 = wave * kUnits;
+  const int s = blockIdx.x * kTrainBlock + lane;
   const bool live = s < batch;
   int src = 0;
-  if (live) {
-    if (idx) src = idx[s];
-    else src = (int)(mix64(seed ^ mix64(((uint64_t)it << 32) | (uint32_t)s)) % (uint64_t)npairs);
-  }
-  for (int k = 0; k < kIn; ++k)
-    sx[t][k] = live ? bfr(norm_in(norm, k, feat[(size_t)src * kIn + k])) : 0.0f;
-  // the difference of the target from one sweep f[24..25], standardised
-  const float t0 =
-      live ? ((targ[(size_t)src * kOut] - feat[(size_t)src * kIn + 24]) - norm[kNormMuT]) /
-                 norm[kNormSigT]
-           : 0.0f;
-  const float t1 =
-      live ? ((targ[(size_t)src * kOut + 1] - feat[(size_t)src * kIn + 25]) - norm[kNormMuT + 1]) /
-                 norm[kNormSigT + 1]
-           : 0.0f;
+  if (live)
+    src = drawn ? (int)(mix64(seed ^ mix64(((uint64_t)it << 32) | (uint32_t)s)) % (uint64_t)npairs)
+                : s;
+  // the inputs: a wave loads every fourth column of its lanes' samples
+  for (int k = wave; k < kIn; k += kTrainThreads / 64)
+    sx[lane][k] = live ? bfr(norm_in(norm, k, feat[(size_t)src * kIn + k])) : 0.0f;
   __syncthreads();
-  for (int i = 0; i < kHid; ++i) {
-    float acc = 0.0f;
-    for (int k = 0; k < kIn; ++k) acc = fmaf(sw[kOffW1 + i * kIn + k], sx[t][k], acc);
-    const float z = acc + sw[kOffB1 + i];
-    sd1[t][i] = z;
-    sa1[t][i] = bfr(z > 0.0f ? z : 0.0f);
+  float z1[kUnits], z2[kUnits], d1[kUnits];
+  train_dot<kIn>(wr + kOffW1 + u0 * kIn, kIn, 1, sx[lane], z1);
+#pragma unroll
+  for (int u = 0; u < kUnits; ++u) {
+    z1[u] = z1[u] + wr[kOffB1 + u0 + u];
+    sa1[lane][u0 + u] = bfr(z1[u] > 0.0f ? z1[u] : 0.0f);
   }
-  for (int i = 0; i < kHid; ++i) {
-    float acc = 0.0f;
-    for (int k = 0; k < kHid; ++k) acc = fmaf(sw[kOffW2 + i * kHid + k], sa1[t][k], acc);
-    const float z = acc + sw[kOffB2 + i];
-    sd2[t][i] = z;
-    sa2[t][i] = bfr(z > 0.0f ? z : 0.0f);
+  __syncthreads();
+  train_dot<kHid>(wr + kOffW2 + u0 * kHid, kHid, 1, sa1[lane], z2);
+#pragma unroll
+  for (int u = 0; u < kUnits; ++u) {
+    z2[u] = z2[u] + wr[kOffB2 + u0 + u];
+    sa2[lane][u0 + u] = bfr(z2[u] > 0.0f ? z2[u] : 0.0f);
   }
-  float loss = 0.0f;
+  __syncthreads();
+  // the output layer, by every wave for its own use of dL/dy
+  float d3[kOut], y[kOut] = {0.0f, 0.0f}, loss = 0.0f;
+#pragma unroll 2
+  for (int k = 0; k < kHid; k += 4) {
+    float x[4];
+    row_load<4>(&sa2[lane][k], x);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int o = 0; o < kOut; ++o) y[o] = fmaf(wr[kOffW3 + o * kHid + k + c], x[c], y[o]);
+  }
+#pragma unroll
   for (int o = 0; o < kOut; ++o) {
-    float acc = 0.0f;
-    for (int k = 0; k < kHid; ++k) acc = fmaf(sw[kOffW3 + o * kHid + k], sa2[t][k], acc);
-    const float r = acc + sw[kOffB3 + o] - (o == 0 ? t0 : t1);
+    // the difference of the target from one sweep f[24..25], standardised
+    const float target =
+        live ? ((targ[(size_t)src * kOut + o] - feat[(size_t)src * kIn + 24 + o]) -
+                norm[kNormMuT + o]) / norm[kNormSigT + o]
+             : 0.0f;
+    const float r = y[o] + wr[kOffB3 + o] - target;
     loss = loss + r * r;
     // d(mean over batch and outputs of r^2)/dy
-    sd3[t][o] = live ? 2.0f * r / (float)(batch * kOut) : 0.0f;
+    d3[o] = live ? 2.0f * r / (float)(batch * kOut) : 0.0f;
   }
-  sloss[t] = live ? loss : 0.0f;
-  for (int i = 0; i < kHid; ++i) {
-    const float acc = fmaf(sw[kOffW3 + i], sd3[t][0], sw[kOffW3 + kHid + i] * sd3[t][1]);
-    sd2[t][i] = sd2[t][i] > 0.0f ? acc : 0.0f;
+  if (wave == 0) {
+    sd3[lane][0] = d3[0];
+    sd3[lane][1] = d3[1];
+    sloss[lane] = live ? loss : 0.0f;
   }
-  for (int i = 0; i < kHid; ++i) {
-    float acc = 0.0f;
-    for (int k = 0; k < kHid; ++k) acc = fmaf(sw[kOffW2 + k * kHid + i], sd2[t][k], acc);
-    sd1[t][i] = sd1[t][i] > 0.0f ? acc : 0.0f;
+#pragma unroll
+  for (int u = 0; u < kUnits; ++u) {
+    const int i = u0 + u;
+    const float acc = fmaf(wr[kOffW3 + i], d3[0], wr[kOffW3 + kHid + i] * d3[1]);
+    sd2[lane][i] = z2[u] > 0.0f ? acc : 0.0f;
   }
   __syncthreads();
-  // this workgroup's gradient: parameter p summed over the samples in order
+  train_dot<kHid>(wr + kOffW2 + u0, 1, kHid, sd2[lane], d1);
+#pragma unroll
+  for (int u = 0; u < kUnits; ++u) sd1[lane][u0 + u] = z1[u] > 0.0f ? d1[u] : 0.0f;
+  __syncthreads();
+  // this workgroup's gradient: each parameter summed over the samples in order
   float* out = part + (size_t)blockIdx.x * kNParam;
-  for (int p = t; p < kNParam; p += kTrainBlock) {
-    float g = 0.0f;
-    if (p < kOffB1) {
-      const int i = p / kIn, k = p % kIn;
-      for (int q = 0; q < kTrainBlock; ++q) g = fmaf(sd1[q][i], sx[q][k], g);
-    } else if (p < kOffW2) {
-      const int i = p - kOffB1;
-      for (int q = 0; q < kTrainBlock; ++q) g = g + sd1[q][i];
-    } else if (p < kOffB2) {
-      const int i = (p - kOffW2) / kHid, k = (p - kOffW2) % kHid;
-      for (int q = 0; q < kTrainBlock; ++q) g = fmaf(sd2[q][i], sa1[q][k], g);
-    } else if (p < kOffW3) {
-      const int i = p - kOffB2;
-      for (int q = 0; q < kTrainBlock; ++q) g = g + sd2[q][i];
-    } else if (p < kOffB3) {
-      const int o = (p - kOffW3) / kHid, k = (p - kOffW3) % kHid;
-      for (int q = 0; q < kTrainBlock; ++q) g = fmaf(sd3[q][o], sa2[q][k], g);
-    } else {
-      const int o = p - kOffB3;
-      for (int q = 0; q < kTrainBlock; ++q) g = g + sd3[q][o];
-    }
-    out[p] = g;
+  {
+    const int i = 4 * (t / (kHid / kCols2)), k = kCols2 * (t % (kHid / kCols2));
+    float g[4][kCols2];
+    grad_block<kCols2, kHidP, kHidP>(&sd2[0][i], &sa1[0][k], g);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int c = 0; c < kCols2; ++c) out[kOffW2 + (i + r) * kHid + k + c] = g[r][c];
   }
-  if (t == 0) {
+  if (t < (kHid / 4) * (kIn / kCols1)) {
+    const int i = 4 * (t / (kIn / kCols1)), k = kCols1 * (t % (kIn / kCols1));
+    float g[4][kCols1];
+    grad_block<kCols1, kHidP, kInP>(&sd1[0][i], &sx[0][k], g);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int c = 0; c < kCols1; ++c) out[kOffW1 + (i + r) * kIn + k + c] = g[r][c];
+  }
+  // the output layer and the biases
+  float g = 0.0f;
+  if (t < kOut * kHid) {
+    const int o = t / kHid, k = t % kHid;
+#pragma unroll 8
+    for (int q = 0; q < kTrainBlock; ++q) g = fmaf(sd3[q][o], sa2[q][k], g);
+    out[kOffW3 + t] = g;
+  } else if (t < kOut * kHid + kHid) {
+    const int i = t - kOut * kHid;
+#pragma unroll 8
+    for (int q = 0; q < kTrainBlock; ++q) g = g + sd1[q][i];
+    out[kOffB1 + i] = g;
+  } else if (t < kOut * kHid + 2 * kHid) {
+    const int i = t - kOut * kHid - kHid;
+#pragma unroll 8
+    for (int q = 0; q < kTrainBlock; ++q) g = g + sd2[q][i];
+    out[kOffB2 + i] = g;
+  }
+  if (t <= kOut) {
     float l = 0.0f;
-    for (int q = 0; q < kTrainBlock; ++q) l = l + sloss[q];
-    lpart[blockIdx.x] = l;
+#pragma unroll 8
+    for (int q = 0; q < kTrainBlock; ++q) l = l + (t < kOut ? sd3[q][t % kOut] : sloss[q]);
+    if (t < kOut) out[kOffB3 + t] = l;
+    else lpart[blockIdx.x] = l;
   }
 }
+static_assert(kOut * kHid + 2 * kHid <= kTrainThreads, "the last sums, one a thread");
 
-// the gradient: workgroup partials summed in order; loss likewise
-__global__ void k_mlp_reduce(int nblk, const float* __restrict__ part,
-                             const float* __restrict__ lpart, float* __restrict__ grad,
-                             float* __restrict__ loss, int batch) {
+// the weights as the matrix cores see them (rounded to BF16) beside the FP32
+// biases, for k_mlp_train
+__device__ __forceinline__ float round_param(int p, float w) {
+  const bool is_w = (p < kOffB1) || (p >= kOffW2 && p < kOffB2) || (p >= kOffW3 && p < kOffB3);
+  return is_w ? bfr(w) : w;
+}
+__global__ void k_mlp_round(const float* __restrict__ w, float* __restrict__ wr) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < kNParam) {
-    float g = 0.0f;
-    for (int b = 0; b < nblk; ++b) g = g + part[(size_t)b * kNParam + p];
-    grad[p] = g;
-  }
-  if (p == 0) {
-    float l = 0.0f;
-    for (int b = 0; b < nblk; ++b) l = l + lpart[b];
-    *loss = l / (float)(batch * kOut);
-  }
+  if (p < kNParam) wr[p] = round_param(p, w[p]);
 }
 
-// Adam (beta1 0.9, beta2 0.999, eps 1e-8) on the FP32 master weights
-__global__ void k_mlp_adam(float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
-                           const float* __restrict__ g, float lr, int step) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+// the gradient of parameter p: the workgroups' partials summed in order (32
+// loads in flight), its loss likewise
+__device__ __forceinline__ float sum_parts(int nblk, const float* __restrict__ part, int stride) {
+  constexpr int kAhead = 32;
+  float g = 0.0f;
+  int b = 0;
+  for (; b + kAhead <= nblk; b += kAhead) {
+    float v[kAhead];
+#pragma unroll
+    for (int r = 0; r < kAhead; ++r) v[r] = part[(size_t)(b + r) * stride];
+#pragma unroll
+    for (int r = 0; r < kAhead; ++r) g = g + v[r];
+  }
+  for (; b < nblk; ++b) g = g + part[(size_t)b * stride];
+  return g;
+}
+constexpr int kSumBlock = 64;  // a wave a workgroup: 94 workgroups
+
+__global__ void __launch_bounds__(kSumBlock)
+k_mlp_reduce(int nblk, const float* __restrict__ part, const float* __restrict__ lpart,
+             float* __restrict__ grad, float* __restrict__ loss, int batch) {
+  const int p = blockIdx.x * kSumBlock + threadIdx.x;
+  if (p < kNParam) grad[p] = sum_parts(nblk, part + p, kNParam);
+  // (the parameters end inside the last workgroup, whose last thread is free)
+  if (p == (int)gridDim.x * kSumBlock - 1) *loss = sum_parts(nblk, lpart, 1) / (float)(batch * kOut);
+}
+static_assert(kNParam % kSumBlock != 0, "a thread for the loss");
+
+// the reduction and Adam (beta1 0.9, beta2 0.999, eps 1e-8) on the FP32
+// master weights in one launch, with the rounded copy of the next step (128
+// partials: 5.5 us, where a reduction of 24 workgroups with one load in
+// flight and a launch of Adam's own took 40)
+__global__ void __launch_bounds__(kSumBlock)
+k_mlp_adam(int nblk, const float* __restrict__ part, const float* __restrict__ lpart,
+           float* __restrict__ loss, int batch, float* __restrict__ w, float* __restrict__ wr,
+           float* __restrict__ m, float* __restrict__ v, float* __restrict__ grad, float lr,
+           int step) {
+  const int p = blockIdx.x * kSumBlock + threadIdx.x;
+  if (p == (int)gridDim.x * kSumBlock - 1) *loss = sum_parts(nblk, lpart, 1) / (float)(batch * kOut);
   if (p >= kNParam) return;
+  const float g = sum_parts(nblk, part + p, kNParam);
+  grad[p] = g;
   const float b1 = 0.9f, b2 = 0.999f;
-  m[p] = b1 * m[p] + (1.0f - b1) * g[p];
-  v[p] = b2 * v[p] + (1.0f - b2) * g[p] * g[p];
-  const float mh = m[p] / (1.0f - powf(b1, (float)step));
-  const float vh = v[p] / (1.0f - powf(b2, (float)step));
-  w[p] = w[p] - lr * mh / (sqrtf(vh) + 1.0e-8f);
+  const float m1 = b1 * m[p] + (1.0f - b1) * g;
+  const float v1 = b2 * v[p] + (1.0f - b2) * g * g;
+  m[p] = m1;
+  v[p] = v1;
+  const float mh = m1 / (1.0f - powf(b1, (float)step));
+  const float vh = v1 / (1.0f - powf(b2, (float)step));
+  const float w1 = w[p] - lr * mh / (sqrtf(vh) + 1.0e-8f);
+  w[p] = w1;
+  wr[p] = round_param(p, w1);
 }
 
 // pack the master weights as BF16 A operands (the layout of MlpPacked)
@@ -772,11 +898,14 @@ __global__ void k_mlp_pack(const float* __restrict__ w, u64x2* __restrict__ w1p,
 
 using namespace bl;
 
+constexpr int kLossCap = 4096;  // losses of a training call before it grows
+
 struct bl_mlp {
   float* w = nullptr;  // FP32 master (kNParam)
   float* m = nullptr;
   float* v = nullptr;
   float* g = nullptr;
+  float* wr = nullptr;  // the weights rounded to BF16, as training reads them
   u64x2* w1p = nullptr;
   u64x2* w2p = nullptr;
   u64x2* w3p = nullptr;
@@ -789,7 +918,8 @@ struct bl_mlp {
   int32_t cap = 0;
   float* part = nullptr;
   float* lpart = nullptr;
-  float* loss = nullptr;
+  float* loss = nullptr;     // loss_cap: one per Adam step of a call
+  int32_t loss_cap = 0;
   int32_t part_blocks = 0;
   int32_t adam_step = 0;
   hipStream_t stream = nullptr;
@@ -842,15 +972,24 @@ int ensure_parts(bl_mlp* m, int nblk) {
   return BL_SUCCESS;
 }
 
-// gradient of the batch's loss into m->g, loss into m->loss
-int mlp_gradient(bl_mlp* m, const int32_t* idx, int npairs, int batch, uint64_t seed, int it) {
-  const int nblk = (batch + kTrainBlock - 1) / kTrainBlock;
+constexpr unsigned kSumGrid = (kNParam + kSumBlock - 1) / kSumBlock;
+
+int train_blocks(int batch) { return (int)(((int64_t)batch + kTrainBlock - 1) / kTrainBlock); }
+
+// the workgroup partials of the batch's gradient and loss (pairs drawn by
+// (seed, it), or pairs 0 .. batch-1)
+int mlp_partials(bl_mlp* m, int drawn, int npairs, int batch, uint64_t seed, int it) {
+  const int nblk = train_blocks(batch);
   if (ensure_parts(m, nblk)) return BL_FAILURE;
-  hipLaunchKernelGGL(k_mlp_train, dim3(nblk), dim3(kTrainBlock), 0, m->stream, m->w,
-                     (const float*)m->norm, m->feat, m->targ, idx, npairs, batch, seed, it,
-                     m->part, m->lpart);
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((kNParam + 255) / 256), dim3(256), 0, m->stream, nblk,
-                     m->part, m->lpart, m->g, m->loss, batch);
+  hipLaunchKernelGGL(k_mlp_train, dim3(nblk), dim3(kTrainThreads), 0, m->stream,
+                     (const float*)m->wr, (const float*)m->norm, (const float*)m->feat,
+                     (const float*)m->targ, drawn, npairs, batch, seed, it, m->part, m->lpart);
+  return hipGetLastError() == hipSuccess ? BL_SUCCESS : BL_FAILURE;
+}
+
+int mlp_round(bl_mlp* m) {
+  hipLaunchKernelGGL(k_mlp_round, dim3(kSumGrid), dim3(kSumBlock), 0, m->stream,
+                     (const float*)m->w, m->wr);
   return hipGetLastError() == hipSuccess ? BL_SUCCESS : BL_FAILURE;
 }
 
@@ -935,6 +1074,7 @@ int bl_mlp_create(uint64_t seed, int32_t capacity, bl_mlp_t** out) {
             hipMalloc(&m->m, sizeof(float) * kNParam) == hipSuccess &&
             hipMalloc(&m->v, sizeof(float) * kNParam) == hipSuccess &&
             hipMalloc(&m->g, sizeof(float) * kNParam) == hipSuccess &&
+            hipMalloc(&m->wr, sizeof(float) * kNParam) == hipSuccess &&
             hipMalloc(&m->w1p, sizeof(u64x2) * kW1Groups * 64) == hipSuccess &&
             hipMalloc(&m->w2p, sizeof(u64x2) * kW2Groups * 64) == hipSuccess &&
             hipMalloc(&m->w3p, sizeof(u64x2) * kW3Groups * 64) == hipSuccess &&
@@ -943,7 +1083,8 @@ int bl_mlp_create(uint64_t seed, int32_t capacity, bl_mlp_t** out) {
             hipMalloc(&m->feat, sizeof(float) * kIn * (size_t)std::max(capacity, 1)) == hipSuccess &&
             hipMalloc(&m->targ, sizeof(float) * kOut * (size_t)std::max(capacity, 1)) == hipSuccess &&
             hipMalloc(&m->count, sizeof(int32_t)) == hipSuccess &&
-            hipMalloc(&m->loss, sizeof(float)) == hipSuccess;
+            hipMalloc(&m->loss, sizeof(float) * kLossCap) == hipSuccess;
+  m->loss_cap = kLossCap;
   if (!ok) { set_error("bl_mlp_create: out of device memory"); bl_mlp_destroy(m); return BL_FAILURE; }
   // He-uniform initial weights from the seed (host), zero biases
   std::vector<float> w(kNParam, 0.0f);
@@ -978,7 +1119,7 @@ int bl_mlp_create(uint64_t seed, int32_t capacity, bl_mlp_t** out) {
 int bl_mlp_destroy(bl_mlp_t* m) {
   if (!m) return BL_SUCCESS;
   if (m->stream) hipStreamSynchronize(m->stream);
-  void* bufs[] = {m->w, m->m, m->v, m->g, m->w1p, m->w2p, m->w3p, m->bias, m->norm, m->feat,
+  void* bufs[] = {m->w, m->m, m->v, m->g, m->wr, m->w1p, m->w2p, m->w3p, m->bias, m->norm, m->feat,
                   m->targ, m->count, m->part, m->lpart, m->loss};
   for (void* p : bufs) if (p) hipFree(p);
   if (m->stream) hipStreamDestroy(m->stream);
@@ -1064,15 +1205,11 @@ int bl_mlp_gradient(bl_mlp_t* m, int32_t n, float* grad, float* loss) {
   int32_t c = 0;
   BL_HIP(hipMemcpy(&c, m->count, sizeof(int32_t), hipMemcpyDeviceToHost));
   if (n > c) { set_error("bl_mlp_gradient: more samples than pairs"); return BL_FAILURE; }
-  std::vector<int32_t> idx(n);
-  for (int i = 0; i < n; ++i) idx[i] = i;
-  int32_t* didx = nullptr;
-  BL_HIP(hipMalloc(&didx, sizeof(int32_t) * n));
-  hipMemcpy(didx, idx.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice);
-  int rc = mlp_gradient(m, didx, c, n, 0, 0);
-  hipStreamSynchronize(m->stream);
-  hipFree(didx);
-  if (rc) return BL_FAILURE;
+  if (mlp_round(m) || mlp_partials(m, 0, c, n, 0, 0)) return BL_FAILURE;
+  hipLaunchKernelGGL(k_mlp_reduce, dim3(kSumGrid), dim3(kSumBlock), 0, m->stream, train_blocks(n),
+                     (const float*)m->part, (const float*)m->lpart, m->g, m->loss, n);
+  BL_HIP(hipGetLastError());
+  BL_HIP(hipStreamSynchronize(m->stream));
   BL_HIP(hipMemcpy(grad, m->g, sizeof(float) * kNParam, hipMemcpyDeviceToHost));
   BL_HIP(hipMemcpy(loss, m->loss, sizeof(float), hipMemcpyDeviceToHost));
   return BL_SUCCESS;
@@ -1086,18 +1223,32 @@ int bl_mlp_train(bl_mlp_t* m, int32_t iters, int32_t batch, float lr, uint64_t s
   BL_HIP(hipMemcpy(&c, m->count, sizeof(int32_t), hipMemcpyDeviceToHost));
   if (c <= 0) { set_error("bl_mlp_train: no training pairs"); return BL_FAILURE; }
   if (!m->norm_set && mlp_normalize(m)) return BL_FAILURE;
-  std::vector<float> lh(iters);
+  if (iters > m->loss_cap) {
+    hipFree(m->loss);
+    m->loss = nullptr;
+    m->loss_cap = 0;
+    if (hipMalloc(&m->loss, sizeof(float) * (size_t)iters) != hipSuccess) {
+      set_error("mlp: out of device memory");
+      return BL_FAILURE;
+    }
+    m->loss_cap = iters;
+  }
+  // the losses stay on the device until the call's end: no host round trip
+  // between the steps (a copy of each one took a third of a step)
+  const int nblk = train_blocks(batch);
+  if (iters > 0 && mlp_round(m)) return BL_FAILURE;
   for (int it = 0; it < iters; ++it) {
-    if (mlp_gradient(m, nullptr, c, batch, seed, it)) return BL_FAILURE;
+    if (mlp_partials(m, 1, c, batch, seed, it)) return BL_FAILURE;
     ++m->adam_step;
-    hipLaunchKernelGGL(k_mlp_adam, dim3((kNParam + 255) / 256), dim3(256), 0, m->stream, m->w,
-                       m->m, m->v, (const float*)m->g, lr, m->adam_step);
-    if (loss_hist)
-      BL_HIP(hipMemcpyAsync(&lh[it], m->loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
+    hipLaunchKernelGGL(k_mlp_adam, dim3(kSumGrid), dim3(kSumBlock), 0, m->stream, nblk,
+                       (const float*)m->part, (const float*)m->lpart, m->loss + it, batch, m->w,
+                       m->wr, m->m, m->v, m->g, lr, m->adam_step);
+    BL_HIP(hipGetLastError());
   }
   if (mlp_pack(m)) return BL_FAILURE;
   BL_HIP(hipStreamSynchronize(m->stream));
-  if (loss_hist) std::copy(lh.begin(), lh.end(), loss_hist);
+  if (loss_hist && iters > 0)
+    BL_HIP(hipMemcpy(loss_hist, m->loss, sizeof(float) * (size_t)iters, hipMemcpyDeviceToHost));
   return BL_SUCCESS;
 }
 
