@@ -620,9 +620,8 @@ int bl_create(const bl_sizes_t* sizes, bl_handle_t** out) {
   if (hipMalloc(&h->d_part, sizeof(double) * 4 * h->npart) != hipSuccess ||
       hipMalloc(&h->d_parti, sizeof(int32_t) * 4 * h->npart) != hipSuccess ||
       hipMalloc(&h->d_ticket, sizeof(uint32_t) * 16) != hipSuccess ||
-      hipMalloc(&h->d_dtres, sizeof(DtResult)) != hipSuccess ||
+      hipMalloc(&h->d_state, 3 * sizeof(StepState)) != hipSuccess ||
       hipHostMalloc(&h->h_dtres, sizeof(DtResult)) != hipSuccess ||
-      hipMalloc(&h->d_ts, sizeof(DevTimestep)) != hipSuccess ||
       hipHostMalloc(&h->h_ts, sizeof(DevTimestep)) != hipSuccess ||
       hipHostMalloc(&h->h_pub_ts, sizeof(DevTimestep), hipHostMallocCoherent) != hipSuccess) {
     set_error("bl_create: out of device memory"); bl_destroy(h); return BL_FAILURE;
@@ -631,8 +630,9 @@ int bl_create(const bl_sizes_t* sizes, bl_handle_t** out) {
   // failed look-up is reported by that entry point, not here)
   if (!noalloc_scratch(h->device)) g_last_error.clear();
   hipMemsetAsync(h->d_ticket, 0, sizeof(uint32_t) * 16, h->stream);
-  hipMemsetAsync(h->d_dtres, 0, sizeof(DtResult), h->stream);
-  hipMemsetAsync(h->d_ts, 0, sizeof(DevTimestep), h->stream);
+  h->d_ts = &h->d_state[0].ts;
+  h->d_dtres = &h->d_state[0].res;
+  hipMemsetAsync(h->d_state, 0, 3 * sizeof(StepState), h->stream);
   if (hipStreamSynchronize(h->stream) != hipSuccess) {
     set_error("bl_create: initialisation failed"); bl_destroy(h); return BL_FAILURE;
   }
@@ -672,7 +672,7 @@ int bl_destroy(bl_handle_t* h) {
   void* bufs[] = {h->d_kappareg, h->d_pmeritreg, h->d_zdtnotreg, h->d_zmidlength,
                   h->d_eos_itype, h->d_eos_param, h->d_hyd_ptr, h->d_hyd_idx,
                   h->d_ale_ptr, h->d_ale_idx, h->d_el_ptr, h->d_el_idx, h->d_part,
-                  h->d_parti, h->d_ticket, h->d_dtres, h->d_ts, h->d_hist, h->d_outer,
+                  h->d_parti, h->d_ticket, h->d_state, h->d_lim, h->d_hist, h->d_outer,
                   h->d_diag_hist, h->d_diag_count, h->d_diag_part, h->d_ring, h->d_work, h->d_rest, h->d_vstats,
                   h->d_rlist, h->d_zlist, h->d_lflag, h->d_lmark, h->d_ld1, h->d_nbfc, h->d_cw[0], h->d_cw[1],
                   h->d_eoff, h->d_lboff, h->d_einst, h->d_ninst, h->d_inst, h->d_inst_dt, h->d_cnt,

@@ -350,8 +350,10 @@ namespace bl {
 
 // the per-step record of the fused step from the node set the step wrote
 int launch_diag(Handle* h, const double* ndx, const double* ndy, const double* ndu,
-                const double* ndv, const double* rho, const double* en, const double* pre) {
+                const double* ndv, const double* rho, const double* en, const double* pre,
+                const DevTimestep* ts) {
   if (!h->diag_on) return BL_SUCCESS;
+  if (!ts) ts = h->d_ts;
   if (!rho) rho = h->R(BL_ELDENSITY);
   if (!en) en = h->R(BL_ELENERGY);
   if (!pre) pre = h->R(BL_ELPRESSURE);
@@ -362,15 +364,15 @@ int launch_diag(Handle* h, const double* ndx, const double* ndy, const double* n
   BL_LAUNCH(h, "diag_shortprint", k_sp_elements<true>, nb, kBlock, nel, nreg, h->cfg.dencut,
             (const int32_t*)h->I(BL_IELREG), (const int32_t*)h->I(BL_IELND), rho, en, pre,
             (const double*)nullptr, (const double*)h->R(BL_ELMASS), (const double*)nullptr, ndx,
-            ndy, ndu, ndv, part, (const DevTimestep*)h->d_ts);
+            ndy, ndu, ndv, part, ts);
   BL_LAUNCH(h, "diag_l1", k_l1<true>, nb, kBlock, nel, (const int32_t*)h->I(BL_IELND), ndx, ndy,
             (const double*)nullptr, rho, en, h->diag_x0, h->diag_scale,
-            (const double*)&h->d_ts->time, 0.0, part2, (const DevTimestep*)h->d_ts);
+            (const double*)&ts->time, 0.0, part2, ts);
   double* col = part2 + (size_t)nb * kNq;
   BL_LAUNCH(h, "diag_columns", k_diag_columns, nreg * kNq + 3, kBlock, (int)nb, nreg,
-            (const double*)part, (const double*)part2, col, (const DevTimestep*)h->d_ts);
+            (const double*)part, (const double*)part2, col, ts);
   BL_LAUNCH(h, "diag_record", k_diag_record, 1, 64, nreg, (const double*)col,
-            h->d_diag_hist, h->d_diag_count, h->diag_max, (const DevTimestep*)h->d_ts);
+            h->d_diag_hist, h->d_diag_count, h->diag_max, ts);
   return BL_SUCCESS;
 }
 

@@ -31,6 +31,15 @@ struct FusedNodesOut {
   double* v;
 };
 
+// a limiter workgroup's first-index DIV maximum and CFL minimum
+struct alignas(32) LimPart {
+  double div, cfl;
+  int32_t di, ci;
+};
+// the limiter workgroups of a step on a tiling: two of 256 threads a CU is
+// all that its registers let run at once, and every tile reads every partial
+constexpr int kLimParts = 512;
+
 // everything a step kernel needs, passed by value (kernel argument space)
 struct FusedArgs {
   int nel, nnd;
@@ -116,6 +125,13 @@ struct FusedArgs {
   uint64_t* rest_next;
   DtResult* dtres;
   DevTimestep* ts;
+  // a step on a tiling: the state the step before left (its timestep and
+  // outcome), the timestep between the limiter pass and the tile step, and
+  // the limiter pass's nlim partials; ts and dtres are then the step's own
+  const StepState* before;
+  DevTimestep* mid;
+  struct LimPart* lim;
+  int nlim;
   double* hist;
   int hist_cap;
   MixArgs mx;  // mixed cells (mx.ncp == 0: none)

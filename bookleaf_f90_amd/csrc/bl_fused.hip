@@ -360,7 +360,8 @@ __device__ __forceinline__ void select_dt(const FusedArgs& A, double dt_prev, in
 // geometry_kn_checkvolume's error halts the reference; a step that moved
 // the nodes wrote the other node set.  Host and device form of the same
 // record (the host runs it for a batch's last step).
-__host__ __device__ inline void step_end(DevTimestep* ts, const DtResult* res) {
+template <typename TS>
+__device__ __forceinline__ void step_end(TS* ts, const DtResult* res) {
   if (!ts->open) return;
   ts->open = 0;
   if (res->negvol) {
@@ -384,22 +385,145 @@ __host__ __device__ inline void step_end(DevTimestep* ts, const DtResult* res) {
   }
 }
 
+// what step_end reads and changes, in registers; and a timestep copied word
+// by word (a struct copy would take a stack slot)
+struct StepEnd {
+  int32_t nstep, open, done, skip, err, err_idx, err_step, flips, cmflips, ale_tile;
+};
+__device__ __forceinline__ void copy_timestep(DevTimestep* to, const DevTimestep* from) {
+  static_assert(sizeof(DevTimestep) % 8 == 0, "whole words");
+  const uint64_t* a = reinterpret_cast<const uint64_t*>(from);
+  uint64_t* b = reinterpret_cast<uint64_t*>(to);
+#pragma unroll
+  for (int k = 0; k < (int)(sizeof(DevTimestep) / 8); ++k) b[k] = a[k];
+}
+
+// The limiter of one element by the four lanes of a quad, an edge each: edge
+// f's own ends and the two outer nodes of its limiter ratios are all a lane
+// gathers, the centroid, the largest elvisc term, the corner forces and the
+// shortest side come from the quad by register moves.  The arithmetic of each
+// edge is f1_viscosity's (and f1_cfl's side), in its order.  For the few
+// elements of a nearly empty pass: a quarter of the dependent square roots
+// and divisions of a lane that does a whole element (with every lane taken,
+// whole elements are faster: 95 against 162 us for a million).  Returns the
+// CFL term (the same in all four lanes).
+template <int CTRL>
+__device__ __forceinline__ double quad_move(double x) {
+  const int2 h = __builtin_bit_cast(int2, x);
+  return __builtin_bit_cast(double,
+                            make_int2(__builtin_amdgcn_mov_dpp(h.x, CTRL, 0xf, 0xf, true),
+                                      __builtin_amdgcn_mov_dpp(h.y, CTRL, 0xf, 0xf, true)));
+}
+__device__ __forceinline__ void quad_all(double x, double v[4]) {
+  v[0] = quad_move<0x00>(x);
+  v[1] = quad_move<0x55>(x);
+  v[2] = quad_move<0xaa>(x);
+  v[3] = quad_move<0xff>(x);
+}
+__device__ __forceinline__ double f1_moving_quad(const FusedArgs& A, const FusedNodes& N, int e,
+                                                 int f, bool live) {
+  const int g = (f + 1) & 3;
+  // edges 1 and 3 belong to limiter direction 0, edges 0 and 2 to direction 1
+  const int iside = (f & 1) ? 0 : 1;
+  const bool first = f == ((iside + 3) & 3);  // is1 of its direction, else is2
+  const int4 nd4 = reinterpret_cast<const int4*>(A.ielnd)[e];
+  const int4 nb4 = reinterpret_cast<const int4*>(A.ielel)[e];
+  const int nd[4] = {nd4.x - 1, nd4.y - 1, nd4.z - 1, nd4.w - 1};
+  const int nb[4] = {nb4.x - 1, nb4.y - 1, nb4.z - 1, nb4.w - 1};
+  const int* o = A.outer + 8 * (size_t)e + 4 * iside + (first ? 0 : 1);
+  const NodeUVXY oa = node_uvxy(N, o[0] - 1), ob = node_uvxy(N, o[2] - 1);
+  const NodeUVXY p0 = node_uvxy(N, f == 0 ? nd[0] : f == 1 ? nd[1] : f == 2 ? nd[2] : nd[3]);
+  const NodeUVXY p1 = node_uvxy(N, g == 0 ? nd[0] : g == 1 ? nd[1] : g == 2 ? nd[2] : nd[3]);
+  const int in1 = iside == 0 ? nb[0] : nb[1], in2 = iside == 0 ? nb[2] : nb[3];
+  const int ins = f == 0 ? nb[0] : f == 1 ? nb[1] : f == 2 ? nb[2] : nb[3];
+  const double cs2e = A.cs2[e], rhoe = A.rho[e], cs2n = A.cs2[ins], rhon = A.rho[ins];
+  const CflIn r = cfl_in(A, e);
+  double ou, ov, ox, oy, au, av, ax, ay, bu, bv, bx, by, sa, sb;
+  edge_diff(p0, p1, ou, ov, ox, oy);
+  // is1: own edge's end -> outer, outer -> its start; is2 the other way
+  if (first) {
+    edge_diff(p1, oa, au, av, ax, ay);
+    edge_diff(ob, p0, bu, bv, bx, by);
+  } else {
+    edge_diff(oa, p0, au, av, ax, ay);
+    edge_diff(p1, ob, bu, bv, bx, by);
+  }
+  limiter_ratios(ou, ov, ox, oy, au, av, ax, ay, bu, bv, bx, by, A.zerocut, sa, sb);
+  if (in1 == e) {
+    const int ic1 = iside == 0 ? nd[0] : nd[1], ic2 = iside == 0 ? nd[1] : nd[2];
+    sa = (A.indtype[ic1] < 0 && A.indtype[ic2] < 0 && in2 != e) ? 1.0 : 0.0;
+  }
+  if (in2 == e) {
+    const int ic1 = iside == 0 ? nd[2] : nd[3], ic2 = iside == 0 ? nd[3] : nd[0];
+    sb = (A.indtype[ic1] < 0 && A.indtype[ic2] < 0 && in1 != e) ? 1.0 : 0.0;
+  }
+  double t = -__builtin_inf();  // (leaves limiter_edge's term itself)
+  const double ed = limiter_edge(sa, sb, ou, ov, cs2e, cs2n, rhoe, rhon, A.cvisc1, A.cvisc2,
+                                 A.zerocut, t);
+  // the four terms in f1_viscosity's order: edges 3, 1, 0, 2
+  double tt[4], x[4], y[4];
+  quad_all(t, tt);
+  quad_all(p0.x, x);
+  quad_all(p0.y, y);
+  double ev = 0.0;
+  ev = dmax(ev, tt[3]);
+  ev = dmax(ev, tt[1]);
+  ev = dmax(ev, tt[0]);
+  ev = dmax(ev, tt[2]);
+  const double xc = 0.25 * (x[0] + x[1] + x[2] + x[3]);
+  const double yc = 0.25 * (y[0] + y[1] + y[2] + y[3]);
+  double ex, ey;
+  edge_viscosity(p0.x, p1.x, p0.y, p1.y, xc, yc, p1.u - p0.u, p1.v - p0.v, ed, ed, A.zerocut, ex,
+                 ey);
+  // corner f: its edge less the edge before it (quad_perm 3, 0, 1, 2)
+  const double qx = ex - quad_move<0x93>(ex), qy = ey - quad_move<0x93>(ey);
+  // the side f, f + 1 against f + 2, f + 3 (geometry_kn_dln), or the
+  // element's middle lines
+  double len;
+  if (r.mid) {
+    len = minlength(x, y, A.zcut, true);
+  } else {
+    const int h2 = (f + 2) & 3, h3 = (f + 3) & 3;
+    const double xs[4] = {p0.x, p1.x, h2 == 0 ? x[0] : h2 == 1 ? x[1] : h2 == 2 ? x[2] : x[3],
+                          h3 == 0 ? x[0] : h3 == 1 ? x[1] : h3 == 2 ? x[2] : x[3]};
+    const double ys[4] = {p0.y, p1.y, h2 == 0 ? y[0] : h2 == 1 ? y[1] : h2 == 2 ? y[2] : y[3],
+                          h3 == 0 ? y[0] : h3 == 1 ? y[1] : h3 == 2 ? y[2] : y[3]};
+    double side[4];
+    quad_all(dln_side(xs, ys, 0, 1, 2, 3, A.zcut), side);
+    len = dmin(dmin(dmin(side[0], side[1]), side[2]), side[3]);
+  }
+  if (live) {
+    A.cnviscx[4 * (size_t)e + f] = qx;
+    A.cnviscy[4 * (size_t)e + f] = qy;
+    if (f == 0) A.elvisc[e] = ev;
+  }
+  double c2 = cs2e + ev;
+  if (A.mx.ncp > 0) {
+    const int im = A.ielmat[e];
+    if (im < 0) c2 = mix_cs2(A.mx, -im - 1);
+  }
+  const double c = r.dtnot ? DBL_MAX : len / c2;
+  return (c == c) ? c : DBL_MAX;
+}
+
 // F1L: the elements in motion, found from the step's at-rest mask (bits
 // in A.rest, or the tile step's bytes in A.rest8) over this workgroup's run
 // of element blocks (its XCD's part of the mesh, as xcd_block deals them),
 // compacted chunk by chunk in LDS so that every lane of a pass has an
 // element, in element order.  Each workgroup also folds a slice of the nb1
 // partials of F1 (or of the step kernels that did F1's work) of each
-// control into its own, so that F1b reduces one (CFL, DIV) pair per F1L
-// workgroup: CFL at part + 3 * nb1, DIV at part + nb1 (first-index extrema
-// are associative, so the result is F1b's over all partials)
+// control into its own, so that what selects dt reduces one (CFL, DIV) pair
+// per F1L workgroup (first-index extrema are associative, so the result is
+// that over all partials).
+//
+// SEL (a step on a tiling): the pairs go to A.lim, and the tile step selects
+// dt from them (tile_select).  The first thread of the grid also records the
+// end of the step before (step_end) on the way from its state to A.mid, and
+// clears the outcome this step will write.  Without it: CFL at part + 3 * nb1,
+// DIV at part + nb1, for F1b.
+template <bool SEL>
 __global__ void __launch_bounds__(kBlock)
 k_f1_limiter(FusedArgs A, FusedNodes N, int nb1) {
-  if (step_skipped(A, A.ts)) return;
-  // the step before found a negative volume that F1b has not recorded yet:
-  // this step does nothing (F1b makes it so)
-  // (one group of loads: tested one by one each would wait for the last)
-  if (A.end_in_f1b && (A.dtres->negvol | A.dtres->negvol2 | A.dtres->negvol3)) return;
   __shared__ int32_t list[kScanPer * kBlock];
   __shared__ uint32_t wave_n[kBlock / 64];
   double best = DBL_MAX, dv = -1.0;
@@ -412,45 +536,76 @@ k_f1_limiter(FusedArgs A, FusedNodes N, int nb1) {
   const int k0 = lo + (int)threadIdx.x, kc = min(k0, nb1 - 1);
   const double fdv = A.part[kc], fcv = A.part[2 * nb1 + kc];
   const int fdi = A.parti[kc], fci = A.parti[2 * nb1 + kc];
-  const int nbe = (A.nel + kBlock - 1) / kBlock;
+  // blocks of elements dealt to the workgroups in runs
+  constexpr int kRun = SEL ? 64 : kBlock;
+  const int nbe = (A.nel + kRun - 1) / kRun;
   const int lb = xcd_block();
-  const int e0 = (int)(((long long)lb * nbe) / gridDim.x) * kBlock;
-  const int e1 = min(A.nel, (int)(((long long)(lb + 1) * nbe) / gridDim.x) * kBlock);
+  const int e0 = (int)(((long long)lb * nbe) / gridDim.x) * kRun;
+  const int e1 = min(A.nel, (int)(((long long)(lb + 1) * nbe) / gridDim.x) * kRun);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  uint32_t listed = 0;
   // a pass covers kScanPer elements per thread (from a multiple of 8, so a
   // thread's flags are one aligned 8-byte word of bytes, or 8 bits of one
   // 64-bit word) and lists all the pass's moving elements before any
   // limiter work, so that a range with few of them costs one scan and one
   // limiter pass
   const int span = kScanPer * (int)blockDim.x;
+  auto flags = [&](int b) -> uint32_t {  // bit k: element b + k moves
+    uint32_t mv = 0;
+    if (b >= e1) return mv;
+    if (A.rest8) {
+      if (b + kScanPer <= e1) {
+        const uint64_t w = *reinterpret_cast<const uint64_t*>(A.rest8 + b);
+#pragma unroll
+        for (int k = 0; k < kScanPer; ++k) mv |= (((w >> (8 * k)) & 0xffull) == 0) ? 1u << k : 0u;
+      } else {
+        for (int k = 0; b + k < e1; ++k) mv |= A.rest8[b + k] == 0 ? 1u << k : 0u;
+      }
+    } else {
+      const uint32_t rest = (uint32_t)(A.rest[b >> 6] >> (b & 63)) & 0xffu;
+      mv = ~rest & 0xffu;
+      if (b + kScanPer > e1) mv &= (1u << (e1 - b)) - 1u;
+    }
+    return mv;
+  };
+  // (the first pass's flags load beside the gate's)
+  uint32_t mv = flags(e0 + kScanPer * (int)threadIdx.x);
+  if (SEL) {
+    const DevTimestep* ts = &A.before->ts;
+    const DtResult* res = &A.before->res;
+    const int neg = res->negvol | res->negvol2 | res->negvol3;
+    const bool late = A.stop_at_time_end && ts->time >= A.time_end;
+    const bool skip = ts->done || late || (ts->open && neg);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      StepEnd m{ts->nstep, ts->open,     ts->done,    ts->skip,  ts->err,
+                ts->err_idx, ts->err_step, ts->flips, ts->cmflips, ts->ale_tile};
+      step_end(&m, res);
+      copy_timestep(A.mid, ts);
+      A.mid->open = m.open;
+      A.mid->done = skip ? 1 : m.done;
+      A.mid->skip = skip ? 1 : 0;
+      A.mid->err = m.err;
+      A.mid->err_idx = m.err_idx;
+      A.mid->err_step = m.err_step;
+      A.mid->flips = m.flips;
+      A.mid->cmflips = m.cmflips;
+      *A.dtres = DtResult{};
+    }
+    if (skip) return;
+  } else {
+    if (step_skipped(A, A.ts)) return;
+    // the step before found a negative volume that F1b has not recorded yet:
+    // this step does nothing (F1b makes it so)
+    // (one group of loads: tested one by one each would wait for the last)
+    if (A.end_in_f1b && (A.dtres->negvol | A.dtres->negvol2 | A.dtres->negvol3)) return;
+  }
+  uint32_t listed = 0;
   for (int c = e0; c < e1; c += span) {
     const int b = c + kScanPer * (int)threadIdx.x;  // this thread's first element
-    uint32_t mv = 0;                                 // bit k: element b + k moves
-    if (b < e1) {
-      if (A.rest8) {
-        if (b + kScanPer <= e1) {
-          const uint64_t w = *reinterpret_cast<const uint64_t*>(A.rest8 + b);
-#pragma unroll
-          for (int k = 0; k < kScanPer; ++k) mv |= (((w >> (8 * k)) & 0xffull) == 0) ? 1u << k : 0u;
-        } else {
-          for (int k = 0; b + k < e1; ++k) mv |= A.rest8[b + k] == 0 ? 1u << k : 0u;
-        }
-      } else {
-        const uint32_t rest = (uint32_t)(A.rest[b >> 6] >> (b & 63)) & 0xffu;
-        mv = ~rest & 0xffu;
-        if (b + kScanPer > e1) mv &= (1u << (e1 - b)) - 1u;
-      }
-    }
+    if (c != e0) mv = flags(b);
     // the block's exclusive prefix of the counts: within the wave by
-    // shuffles, then over the waves
+    // register moves, then over the waves
     const uint32_t cnt = (uint32_t)__popc(mv);
-    uint32_t incl = cnt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const uint32_t t = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += t;
-    }
+    const uint32_t incl = wave_prefix(cnt);
     if (lane == 63) wave_n[wid] = incl;
     __syncthreads();
     uint32_t base = 0, total = 0;
@@ -461,9 +616,24 @@ k_f1_limiter(FusedArgs A, FusedNodes N, int nb1) {
     uint32_t at = base + incl - cnt;
     for (uint32_t m = mv; m; m &= m - 1) list[at++] = b + __ffs(m) - 1;
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < total; i += blockDim.x) {
-      const int el = list[i];
-      better_min(best, bi, f1_moving(A, N, el), el + 1);
+    // whole elements while there are more than a quarter of the lanes left,
+    // then a quad each
+    uint32_t i = 0;
+    for (; 4 * (total - i) > blockDim.x; i += min(total - i, blockDim.x)) {
+      const uint32_t k = i + threadIdx.x;
+      if (k < total) {
+        const int el = list[k];
+        better_min(best, bi, f1_moving(A, N, el), el + 1);
+      }
+    }
+    if (i < total) {
+      const uint32_t k = i + (threadIdx.x >> 2);
+      // (whole waves: a quad past the end repeats the last element)
+      if (i + 16 * wid < total) {
+        const int el = list[min(k, total - 1)];
+        const double cfl = f1_moving_quad(A, N, el, threadIdx.x & 3, k < total);
+        better_min(best, bi, cfl, el + 1);
+      }
     }
     listed += total;
     __syncthreads();  // the list is refilled
@@ -477,10 +647,15 @@ k_f1_limiter(FusedArgs A, FusedNodes N, int nb1) {
     better_max(dv, di, A.part[k], A.parti[k]);
     better_min(best, bi, A.part[2 * nb1 + k], A.parti[2 * nb1 + k]);
   }
-  // (one pass of shuffles and one barrier for both)
   if (!(best == best)) best = DBL_MAX;  // a NaN never wins the strict '<' scan
-  block_reduce_div_cfl(dv, di, best, bi, A.part + nb1 + blockIdx.x, A.parti + nb1 + blockIdx.x,
-                       A.part + 3 * nb1 + blockIdx.x, A.parti + 3 * nb1 + blockIdx.x);
+  if (SEL) {
+    LimPart* o = A.lim + blockIdx.x;
+    block_reduce_div_cfl(dv, di, best, bi, &o->div, &o->di, &o->cfl, &o->ci);
+  } else {
+    block_reduce_div_cfl(dv, di, best, bi, A.part + nb1 + blockIdx.x,
+                         A.parti + nb1 + blockIdx.x, A.part + 3 * nb1 + blockIdx.x,
+                         A.parti + 3 * nb1 + blockIdx.x);
+  }
 }
 
 // F1b: one workgroup -- combine the partials of F1 and F1L, then the
@@ -504,7 +679,6 @@ __global__ void __launch_bounds__(kFinalBlock) k_f1b_select(FusedArgs A, int nb,
   if (threadIdx.x == 0) {
     if (skip) ts->done = 1;
     ts->skip = skip ? 1 : 0;
-    ts->bad = 0;
     A.dtres->negvol = 0;
     A.dtres->negvol2 = 0;
     A.dtres->negvol3 = 0;
@@ -943,7 +1117,6 @@ __device__ __forceinline__ void f2_element(const FusedArgs& A, const FusedNodes&
   // last: no load of the element passes this atomic
   if (check_volume && gh.vol < 0.0) {
     atomicMax(&A.dtres->negvol, e + 1);
-    A.ts->bad = 1;
   }
 }
 
@@ -1108,7 +1281,6 @@ __device__ __forceinline__ double f4_state_from(const FusedArgs& A, int e, doubl
   // last: no load of the element passes this atomic
   if (g.vol < 0.0) {
     atomicMax(&A.dtres->negvol2, e + 1);
-    A.ts->bad = 1;
   }
   return c2;
 }
@@ -1230,6 +1402,102 @@ __device__ __forceinline__ void ens_list(const FusedArgs& A, const EnsArgs& E, i
   if (moving && slot < (uint32_t)(E.eoff[k + 1] - E.eoff[k])) A.work[E.eoff[k] + slot] = e;
 }
 
+// A step on a tiling of few tiles selects its dt in every tile: the limiter pass's
+// partials (at most two a thread, loaded beside the tile's own first loads)
+// reduced by the workgroup, then hydro_dr_getdt's candidates and
+// time_dr_calc / time_dr_end as F1b does them, the same in every tile.  The
+// grid's first thread writes the step's state (A.ts, one the other tiles do
+// not read) and the history.  A selection launch of its own (F1b: one
+// workgroup, 5 us a step) cost more than the repeated reductions.  Returns
+// whether the step runs.
+__device__ __forceinline__ bool tile_select(const FusedArgs& A, double& dt, double& rdt,
+                                            bool& last) {
+  __shared__ double sv[2][kBlock / 64];
+  __shared__ int si[2][kBlock / 64];
+  const int tid = threadIdx.x;
+  static_assert(kLimParts == 2 * kBlock, "two partials a thread");
+  // (a repeated partial changes nothing)
+  const LimPart* qa = A.lim + min(tid, A.nlim - 1);
+  const LimPart* qb = A.lim + min(tid + kBlock, A.nlim - 1);
+  double dv = qa->div, cv = qa->cfl;
+  int di = qa->di, ci = qa->ci;
+  const double dvb = qb->div, cvb = qb->cfl;
+  const int dib = qb->di, cib = qb->ci;
+  const DevTimestep* m = A.mid;
+  const bool writer = blockIdx.x == 0 && tid == 0;
+  if (m->skip) {
+    if (writer) copy_timestep(A.ts, m);
+    return false;
+  }
+  better_max(dv, di, dvb, dib);
+  better_min(cv, ci, cvb, cib);
+  wave_reduce<false>(dv, di);
+  wave_reduce<true>(cv, ci);
+  if ((tid & 63) == 0) {
+    sv[0][tid >> 6] = dv; si[0][tid >> 6] = di;
+    sv[1][tid >> 6] = cv; si[1][tid >> 6] = ci;
+  }
+  __syncthreads();
+  dv = sv[0][0]; di = si[0][0];
+  cv = sv[1][0]; ci = si[1][0];
+#pragma unroll
+  for (int w = 1; w < kBlock / 64; ++w) {
+    better_max(dv, di, sv[0][w], si[0][w]);
+    better_min(cv, ci, sv[1][w], si[1][w]);
+  }
+  if (!(dv > DBL_MIN)) { dv = DBL_MIN; di = 0; }
+  double best;
+  int bidx, bsdt;
+  select_dt(A, m->dt, m->nstep, cv, ci, dv, di, best, bidx, bsdt);
+  const bool negative = cv < 0.0;            // hydro_kn_getdt.f90:75-78
+  const bool small = best < A.dt_min;        // time_dr_advance.f90:122-127
+  dt = best;
+  rdt = 1.0 / best;  // hydro_kn_getforce.f90:88 (w4 = 1/dt, once per call)
+  const double time = m->time + best;
+  const int nstep = m->nstep + 1;
+  // the batch's last step (the one after it would be skipped)
+  last = nstep == m->last_step || (A.stop_at_time_end && time >= A.time_end);
+  if (writer) {
+    DevTimestep* t = A.ts;
+    copy_timestep(t, m);
+    if (negative || small) {
+      t->err = negative ? 2 : 3;
+      t->done = 1;
+      t->skip = 1;
+      t->err_step = nstep;
+    } else {
+      t->open = 1;
+    }
+    if (!negative) {
+      t->nstep = nstep;
+      t->dt = best;
+      t->rdt = rdt;
+      t->idtel = bidx;
+      t->sdt = bsdt;
+      t->time = time;
+      t->dts = best;
+      t->last = last ? 1 : 0;
+      t->ale_on = A.zexist && time >= A.mintime && time <= A.maxtime;
+      const int k = m->hist_n;
+      if (A.hist && k < A.hist_cap) {
+        t->hist_n = k + 1;
+        A.hist[3 * k] = best;
+        A.hist[3 * k + 1] = (double)bidx;
+        A.hist[3 * k + 2] = (double)bsdt;
+      }
+    }
+  }
+  return !(negative || small);
+}
+
+// the same in a launch of its own, for the tilings of more tiles than
+// kSelectTiles
+__global__ void __launch_bounds__(kBlock) k_select(FusedArgs A) {
+  double dt, rdt;
+  bool last;
+  tile_select(A, dt, rdt, last);
+}
+
 // The partial slots of one workgroup of F1's terms: its DIV maximum and
 // CFL minimum to slots seg and 2 * nseg + seg.  Inactive lanes carry the
 // neutral values and an index that never wins a tie.
@@ -1246,7 +1514,7 @@ __device__ __forceinline__ void seg_collect(const FusedArgs& A, int seg, int nse
 // the corner weights and the volume at x^{n+1} are written for it.  MIX: mixed
 // cells take their components' force.
 // (three waves per SIMD: at most 168 VGPRs; LDS allows three workgroups)
-template <bool ALE, bool MIX>
+template <bool ALE, bool MIX, bool ENS, bool SELF>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3)))
 k_lag_tile(FusedArgs A, FusedNodes N, FusedNodesOut O, EnsArgs E) {
   // slot-fastest, so that a wave's lanes of one (quantity, corner) are
@@ -1268,29 +1536,34 @@ k_lag_tile(FusedArgs A, FusedNodes N, FusedNodesOut O, EnsArgs E) {
   const uint32_t cm = A.tile_ncm[nb + min(tid, nn - 1)];
   const int2 ent = A.tile_el[eb + min(tid, ne - 1)];
   const int4 q = A.tile_nd[eb + min(tid, ne - 1)];
-  const DevTimestep* ts = A.ts;
-  if (ts->skip || ens_pending(A, ts)) return;
+  double dt, rdt;
+  bool last;
+  int inst = 0;
+  if (SELF) {
+    if (!tile_select(A, dt, rdt, last)) return;
+  } else {
+    const DevTimestep* ts = A.ts;
+    if (ts->skip || (ENS && ens_pending(A, ts))) return;
+    dt = ts->dt;
+    rdt = ts->rdt;
+    last = ts->last != 0;
+    if (ENS) {  // an ensemble tile lies in one instance: its dt
+      inst = A.einst[A.tile_el[eb].x & 0x3fffffff];
+      dt = A.inst_dt[inst];
+      rdt = A.inst_rdt[inst];
+    }
+  }
   // the high bit of the node's entry: this tile writes it (other tiles
   // holding it compute the same values for their own elements)
   const int n = (int)(nv & 0x7fffffffu);
   const bool writes = own && (nv >> 31) != 0;
-  // an ensemble tile lies in one instance: its dt
-  int inst = 0;
-  double dt = ts->dt, rdt = ts->rdt;
-  if (A.einst) {
-    inst = A.einst[A.tile_el[eb].x & 0x3fffffff];
-    dt = A.inst_dt[inst];
-    rdt = A.inst_rdt[inst];
-  }
   // --- F2: every element around the tile's nodes, one per thread
   // (every thread's entry names an element of the tile)
   const int e = ent.x & 0x3fffffff;
   const uint32_t flags = active ? (uint32_t)ent.x >> 30 : 0u;
   const uint32_t slots = (uint32_t)ent.y;
-  // its at-rest bytes now and in the step before, and whether this is the
-  // batch's last step, read before any branch
+  // its at-rest bytes now and in the step before, read before any branch
   const bool at_rest = A.rest8[e] != 0, rest_before = A.rest8_prev[e] != 0;
-  const bool last = ts->last != 0;
   double fx[4], fy[4];
   bool zeroed = false;
   if (active) {
@@ -1409,7 +1682,7 @@ k_lag_tile(FusedArgs A, FusedNodes N, FusedNodesOut O, EnsArgs E) {
   }
   if (ALE) return;
   // an ensemble's next-step limiter reads its instance's worklist
-  if (A.einst) ens_list(A, E, inst, tid & 63, interior && moving, e);
+  if (ENS) ens_list(A, E, inst, tid & 63, interior && moving, e);
   seg_collect(A, t, A.nseg, interior, e, cflv, divv);
 }
 
@@ -1761,7 +2034,7 @@ __global__ void __launch_bounds__(kBlock) k_r5(AleArgs B, DevTimestep* tsw) {
 // wherever the mesh has one; the eleven kernels remain for meshes without.
 
 #define REMAP_TILE_GATE(T) \
-  if ((T)->skip || (T)->bad) return
+  if ((T)->skip || step_bad(T)) return
 
 // R1's face mass fluxes (and a negative volume of the moved mesh, which R3
 // finds in the five-kernel form)
@@ -1876,7 +2149,7 @@ k_remap_tile(AleArgs B, FusedArgs A, FusedNodes H, FusedNodesOut W, double* cm_o
   const int e = ent.x & 0x3fffffff;
   const bool own = active && (((uint32_t)ent.x >> 30) & kTileOwn);
   const uint32_t slots = (uint32_t)ent.y;
-  if (ts->bad) {
+  if (step_bad(ts)) {
     // a negative volume of the corrector leaves the components after the
     // predictor (of the predictor: before it)
     if (MIX && own && !A.dtres->negvol && A.ielmat[e] < 0) {
@@ -2256,6 +2529,27 @@ void tile_args(bl_handle_t* h, FusedArgs& A, int p, int s) {
   A.end_in_f1b = 1;
 }
 
+// a step on a tiling of parity p: its states, and the limiter pass's
+// workgroups (one per 64 elements at least: a small mesh's elements in motion
+// then spread over the chip)
+void select_args(bl_handle_t* h, FusedArgs& A, int p) {
+  A.before = h->d_state + p;
+  A.mid = &h->d_state[2].ts;
+  A.ts = &h->d_state[1 - p].ts;
+  A.dtres = &h->d_state[1 - p].res;
+  A.lim = static_cast<LimPart*>(h->d_lim);
+  A.nlim = std::max(1, std::min((int)nblocks(h->sz.nel, 64),
+                                std::min(h->tune_lim_grid, kLimParts)));
+}
+
+// The tilings whose tiles select dt themselves: at most two rounds of
+// workgroups (three on each of 256 CUs).  A step with the selection in the
+// tiles / in a launch of its own: Sedov 100^2 (56 tiles) 19.4 / 22.0 us, 300^2
+// (500) 23.4 / 25.3, 512^2 (1457) 37.8 / 39.2, 600^2 (2000) 49.0 / 46.3,
+// 1024^2 (5826) 99.6 / 91.2: every round of workgroups waits for the partials
+// again.
+constexpr int kSelectTiles = 2 * 3 * 256;
+
 // the two at-rest masks of a folded run: m[p] is the mask of a step that
 // starts from node set p
 void rest_masks(bl_handle_t* h, uint64_t* m[2]) {
@@ -2273,6 +2567,7 @@ int launch_f1_prologue(bl_handle_t* h, int p, int stop_at_time_end) {
     const int s = h->cur_set;
     tile_args(h, A, p, s);
     A.rest8_next = h->d_rest8 + (size_t)p * h->sz.nel;  // the first step's own bytes
+    A.ts = &h->d_state[p].ts;
     FusedNodes N{h->nodeset[s][0], h->nodeset[s][1], h->nodeset[s][2], h->nodeset[s][3]};
     BL_LAUNCH(h, "f1_seg", k_f1_seg, (unsigned)h->ntile, kBlock, A, N, EnsArgs{});
     return BL_SUCCESS;
@@ -2283,6 +2578,21 @@ int launch_f1_prologue(bl_handle_t* h, int p, int stop_at_time_end) {
   A.rest = m[p];
   FusedNodes N{h->nodeset[p][0], h->nodeset[p][1], h->nodeset[p][2], h->nodeset[p][3]};
   BL_LAUNCH(h, "f1_getdt", k_f1_getdt, nblocks(h->sz.nel), kBlock, A, N);
+  return BL_SUCCESS;
+}
+
+// the dt selection and the tile step
+template <bool ALE, bool MIX>
+int launch_lag_tile(bl_handle_t* h, const FusedArgs& A, const FusedNodes& N,
+                    const FusedNodesOut& O) {
+  if (h->ntile <= kSelectTiles) {
+    BL_LAUNCH(h, "lag_tile", (k_lag_tile<ALE, MIX, false, true>), (unsigned)h->ntile, kBlock, A, N,
+              O, EnsArgs{});
+  } else {
+    BL_LAUNCH(h, "select", k_select, 1, kBlock, A);
+    BL_LAUNCH(h, "lag_tile", (k_lag_tile<ALE, MIX, false, false>), (unsigned)h->ntile, kBlock, A,
+              N, O, EnsArgs{});
+  }
   return BL_SUCCESS;
 }
 
@@ -2298,22 +2608,20 @@ int launch_ale_step(bl_handle_t* h, int p, int stop_at_time_end) {
   FusedNodesOut O{h->nodeset[1 - s][0], h->nodeset[1 - s][1], h->nodeset[1 - s][2],
                   h->nodeset[1 - s][3]};
   tile_args(h, A, p, s);
+  select_args(h, A, p);
   A.cnmass = cm[p];
-  const unsigned nseg = (unsigned)A.nseg;
-  const unsigned nbl = std::min(nseg, (unsigned)h->tune_lim_grid);
-  BL_LAUNCH(h, "f1_limiter", k_f1_limiter, nbl, (unsigned)h->tune_lim_block, A, N, (int)nseg);
-  BL_LAUNCH(h, "f1b_select", k_f1b_select, 1, kF1bThreads, A, (int)nseg, (int)nbl);
-  if (A.mx.ncp > 0)
-    BL_LAUNCH(h, "lag_tile", (k_lag_tile<true, true>), (unsigned)h->ntile, kBlock, A, N, O,
-              EnsArgs{});
-  else
-    BL_LAUNCH(h, "lag_tile", (k_lag_tile<true, false>), (unsigned)h->ntile, kBlock, A, N, O,
-              EnsArgs{});
+  BL_LAUNCH(h, "f1_limiter", k_f1_limiter<true>, (unsigned)A.nlim, (unsigned)h->tune_lim_block, A,
+            N, A.nseg);
+  if (A.mx.ncp > 0 ? launch_lag_tile<true, true>(h, A, N, O)
+                   : launch_lag_tile<true, false>(h, A, N, O))
+    return BL_FAILURE;
   AleArgs B = make_ale(h, O);
+  B.ts = A.ts;
+  B.dtres = A.dtres;
   // node relaxation: the mesh velocity in buffers of its own (the components'
   // energies read the step's ubar after it)
   if (!h->cfg.zeul) {
-    if (mesh_motion(h, O.x, O.y, h->mesh_w[0], h->mesh_w[1], 0.0, h->d_ts)) return BL_FAILURE;
+    if (mesh_motion(h, O.x, O.y, h->mesh_w[0], h->mesh_w[1], 0.0, A.ts)) return BL_FAILURE;
     B.ubar = h->mesh_w[0];
     B.vbar = h->mesh_w[1];
   }
@@ -2335,8 +2643,8 @@ int launch_ale_step(bl_handle_t* h, int p, int stop_at_time_end) {
               cm[1 - p]);
   if (!h->diag_on) return BL_SUCCESS;
   // per-step diagnostics need the step's end first
-  BL_LAUNCH(h, "batch_end", k_batch_end, 1, 64, h->d_ts, (const DtResult*)h->d_dtres);
-  return launch_diag(h, W.x, W.y, W.u, W.v, R.rho_o, R.en_o, R.pre_o);
+  BL_LAUNCH(h, "batch_end", k_batch_end, 1, 64, A.ts, (const DtResult*)A.dtres);
+  return launch_diag(h, W.x, W.y, W.u, W.v, R.rho_o, R.en_o, R.pre_o, A.ts);
 }
 
 // one step (parity p: node set p -> node set 1-p), launched on h->stream
@@ -2353,17 +2661,15 @@ int launch_step(bl_handle_t* h, int p, int stop_at_time_end) {
   FusedNodes Oc{O.x, O.y, O.u, O.v};
   if (use_tiles(h)) {
     tile_args(h, A, p, p);
-    A.end_in_f1b = end_in_f1b(h) ? 1 : 0;  // with per-step diagnostics F5 ends the step
-    const unsigned nseg = (unsigned)A.nseg;
-    const unsigned nbl = std::min(nseg, (unsigned)h->tune_lim_grid);
-    BL_LAUNCH(h, "f1_limiter", k_f1_limiter, nbl, (unsigned)h->tune_lim_block, A, N, (int)nseg);
-    BL_LAUNCH(h, "f1b_select", k_f1b_select, 1, kF1bThreads, A, (int)nseg, (int)nbl);
-    BL_LAUNCH(h, "lag_tile", (k_lag_tile<false, false>), (unsigned)h->ntile, kBlock, A, N, O, EnsArgs{});
-    if (end_in_f1b(h)) return BL_SUCCESS;
-    // per-step diagnostics: F5 records the step's end, then the record of
-    // the node and element sets the step wrote
-    BL_LAUNCH(h, "f5_end", k_f5_end, 1, kBlock, A, Oc);
-    return launch_diag(h, O.x, O.y, O.u, O.v, A.rho_o, A.en_o, A.pre_o);
+    select_args(h, A, p);
+    BL_LAUNCH(h, "f1_limiter", k_f1_limiter<true>, (unsigned)A.nlim, (unsigned)h->tune_lim_block,
+              A, N, A.nseg);
+    if (launch_lag_tile<false, false>(h, A, N, O)) return BL_FAILURE;
+    if (!h->diag_on) return BL_SUCCESS;
+    // per-step diagnostics: the step's end, then the record of the node and
+    // element sets the step wrote
+    BL_LAUNCH(h, "batch_end", k_batch_end, 1, 64, A.ts, (const DtResult*)A.dtres);
+    return launch_diag(h, O.x, O.y, O.u, O.v, A.rho_o, A.en_o, A.pre_o, A.ts);
   }
   const unsigned nbl = std::min(nbe, (unsigned)h->tune_lim_grid);
   A.end_in_f1b = end_in_f1b(h) ? 1 : 0;
@@ -2378,7 +2684,8 @@ int launch_step(bl_handle_t* h, int p, int stop_at_time_end) {
   } else {
     BL_LAUNCH(h, "f1_getdt", k_f1_getdt, nbe, kBlock, A, N);
   }
-  BL_LAUNCH(h, "f1_limiter", k_f1_limiter, nbl, (unsigned)h->tune_lim_block, A, N, (int)nbe);
+  BL_LAUNCH(h, "f1_limiter", k_f1_limiter<false>, nbl, (unsigned)h->tune_lim_block, A, N,
+            (int)nbe);
   BL_LAUNCH(h, "f1b_select", k_f1b_select, 1, kF1bThreads, A, (int)nbe, (int)nbl);
   // F2 and F5 (or R1) take a workgroup per 256 mixed cells for the
   // component work; F2 puts them first, rounded up to whole XCD rounds
@@ -2451,6 +2758,7 @@ int ensure_nodesets(bl_handle_t* h) {
 // or the other forms' corner terms and remap temporaries.  After
 // prepare_tiles, outside any capture.
 int ensure_step_buffers(bl_handle_t* h) {
+  if (!h->d_lim) BL_HIP(hipMalloc(&h->d_lim, sizeof(LimPart) * kLimParts));
   const size_t nel = (size_t)std::max(h->sz.nel, 1), nnd = (size_t)std::max(h->sz.nnd, 1);
   auto alloc = [](double** p, size_t n) {
     if (*p) return hipSuccess;
@@ -2481,16 +2789,17 @@ int ensure_step_buffers(bl_handle_t* h) {
 // step may have left (F1L and F1b read them as the step before's outcome),
 // an ensemble's worklist lengths (a folded run call ends with the next
 // step's lists) and, with set_ts, the device timestep.
-__global__ void k_call_start(DevTimestep init, int set_ts, DevTimestep* __restrict__ ts,
-                             DtResult* __restrict__ dtres, uint64_t* __restrict__ rest,
+__global__ void k_call_start(DevTimestep init, int set_ts, StepState* __restrict__ state, int first,
+                             uint64_t* __restrict__ rest,
                              int64_t nrest, unsigned long long* __restrict__ vstats,
                              uint8_t* __restrict__ rest8, int64_t nrest8,
                              uint32_t* __restrict__ cnt, int ncnt) {
   const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   if (i0 == 0) {
-    *dtres = DtResult{};
-    if (set_ts) *ts = init;
+    state[0].res = DtResult{};
+    state[1].res = DtResult{};
+    if (set_ts) state[first].ts = init;
   }
   for (int64_t i = i0; i < nrest; i += stride) rest[i] = 0;
   for (int64_t i = i0; i < kStatWords; i += stride) vstats[i] = 0;
@@ -2504,7 +2813,9 @@ __global__ void k_call_start(DevTimestep init, int set_ts, DevTimestep* __restri
 // Forget which elements' viscosity fields hold F1's zeros (and the rest of
 // what k_call_start clears); with init, also write the device timestep.
 // keep_masks: a run call that continues the last one keeps the masks
-int clear_rest(bl_handle_t* h, const DevTimestep* init = nullptr, bool keep_masks = false) {
+// (to state first)
+int clear_rest(bl_handle_t* h, const DevTimestep* init = nullptr, bool keep_masks = false,
+               int first = 0) {
   const int64_t nrest = keep_masks ? 0 : 8 * (int64_t)nblocks(std::max(h->sz.nel, 1));
   const int64_t nrest8 = (h->d_rest8 && !keep_masks) ? 2 * (int64_t)std::max(h->sz.nel, 1) : 0;
   const int ncnt = (h->ens_n > 0 && h->d_cnt) ? h->ens_n : 0;
@@ -2512,7 +2823,7 @@ int clear_rest(bl_handle_t* h, const DevTimestep* init = nullptr, bool keep_mask
   const unsigned grid = (unsigned)std::min<int64_t>(1024, (most + kBlock - 1) / kBlock);
   DevTimestep none{};
   BL_LAUNCH(h, "call_start", k_call_start, std::max(grid, 1u), kBlock, init ? *init : none,
-            init ? 1 : 0, h->d_ts, h->d_dtres, h->d_rest, nrest, h->d_vstats, h->d_rest8,
+            init ? 1 : 0, h->d_state, first, h->d_rest, nrest, h->d_vstats, h->d_rest8,
             nrest8, h->d_cnt, ncnt);
   return BL_SUCCESS;
 }
@@ -2601,7 +2912,7 @@ static_assert(std::extent<decltype(bl::Handle::graph_exec)>::value >= (size_t)kG
               "the handle's graph table holds every step graph");
 inline int graph_index(int fin, int si, int p) { return 2 * kGraphLogs * fin + 2 * si + p; }
 
-int launch_batch_end(bl_handle_t* h, const DevTimestep* d_ts, int cur);
+int launch_batch_end(bl_handle_t* h, int state);
 
 // capture graph_exec[graph_index(fin, si, p)]; before any launch of a call
 int capture_graph(bl_handle_t* h, int fin, int si, int p, int stop_at_time_end) {
@@ -2612,7 +2923,7 @@ int capture_graph(bl_handle_t* h, int fin, int si, int p, int stop_at_time_end) 
   int rc = BL_SUCCESS;
   for (int k = 0; k < (1 << si) && rc == BL_SUCCESS; ++k)
     rc = launch_step(h, p ^ (k & 1), stop_at_time_end);
-  if (rc == BL_SUCCESS && fin) rc = launch_batch_end(h, h->d_ts, 0);
+  if (rc == BL_SUCCESS && fin) rc = launch_batch_end(h, p ^ ((1 << si) & 1));
   hipError_t e = hipStreamEndCapture(h->stream, &g);
   h->timing = timing;
   if (rc != BL_SUCCESS || e != hipSuccess) {
@@ -2714,24 +3025,25 @@ __global__ void k_publish(const DevTimestep* __restrict__ ts, const double* __re
 }
 
 // The batch's end: the open end of its last step, then the registry's
-// geometry at the final node set (from ts after the steps, or set cur with
-// ts null; the tile step's last step wrote rscratch23/24 itself), then the
-// results for the host
-int launch_batch_end(bl_handle_t* h, const DevTimestep* d_ts, int cur) {
+// geometry at the final node set (the tile step's last step wrote
+// rscratch23/24 itself), then the results for the host.  state: the state
+// the last step of a batch on a tiling left
+int launch_batch_end(bl_handle_t* h, int state) {
   const bool ale = ale_tiles(h);
-  if (end_in_f1b(h) || ale)
-    BL_LAUNCH(h, "batch_end", k_batch_end, 1, 64, h->d_ts, (const DtResult*)h->d_dtres);
-  const int nel = h->sz.nel;
   const bool tiles = use_tiles(h) || ale;
+  StepState* st = h->d_state + (tiles ? state : 0);
+  if (end_in_f1b(h) || tiles)
+    BL_LAUNCH(h, "batch_end", k_batch_end, 1, 64, &st->ts, (const DtResult*)&st->res);
+  const int nel = h->sz.nel;
   BL_LAUNCH(h, "materialize", k_materialize, nblocks(nel), kBlock, nel, h->I(BL_IELND),
-            h->nodeset[0][0], h->nodeset[0][1], h->nodeset[1][0], h->nodeset[1][1], d_ts, cur,
-            h->R(BL_CNX), h->R(BL_CNY), h->R(BL_A1), h->R(BL_A2), h->R(BL_A3), h->R(BL_B1),
+            h->nodeset[0][0], h->nodeset[0][1], h->nodeset[1][0], h->nodeset[1][1],
+            (const DevTimestep*)&st->ts, 0, h->R(BL_CNX), h->R(BL_CNY), h->R(BL_A1), h->R(BL_A2), h->R(BL_A3), h->R(BL_B1),
             h->R(BL_B2), h->R(BL_B3), h->R(BL_CNWT), h->R(BL_ELVOLUME),
             tiles ? nullptr : (const double*)h->cterm[0],
             tiles ? nullptr : (const double*)h->cterm[1], h->R(BL_RSCRATCH23),
             h->R(BL_RSCRATCH24), h->R(BL_CNMASS),
             ale ? (const double*)h->cm_other : nullptr);
-  BL_LAUNCH(h, "publish", k_publish, 1, kBlock, (const DevTimestep*)h->d_ts,
+  BL_LAUNCH(h, "publish", k_publish, 1, kBlock, (const DevTimestep*)&st->ts,
             (const double*)h->d_hist, h->h_pub_ts, h->h_pub_hist, (int)h->hist_cap);
   return BL_SUCCESS;
 }
@@ -2793,7 +3105,8 @@ int launch_ensemble_step(bl_handle_t* h, int p) {
     BL_LAUNCH(h, "e1_limiter", k_e1_limiter, (unsigned)h->ens_lblocks,
               (unsigned)h->tune_lim_block, A, N, E);
     BL_LAUNCH(h, "e1b_select", k_e1b_select, (unsigned)h->ens_n, kBlock, A, E, (int)h->ntile);
-    BL_LAUNCH(h, "lag_tile", (k_lag_tile<false, false>), (unsigned)h->ntile, kBlock, A, N, O, E);
+    BL_LAUNCH(h, "lag_tile", (k_lag_tile<false, false, true, false>), (unsigned)h->ntile, kBlock, A, N,
+              O, E);
     BL_LAUNCH(h, "f5_end", k_f5_end, 1, kBlock, A, Oc);
     return BL_SUCCESS;
   }
@@ -3068,7 +3381,7 @@ int bl_autotune(bl_handle_t* h, int32_t reps, bl_tuning_t* out) {
             hipLaunchKernelGGL(k_e1_limiter, dim3(h->ens_lblocks), dim3(block), 0, h->stream, A,
                                N, E);
           else
-            hipLaunchKernelGGL(k_f1_limiter, dim3(std::min(nbe, (unsigned)second)), dim3(block),
+            hipLaunchKernelGGL(k_f1_limiter<false>, dim3(std::min(nbe, (unsigned)second)), dim3(block),
                                0, h->stream, A, N, (int)nbe);
           hipEventRecord(e1, h->stream);
           if (hipGetLastError() != hipSuccess || hipEventSynchronize(e1) != hipSuccess) {
@@ -3284,8 +3597,8 @@ int bl_run_graph(bl_handle_t* h, int32_t nsteps, int32_t stop_at_time_end, bl_ti
   d->last_step = ts->nstep + nsteps;
   d->set0 = h->cur_set;
   d->ale_tile = ale ? 1 : 0;
-  if (clear_rest(h, d, resume)) return BL_FAILURE;
   const bool tiles = use_tiles(h) || ale;
+  if (clear_rest(h, d, resume, tiles ? p0 : 0)) return BL_FAILURE;
   int p = p0;
   // F1 of the first step: on a resumed call the last call's last step left
   // its terms, its at-rest mask and the zeros it stands for
@@ -3302,7 +3615,7 @@ int bl_run_graph(bl_handle_t* h, int32_t nsteps, int32_t stop_at_time_end, bl_ti
   // whose F3 ran flipped; the device knows how many did), then one read of
   // the timestep, the dt history (at most one entry per step) and the error
   // state
-  if (plan.empty() && launch_batch_end(h, h->d_ts, 0)) return BL_FAILURE;
+  if (plan.empty() && launch_batch_end(h, p)) return BL_FAILURE;
   if (!h->cfg.zexist && mix_cpu_overlay(h, nullptr)) return BL_FAILURE;
   // the batch's end published the timestep and the history (k_publish)
   BL_HIP(hipStreamSynchronize(h->stream));

@@ -71,9 +71,6 @@ struct DevTimestep {
   int32_t open;
   // the node set the batch started from (the final one is set0 + flips)
   int32_t set0;
-  // the step running found a negative volume before its remap: the kernels
-  // after the tile step do nothing (cleared by F1b)
-  int32_t bad;
   // the batch's steps end with the tiled remap, which puts each step's state
   // back into the node and element set the step started from; and the steps
   // whose remap ran (they alternate the two corner-mass arrays)
@@ -81,6 +78,22 @@ struct DevTimestep {
   int32_t cmflips;
 };
 constexpr int32_t kNoPending = 0x7fffffff;
+
+// The device timestep and the outcome of the step it describes, side by
+// side.  The steps on a tiling alternate between two of them (bl_fused.hip);
+// every other form works in the first.
+struct StepState {
+  DevTimestep ts;
+  DtResult res;
+};
+// whether the step of ts found a negative volume before its remap: the
+// kernels after the Lagrangian part do nothing
+#if defined(__HIPCC__)
+__host__ __device__ inline bool step_bad(const DevTimestep* ts) {
+  const DtResult& r = reinterpret_cast<const StepState*>(ts)->res;
+  return (r.negvol | r.negvol2) != 0;
+}
+#endif
 
 // per-launch kernel timing with HIP events on the handle's stream
 struct TimingClass {
@@ -126,11 +139,15 @@ struct Handle {
   double* d_part = nullptr;  // 4 doubles per workgroup
   int32_t* d_parti = nullptr;
   uint32_t* d_ticket = nullptr;  // 4 counters
-  DtResult* d_dtres = nullptr;
+  // [0] and [1]: the states the steps alternate between; [2].ts: between the
+  // limiter pass and the tile step
+  StepState* d_state = nullptr;
+  DtResult* d_dtres = nullptr;  // d_state[0].res
   DtResult* h_dtres = nullptr;  // pinned
   int64_t npart = 0;
   // fused-step state
-  DevTimestep* d_ts = nullptr;
+  DevTimestep* d_ts = nullptr;  // d_state[0].ts
+  void* d_lim = nullptr;        // the limiter pass's partials of a step on a tiling
   DevTimestep* h_ts = nullptr;  // pinned
   double* d_hist = nullptr;     // dt history (3 values per step)
   // what a run call's end publishes for the host (pinned, coherent host
@@ -290,7 +307,7 @@ int relax_rebuild(Handle* h);
 // element state it wrote: the registry's unless given)
 int launch_diag(Handle* h, const double* ndx, const double* ndy, const double* ndu,
                 const double* ndv, const double* rho = nullptr, const double* en = nullptr,
-                const double* pre = nullptr);
+                const double* pre = nullptr, const DevTimestep* ts = nullptr);
 // ensembles: the limiter pass's workgroups per instance for a chunk of
 // elements each (bl_ensemble.hip)
 int ens_set_chunk(Handle* h, int chunk);

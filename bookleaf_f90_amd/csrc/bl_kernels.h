@@ -56,6 +56,21 @@ __device__ __forceinline__ double lane_value(double x, int lane) {
   return __builtin_bit_cast(double, make_int2(lane_value(h.x, lane), lane_value(h.y, lane)));
 }
 
+// the wave's inclusive prefix sum (whole waves only)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t x) {
+  x += dpp_or_zero<0x111, 0xf>(x);
+  x += dpp_or_zero<0x112, 0xf>(x);
+  x += dpp_or_zero<0x114, 0xf>(x);
+  x += dpp_or_zero<0x118, 0xf>(x);
+  x += dpp_or_zero<0x142, 0xa>(x);
+  x += dpp_or_zero<0x143, 0xc>(x);
+  return x;
+}
+
 // the wave's first-index minimum (maximum) of (v, i), in every lane: the
 // extreme value, the smallest index that has it, and that lane's own value
 // (whole waves only; no NaN)

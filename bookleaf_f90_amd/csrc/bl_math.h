@@ -199,8 +199,46 @@ __device__ __forceinline__ double limiter_edge(double s1, double s2, double du, 
   return w3;
 }
 
-// hydro_kn_geteviscosity for one element (hydro_kn_edgeviscosity.f90:219-282):
-// edge coefficients in ed[4] (edviscx = edviscy on entry), out: corner forces
+// One edge of hydro_kn_geteviscosity (hydro_kn_edgeviscosity.f90:219-282):
+// from its ends (x1, y1), (x2, y2), the element's centroid, the velocity
+// difference along it and its coefficients, the edge's viscosity (ex, ey)
+__device__ __forceinline__ void edge_viscosity(double x1, double x2, double y1, double y2,
+                                               double xc, double yc, double uhat, double vhat,
+                                               double edx_in, double edy_in, double zerocut,
+                                               double& ex, double& ey) {
+  double w1 = x1, w2 = x2;
+  double w3 = 0.5 * (w1 + w2);
+  w1 = w2 - w1;
+  w2 = xc;
+  double w4 = y1, w5 = y2;
+  double w6 = 0.5 * (w4 + w5);
+  w4 = w5 - w4;
+  w5 = yc;
+  double w7 = sqrt((w2 - w3) * (w2 - w3) + (w5 - w6) * (w5 - w6));
+  double w8 = sqrt(w1 * w1 + w4 * w4);
+  double den = 1.0 / w7;
+  double xhat = (w5 - w6) * den;
+  double yhat = (w3 - w2) * den;
+  den = 1.0 / w8;
+  w1 = w1 * den;
+  w2 = w4 * den;
+  w3 = xhat * w1 + yhat * w2;
+  den = -(dsign(1.0, w3) * w7);
+  xhat = xhat * den;
+  yhat = yhat * den;
+  w5 = sqrt((uhat * uhat) + (vhat * vhat));
+  w6 = uhat * xhat + vhat * yhat;
+  den = w6 / dmax(w5, zerocut);
+  ex = edx_in * uhat * den;
+  ey = edy_in * vhat * den;
+  if (w5 <= zerocut || w6 <= zerocut || w7 <= zerocut || w8 <= zerocut) {
+    ex = 0.0;
+    ey = 0.0;
+  }
+}
+
+// hydro_kn_geteviscosity for one element: edge coefficients in ed[4]
+// (edviscx = edviscy on entry), out: corner forces
 __device__ __forceinline__ void geteviscosity(const double x[4], const double y[4],
                                               const double u[4], const double v[4],
                                               const double edx_in[4], const double edy_in[4],
@@ -210,38 +248,9 @@ __device__ __forceinline__ void geteviscosity(const double x[4], const double y[
   double yc = 0.25 * (y[0] + y[1] + y[2] + y[3]);
 #pragma unroll
   for (int is = 0; is < 4; ++is) {
-    int in = (is + 1) & 3;
-    double w1 = x[is], w2 = x[in];
-    double w3 = 0.5 * (w1 + w2);
-    w1 = w2 - w1;
-    w2 = xc;
-    double w4 = y[is], w5 = y[in];
-    double w6 = 0.5 * (w4 + w5);
-    w4 = w5 - w4;
-    w5 = yc;
-    double w7 = sqrt((w2 - w3) * (w2 - w3) + (w5 - w6) * (w5 - w6));
-    double w8 = sqrt(w1 * w1 + w4 * w4);
-    double den = 1.0 / w7;
-    double xhat = (w5 - w6) * den;
-    double yhat = (w3 - w2) * den;
-    den = 1.0 / w8;
-    w1 = w1 * den;
-    w2 = w4 * den;
-    w3 = xhat * w1 + yhat * w2;
-    den = -(dsign(1.0, w3) * w7);
-    xhat = xhat * den;
-    yhat = yhat * den;
-    double uhat = u[in] - u[is];
-    double vhat = v[in] - v[is];
-    w5 = sqrt((uhat * uhat) + (vhat * vhat));
-    w6 = uhat * xhat + vhat * yhat;
-    den = w6 / dmax(w5, zerocut);
-    edx[is] = edx_in[is] * uhat * den;
-    edy[is] = edy_in[is] * vhat * den;
-    if (w5 <= zerocut || w6 <= zerocut || w7 <= zerocut || w8 <= zerocut) {
-      edx[is] = 0.0;
-      edy[is] = 0.0;
-    }
+    const int in = (is + 1) & 3;
+    edge_viscosity(x[is], x[in], y[is], y[in], xc, yc, u[in] - u[is], v[in] - v[is], edx_in[is],
+                   edy_in[is], zerocut, edx[is], edy[is]);
   }
   qx[0] = edx[0] - edx[3]; qx[1] = edx[1] - edx[0];
   qx[2] = edx[2] - edx[1]; qx[3] = edx[3] - edx[2];

@@ -333,7 +333,7 @@ __global__ void __launch_bounds__(256) k_mlp_nodes(MlpPacked W, const float* __r
                                                    int32_t* __restrict__ mark,
                                                    int32_t* __restrict__ flag,
                                                    const DevTimestep* ts) {
-  if (ts && (ts->skip || ts->bad || !ts->ale_on)) return;
+  if (ts && (ts->skip || step_bad(ts) || !ts->ale_on)) return;
   if (ts) dt = ts->dt;
   if ((int)blockIdx.x >= nbm) {
     const int i = ((int)blockIdx.x - nbm) * blockDim.x + threadIdx.x;
@@ -478,7 +478,7 @@ __global__ void k_learned_check(int nel, const int32_t* __restrict__ ielnd,
                                 const float2* __restrict__ d1, double dt, double amax2,
                                 int relative, int stage, int32_t* __restrict__ mark,
                                 int32_t* __restrict__ flag, const DevTimestep* ts) {
-  if (ts && (ts->skip || ts->bad || !ts->ale_on)) return;
+  if (ts && (ts->skip || step_bad(ts) || !ts->ale_on)) return;
   if (ts) dt = ts->dt;
   const int stride = gridDim.x * blockDim.x;
   for (int e = xcd_index(); e < nel; e += stride)
@@ -497,7 +497,7 @@ __global__ void k_learned_recheck(int nel, const int32_t* __restrict__ ielnd,
                                   int relative, const int32_t* __restrict__ rlist, int nr,
                                   int32_t* __restrict__ mark, int32_t* __restrict__ flag,
                                   const DevTimestep* ts) {
-  if (ts && (ts->skip || ts->bad || !ts->ale_on)) return;
+  if (ts && (ts->skip || step_bad(ts) || !ts->ale_on)) return;
   if (flag[4] == 0) return;
   if (ts) dt = ts->dt;
   const int stride = gridDim.x * blockDim.x;
@@ -567,7 +567,7 @@ __global__ void k_collect(RelaxArgs RA, const int32_t* __restrict__ rlist, int n
                           const double* __restrict__ wv, double dt,
                           const int32_t* __restrict__ count, int cap, float* __restrict__ feat,
                           float* __restrict__ targ, const DevTimestep* ts) {
-  if (ts && (ts->skip || ts->bad || !ts->ale_on)) return;
+  if (ts && (ts->skip || step_bad(ts) || !ts->ale_on)) return;
   if (ts) dt = ts->dt;
   const int phase = collect_phase(stride, ts);
   const int take = nr > phase ? (nr - phase + stride - 1) / stride : 0;
@@ -587,7 +587,7 @@ __global__ void k_collect(RelaxArgs RA, const int32_t* __restrict__ rlist, int n
 
 __global__ void k_collect_end(int32_t* __restrict__ count, int nr, int stride, int cap,
                               const DevTimestep* ts) {
-  if (ts && (ts->skip || ts->bad || !ts->ale_on)) return;
+  if (ts && (ts->skip || step_bad(ts) || !ts->ale_on)) return;
   const int phase = collect_phase(stride, ts);
   const int take = nr > phase ? (nr - phase + stride - 1) / stride : 0;
   if (threadIdx.x == 0 && *count + take <= cap) *count = *count + take;

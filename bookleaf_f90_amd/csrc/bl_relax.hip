@@ -23,7 +23,7 @@
 namespace bl {
 
 #define RELAX_GATE(ts) \
-  if (((ts) && ((ts)->skip || (ts)->bad || !(ts)->ale_on)) || (R.only_if && *R.only_if == 0)) return
+  if (((ts) && ((ts)->skip || step_bad(ts) || !(ts)->ale_on)) || (R.only_if && *R.only_if == 0)) return
 
 __global__ void k_relax_sweep(RelaxArgs R, const double* __restrict__ xi,
                               const double* __restrict__ yi, double* __restrict__ xo,
