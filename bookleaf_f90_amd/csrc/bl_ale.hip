@@ -20,15 +20,8 @@
 
 namespace bl {
 
-// Inside a captured step (ts != null) the kernels do nothing when the step is
-// gated off or ALE is inactive (ale_active, ale_dr_utils.f90:35-51), and take
-// dt from the device timestep.
-#define ALE_GATE(ts) \
-  if ((ts) && ((ts)->skip || !(ts)->ale_on)) return
-
 // ale_kn_getmeshstatus (Eulerian, or node relaxation: indstatus = 2)
-__global__ void k_meshstatus(int nnd, int32_t* __restrict__ st, const DevTimestep* ts) {
-  ALE_GATE(ts);
+__global__ void k_meshstatus(int nnd, int32_t* __restrict__ st) {
   int i = xcd_index();
   if (i < nnd) st[i] = 2;
 }
@@ -38,9 +31,7 @@ __global__ void k_meshstatus(int nnd, int32_t* __restrict__ st, const DevTimeste
 __global__ void k_fluxvol_nodes(int nnd, int zeul, double dt, double* __restrict__ st4,
                                 double* __restrict__ st5, double* __restrict__ st2,
                                 double* __restrict__ st3, double* __restrict__ ndx,
-                                double* __restrict__ ndy, const DevTimestep* ts) {
-  ALE_GATE(ts);
-  if (ts) dt = ts->dt;
+                                double* __restrict__ ndy) {
   int i = xcd_index();
   if (i >= nnd) return;
   double u = st4[i], v = st5[i];
@@ -56,8 +47,7 @@ __global__ void k_fluxvol_nodes(int nnd, int zeul, double dt, double* __restrict
 __global__ void k_fluxvol_faces(int nel, double cut, const int32_t* __restrict__ ielnd,
                                 const double* __restrict__ x0, const double* __restrict__ y0,
                                 const double* __restrict__ x1, const double* __restrict__ y1,
-                                double* __restrict__ fcdv, const DevTimestep* ts) {
-  ALE_GATE(ts);
+                                double* __restrict__ fcdv) {
   int e = xcd_index();
   if (e >= nel) return;
   int4 nd4 = reinterpret_cast<const int4*>(ielnd)[e];
@@ -78,9 +68,7 @@ __global__ void k_fluxvol_faces(int nel, double cut, const int32_t* __restrict__
 __global__ void k_el1(int nel, int id1, int id2, const int32_t* __restrict__ ielel,
                       const int32_t* __restrict__ ielfc, const double* __restrict__ fcdv,
                       const double* __restrict__ cnwt, const double* __restrict__ rho,
-                      double* __restrict__ rwork1, double* __restrict__ fcdm,
-                      const DevTimestep* ts) {
-  ALE_GATE(ts);
+                      double* __restrict__ rwork1, double* __restrict__ fcdm) {
   int e = xcd_index();
   if (e >= nel) return;
   NbFc c = load_nbfc(e, ielel, ielfc);
@@ -100,9 +88,7 @@ __global__ void k_el2(int nel, int id1, int id2, double zerocut, double dencut,
                       double* __restrict__ cutm, double* __restrict__ vpr,
                       double* __restrict__ mpr, double* __restrict__ dpr,
                       double* __restrict__ vol, double* __restrict__ mass,
-                      double* __restrict__ rho, double* __restrict__ flux,
-                      const DevTimestep* ts) {
-  ALE_GATE(ts);
+                      double* __restrict__ rho, double* __restrict__ flux) {
   int e = xcd_index();
   if (e >= nel) return;
   NbFc c = load_nbfc(e, ielel, ielfc);
@@ -127,8 +113,7 @@ __global__ void k_el3(int nel, int id1, int id2, const int32_t* __restrict__ iel
                       const int32_t* __restrict__ ielfc, const double* __restrict__ flux,
                       const double* __restrict__ mpr, const double* __restrict__ mass,
                       const double* __restrict__ cutm, double* __restrict__ rwork1,
-                      double* __restrict__ en, const DevTimestep* ts) {
-  ALE_GATE(ts);
+                      double* __restrict__ en) {
   int e = xcd_index();
   if (e >= nel) return;
   NbFc c = load_nbfc(e, ielel, ielfc);
@@ -147,8 +132,7 @@ __global__ void k_nd1(int nel, int id1, int id2, const int32_t* __restrict__ iel
                       double* __restrict__ cnu, double* __restrict__ cnv,
                       double* __restrict__ cnm0, double* __restrict__ cndv,
                       double* __restrict__ cndm, double* __restrict__ cnflux,
-                      double* __restrict__ cnmass, const DevTimestep* ts) {
-  ALE_GATE(ts);
+                      double* __restrict__ cnmass) {
   int e = xcd_index();
   if (e >= nel) return;
   int4 nd = reinterpret_cast<const int4*>(ielnd)[e];
@@ -195,20 +179,41 @@ __global__ void k_nd2(int nnd, const int32_t* __restrict__ ptr, const int32_t* _
                       const double* __restrict__ cnflux, double* __restrict__ ndv0,
                       double* __restrict__ ndv1, double* __restrict__ ndm0,
                       double* __restrict__ ndm1, double* __restrict__ cutv,
-                      double* __restrict__ cutm, const DevTimestep* ts) {
-  ALE_GATE(ts);
+                      double* __restrict__ cutm) {
   int n = xcd_index();
   if (n >= nnd) return;
   double v0 = 0.0, v1 = 0.0, m0 = 0.0;
-  int b = ptr[n], end = ptr[n + 1];
-  for (int k = b; k < end; ++k) {
-    int c = idx[k], e = c >> 2;
-    v0 = v0 + 0.25 * elv0[e];
-    v1 = v1 + 0.25 * elv1[e];
-    m0 = m0 + cnm0[c];
+  const int b = ptr[n], end = ptr[n + 1];
+  // four incidences a pass, every value loaded before any is added
+  double f[4];
+  for (int k = b; k < end; k += 4) {
+    int c[4];
+    double a0[4], a1[4], q[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) c[r] = idx[min(k + r, end - 1)];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      a0[r] = elv0[c[r] >> 2];
+      a1[r] = elv1[c[r] >> 2];
+      q[r] = cnm0[c[r]];
+      f[r] = cnflux[c[r]];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (k + r < end) {
+        v0 = v0 + 0.25 * a0[r];
+        v1 = v1 + 0.25 * a1[r];
+        m0 = m0 + q[r];
+      }
   }
   double m1 = m0;
-  for (int k = b; k < end; ++k) m1 = m1 + cnflux[idx[k]];
+  if (end - b <= 4) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (b + r < end) m1 = m1 + f[r];
+  } else {
+    for (int k = b; k < end; ++k) m1 = m1 + cnflux[idx[k]];
+  }
   ndv0[n] = v0; ndv1[n] = v1; ndm0[n] = m0; ndm1[n] = m1;
   cutv[n] = zerocut;
   cutm[n] = dencut * v0;
@@ -218,8 +223,7 @@ __global__ void k_nd2(int nnd, const int32_t* __restrict__ ptr, const int32_t* _
 __global__ void k_fluxndvl(int nel, const int32_t* __restrict__ ielel,
                            const int32_t* __restrict__ ielfc, const double* __restrict__ cb,
                            const double* __restrict__ cdb, const double* __restrict__ var,
-                           double* __restrict__ cnflux, const DevTimestep* ts) {
-  ALE_GATE(ts);
+                           double* __restrict__ cnflux) {
   int e = xcd_index();
   if (e >= nel) return;
   NbFc c = load_nbfc(e, ielel, ielfc);
@@ -242,12 +246,21 @@ __global__ void k_updatend(int nnd, const int32_t* __restrict__ ptr,
                            const double* __restrict__ base1, double* __restrict__ base1_out,
                            const double* __restrict__ cut,
                            const double* __restrict__ cnflux, double* __restrict__ ndflux,
-                           double* __restrict__ var, const DevTimestep* ts) {
-  ALE_GATE(ts);
+                           double* __restrict__ var) {
   int n = xcd_index();
   if (n >= nnd) return;
   double s = 0.0;
-  for (int k = ptr[n]; k < ptr[n + 1]; ++k) s = s + cnflux[idx[k]];
+  for (int k = ptr[n], end = ptr[n + 1]; k < end; k += 4) {
+    int c[4];
+    double q[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) c[r] = idx[min(k + r, end - 1)];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) q[r] = cnflux[c[r]];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (k + r < end) s = s + q[r];
+  }
   ndflux[n] = s;
   int t = indtype[n];
   bool act = indstatus[n] > 0 && t != ibc && t != -3;
@@ -271,8 +284,7 @@ __global__ void k_ale_update(int nel, const int32_t* __restrict__ ielnd,
                              double* __restrict__ cs2, const int32_t* __restrict__ imat,
                              const int32_t* __restrict__ itype,
                              const double* __restrict__ param, double pcut, double ccut,
-                             DtResult* __restrict__ res, const DevTimestep* ts) {
-  ALE_GATE(ts);
+                             DtResult* __restrict__ res) {
   int e = xcd_index();
   if (e >= nel) return;
   int4 nd = reinterpret_cast<const int4*>(ielnd)[e];
@@ -313,28 +325,28 @@ int bl_ale_active(bl_handle_t* h, const bl_timestep_t* ts) {
 
 namespace bl {
 
-static int meshstatus(bl_handle_t* h, const DevTimestep* dts) {
+static int meshstatus(bl_handle_t* h) {
   if (h->cfg.zeul || h->relax_type != BL_RELAX_OFF) {
     int nnd = h->sz.nnd;
     BL_LAUNCH(h, "ale_meshstatus", k_meshstatus, nblocks(nnd), kBlock, nnd,
-              h->I(BL_ISCRATCH11), dts);
+              h->I(BL_ISCRATCH11));
   }
   return BL_SUCCESS;
 }
 
-static int fluxvolume(bl_handle_t* h, double dt, const DevTimestep* dts) {
+static int fluxvolume(bl_handle_t* h, double dt) {
   int nnd = h->sz.nnd, nel = h->sz.nel;
   // the relaxation's mesh velocity replaces the Lagrangian one in store4/5
   if (!h->cfg.zeul && h->relax_type != BL_RELAX_OFF &&
       mesh_motion(h, h->R(BL_NDX), h->R(BL_NDY), h->R(BL_RSCRATCH14), h->R(BL_RSCRATCH15), dt,
-                  dts))
+                  nullptr))
     return BL_FAILURE;
   BL_LAUNCH(h, "ale_fluxvol_nodes", k_fluxvol_nodes, nblocks(nnd), kBlock, nnd, h->cfg.zeul,
             dt, h->R(BL_RSCRATCH14), h->R(BL_RSCRATCH15), h->R(BL_RSCRATCH12),
-            h->R(BL_RSCRATCH13), h->R(BL_NDX), h->R(BL_NDY), dts);
+            h->R(BL_RSCRATCH13), h->R(BL_NDX), h->R(BL_NDY));
   BL_LAUNCH(h, "ale_fluxvol_faces", k_fluxvol_faces, nblocks(nel), kBlock, nel,
             h->cfg.zerocut, h->I(BL_IELND), h->R(BL_RSCRATCH12), h->R(BL_RSCRATCH13),
-            h->R(BL_NDX), h->R(BL_NDY), h->R(BL_RSCRATCH21), dts);
+            h->R(BL_NDX), h->R(BL_NDY), h->R(BL_RSCRATCH21));
   return BL_SUCCESS;
 }
 
@@ -345,13 +357,13 @@ extern "C" {
 int bl_ale_getmeshstatus(bl_handle_t* h) {
   bl_touch(h);
   if (!h) return BL_FAILURE;
-  return meshstatus(h, nullptr);
+  return meshstatus(h);
 }
 
 int bl_ale_getfluxvolume(bl_handle_t* h, const bl_timestep_t* ts) {
   bl_touch(h);
   if (!h || !ts) return BL_FAILURE;
-  return fluxvolume(h, ts->dt, nullptr);
+  return fluxvolume(h, ts->dt);
 }
 
 }  // extern "C"
@@ -369,72 +381,51 @@ double* tmp_buffer(Handle* h, int k) {
   return h->d_tmp[k];
 }
 
-static int advectel(bl_handle_t* h, int id1, int id2, const DevTimestep* dts) {
+static int advectel(bl_handle_t* h, int id1, int id2) {
   int nel = h->sz.nel;
   unsigned nb = nblocks(nel);
   // 0-based face passes
   int a = id1 - 1, b = id2 - 1;
   BL_LAUNCH(h, "ale_el1", k_el1, nb, kBlock, nel, a, b, h->I(BL_IELEL), h->I(BL_IELFC),
             h->R(BL_RSCRATCH21), h->R(BL_CNWT), h->R(BL_ELDENSITY), h->R(BL_RSCRATCH24),
-            h->R(BL_RSCRATCH22), dts);
+            h->R(BL_RSCRATCH22));
   BL_LAUNCH(h, "ale_el2", k_el2, nb, kBlock, nel, a, b, h->cfg.zerocut, h->cfg.dencut,
             h->I(BL_IELEL), h->I(BL_IELFC), h->R(BL_RSCRATCH22), h->R(BL_RSCRATCH24),
             h->R(BL_CNMASS), h->R(BL_ELENERGY), h->R(BL_RSCRATCH25), h->R(BL_RSCRATCH15),
             h->R(BL_RSCRATCH16), h->R(BL_RSCRATCH11), h->R(BL_RSCRATCH12), h->R(BL_RSCRATCH13),
-            h->R(BL_ELVOLUME), h->R(BL_ELMASS), h->R(BL_ELDENSITY), h->R(BL_RSCRATCH23), dts);
+            h->R(BL_ELVOLUME), h->R(BL_ELMASS), h->R(BL_ELDENSITY), h->R(BL_RSCRATCH23));
   BL_LAUNCH(h, "ale_el3", k_el3, nb, kBlock, nel, a, b, h->I(BL_IELEL), h->I(BL_IELFC),
             h->R(BL_RSCRATCH23), h->R(BL_RSCRATCH12), h->R(BL_ELMASS), h->R(BL_RSCRATCH16),
-            h->R(BL_RSCRATCH24), h->R(BL_ELENERGY), dts);
+            h->R(BL_RSCRATCH24), h->R(BL_ELENERGY));
   return BL_SUCCESS;
 }
 
-static int advectnd(bl_handle_t* h, int id1, int id2, const DevTimestep* dts) {
+static int advectnd(bl_handle_t* h, int id1, int id2) {
   int nel = h->sz.nel, nnd = h->sz.nnd;
   unsigned nbe = nblocks(nel), nbn = nblocks(nnd);
   int a = id1 - 1, b = id2 - 1;
   BL_LAUNCH(h, "ale_nd1", k_nd1, nbe, kBlock, nel, a, b, h->I(BL_IELND), h->I(BL_IELEL),
             h->I(BL_IELFC), h->R(BL_NDU), h->R(BL_NDV), h->R(BL_RSCRATCH21),
             h->R(BL_RSCRATCH22), h->R(BL_RSCRATCH27), h->R(BL_RSCRATCH28), h->R(BL_RSCRATCH26),
-            h->R(BL_RSCRATCH24), h->R(BL_RSCRATCH25), h->R(BL_RSCRATCH23), h->R(BL_CNMASS), dts);
+            h->R(BL_RSCRATCH24), h->R(BL_RSCRATCH25), h->R(BL_RSCRATCH23), h->R(BL_CNMASS));
   double* ndm1 = tmp_buffer(h, 0);
   if (!ndm1) return BL_FAILURE;
   BL_LAUNCH(h, "ale_nd2", k_nd2, nbn, kBlock, nnd, h->d_ale_ptr, h->d_ale_idx, h->cfg.zerocut,
             h->cfg.dencut, h->R(BL_RSCRATCH11), h->R(BL_ELVOLUME), h->R(BL_RSCRATCH26),
             h->R(BL_RSCRATCH23), h->R(BL_RSCRATCH13), h->R(BL_RSCRATCH14), h->R(BL_RSCRATCH12),
-            ndm1, h->R(BL_RSCRATCH15), h->R(BL_RSCRATCH16), dts);
+            ndm1, h->R(BL_RSCRATCH15), h->R(BL_RSCRATCH16));
   BL_LAUNCH(h, "ale_fluxndvl", k_fluxndvl, nbe, kBlock, nel, h->I(BL_IELEL), h->I(BL_IELFC),
-            h->R(BL_RSCRATCH26), h->R(BL_RSCRATCH25), h->R(BL_RSCRATCH27), h->R(BL_RSCRATCH23),
-            dts);
+            h->R(BL_RSCRATCH26), h->R(BL_RSCRATCH25), h->R(BL_RSCRATCH27), h->R(BL_RSCRATCH23));
   BL_LAUNCH(h, "ale_updatend", k_updatend, nbn, kBlock, nnd, h->d_el_ptr, h->d_el_idx, -1,
             h->I(BL_ISCRATCH11), h->I(BL_INDTYPE), h->Z(BL_ZSCRATCH11), 0, h->R(BL_RSCRATCH12),
             (const double*)ndm1, h->R(BL_RSCRATCH11), h->R(BL_RSCRATCH16), h->R(BL_RSCRATCH23),
-            h->R(BL_RSCRATCH22), h->R(BL_NDU), dts);
+            h->R(BL_RSCRATCH22), h->R(BL_NDU));
   BL_LAUNCH(h, "ale_fluxndvl", k_fluxndvl, nbe, kBlock, nel, h->I(BL_IELEL), h->I(BL_IELFC),
-            h->R(BL_RSCRATCH26), h->R(BL_RSCRATCH25), h->R(BL_RSCRATCH28), h->R(BL_RSCRATCH23),
-            dts);
+            h->R(BL_RSCRATCH26), h->R(BL_RSCRATCH25), h->R(BL_RSCRATCH28), h->R(BL_RSCRATCH23));
   BL_LAUNCH(h, "ale_updatend", k_updatend, nbn, kBlock, nnd, h->d_el_ptr, h->d_el_idx, -2,
             h->I(BL_ISCRATCH11), h->I(BL_INDTYPE), h->Z(BL_ZSCRATCH11), 1, h->R(BL_RSCRATCH12),
             (const double*)h->R(BL_RSCRATCH11), (double*)nullptr, h->R(BL_RSCRATCH16),
-            h->R(BL_RSCRATCH23), h->R(BL_RSCRATCH22), h->R(BL_NDV), dts);
-  return BL_SUCCESS;
-}
-
-// the ALE step inside a captured step: mesh status, flux volumes, unsplit
-// advection (adv_type=1) and the hydro update, gated by the device timestep
-int ale_step_device(Handle* hb, const DevTimestep* d_ts) {
-  bl_handle_t* h = static_cast<bl_handle_t*>(hb);
-  if (meshstatus(h, d_ts) || fluxvolume(h, 0.0, d_ts) || advectel(h, 1, 2, d_ts) ||
-      advectnd(h, 1, 2, d_ts))
-    return BL_FAILURE;
-  int nel = h->sz.nel;
-  BL_LAUNCH(h, "ale_update", k_ale_update, nblocks(nel), kBlock, nel, h->I(BL_IELND),
-            h->R(BL_NDX), h->R(BL_NDY), h->R(BL_CNX), h->R(BL_CNY), h->R(BL_A1), h->R(BL_A2),
-            h->R(BL_A3), h->R(BL_B1), h->R(BL_B2), h->R(BL_B3), h->R(BL_CNWT),
-            h->R(BL_ELVOLUME), h->R(BL_ELMASS), h->R(BL_ELDENSITY), h->R(BL_ELENERGY),
-            h->R(BL_ELPRESSURE), h->R(BL_ELCS2), h->I(BL_IELMAT), h->d_eos_itype,
-            h->d_eos_param, h->cfg.pcut, h->cfg.ccut, h->d_dtres, d_ts);
-  // mixed cells: component geometry, density and EOS of the hydro update
-  if (mix_geometry(h, d_ts) || mix_density(h, d_ts) || mix_eos(h, d_ts)) return BL_FAILURE;
+            h->R(BL_RSCRATCH23), h->R(BL_RSCRATCH22), h->R(BL_NDV));
   return BL_SUCCESS;
 }
 
@@ -448,13 +439,13 @@ int bl_ale_advect(bl_handle_t* h, const bl_timestep_t* ts, bl_error_t* err) {
   if (!h->maps_built) { set_error("bl_ale_advect: maps not built"); return BL_FAILURE; }
   switch (h->cfg.adv_type) {
     case 1:
-      if (advectel(h, 1, 2, nullptr) || advectnd(h, 1, 2, nullptr)) return BL_FAILURE;
+      if (advectel(h, 1, 2) || advectnd(h, 1, 2)) return BL_FAILURE;
       break;
     case 2: {
       int ii = (ts->nstep + 1) % 2;
       int i1 = 1 + ii, i2 = 2 - ii, i3 = i2 - i1;
       for (ii = i1; (i3 > 0) ? (ii <= i2) : (ii >= i2); ii += i3)
-        if (advectel(h, ii, ii, nullptr) || advectnd(h, ii, ii, nullptr)) return BL_FAILURE;
+        if (advectel(h, ii, ii) || advectnd(h, ii, ii)) return BL_FAILURE;
       break;
     }
     default:
@@ -474,9 +465,20 @@ int bl_ale_advect(bl_handle_t* h, const bl_timestep_t* ts, bl_error_t* err) {
 int bl_ale_hydroupdate(bl_handle_t* h, bl_error_t* err) {
   bl_touch(h);
   if (!h) return BL_FAILURE;
-  int rc = bl_geometry_getgeometry(h, err);
-  if (bl_density_getdensity(h) || bl_hydro_geteos(h)) return BL_FAILURE;
-  return rc;
+  if (!h->d_eos_itype) { set_error("bl_ale_hydroupdate: EOS not set"); return BL_FAILURE; }
+  // geometry, density and EOS in one pass (after a negative volume too, whose
+  // error is the call's result)
+  const int nel = h->sz.nel;
+  BL_HIP(hipMemsetAsync(&h->d_dtres->negvol, 0, sizeof(int32_t), h->stream));
+  BL_LAUNCH(h, "ale_update", k_ale_update, nblocks(nel), kBlock, nel, h->I(BL_IELND),
+            h->R(BL_NDX), h->R(BL_NDY), h->R(BL_CNX), h->R(BL_CNY), h->R(BL_A1), h->R(BL_A2),
+            h->R(BL_A3), h->R(BL_B1), h->R(BL_B2), h->R(BL_B3), h->R(BL_CNWT),
+            h->R(BL_ELVOLUME), h->R(BL_ELMASS), h->R(BL_ELDENSITY), h->R(BL_ELENERGY),
+            h->R(BL_ELPRESSURE), h->R(BL_ELCS2), h->I(BL_IELMAT), h->d_eos_itype,
+            h->d_eos_param, h->cfg.pcut, h->cfg.ccut, h->d_dtres);
+  if (mix_geometry(h, nullptr) || mix_density(h, nullptr) || mix_eos(h, nullptr))
+    return BL_FAILURE;
+  return volume_flag(h, err);
 }
 
 }  // extern "C"

@@ -178,6 +178,19 @@ __global__ void k_divide(int n, const double* __restrict__ num, const double* __
   if (i < n) out[i] = num[i] / den[i];
 }
 
+// density_dr_getdensity of pure cells behind the geometry of the same driver
+// call: the flag of a negative volume to the host (pinned, coherent memory),
+// and the densities when there is none (the driver stops in the geometry
+// otherwise), so that the host waits once, after both
+__global__ void k_density_checked(int nel, const double* __restrict__ m,
+                                  const double* __restrict__ vol, double* __restrict__ rho,
+                                  const int32_t* __restrict__ negvol,
+                                  int32_t* __restrict__ host) {
+  const int e = xcd_index(), neg = *negvol;
+  if (e == 0) *host = neg;
+  if (e < nel && !neg) rho[e] = m[e] / vol[e];
+}
+
 // eos_kn_geteos (eos_kn_geteos.f90:28-52)
 __global__ void k_geteos(int n, const int32_t* __restrict__ imat, const double* __restrict__ rho,
                          const double* __restrict__ en, double* __restrict__ pre,
@@ -220,10 +233,12 @@ __global__ void k_spmassinit(int nel, const double* __restrict__ rho,
 }
 
 // geometry_kn_getvertex (geometry_kn_position.f90:28-43)
+// (clear: the negative-volume flag of the geometry that follows)
 __global__ void k_getvertex(int nnd, double dt, double* __restrict__ ndx,
                             double* __restrict__ ndy, const double* __restrict__ ndu,
-                            const double* __restrict__ ndv) {
+                            const double* __restrict__ ndv, int32_t* __restrict__ clear) {
   int i = xcd_index();
+  if (i == 0) *clear = 0;
   if (i >= nnd) return;
   ndx[i] = ndx[i] + dt * ndu[i];
   ndy[i] = ndy[i] + dt * ndv[i];
@@ -298,21 +313,37 @@ __global__ void k_scatteracc(int nnd, const int32_t* __restrict__ ptr,
   int n = xcd_index();
   if (n >= nnd) return;
   double m = 0.0, a = 0.0, fu = 0.0, fv = 0.0;
-  int b = ptr[n], end = ptr[n + 1];
-  for (int k = b; k < end; ++k) {
-    int c = idx[k];
-    int e = c >> 2, j = c & 3;
-    double cm = cnmass[c];
-    if (cm > zerocut) {
-      m = m + cm;
-    } else {
-      double cp = cnmass[4 * e + ((j + 3) & 3)];
-      if (cp > zerocut) m = m + cp;
-      else m = m + rho[e] * cnwt[c];
+  const int b = ptr[n], end = ptr[n + 1];
+  // four incidences a pass: their corners, then every value, loaded before
+  // any is added (one at a time, each waits for its corner's load: 18.6 us
+  // against 10 at 263 000 nodes)
+  for (int k = b; k < end; k += 4) {
+    int c[4];
+    double cm[4], w[4], x[4], y[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) c[r] = idx[min(k + r, end - 1)];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      cm[r] = cnmass[c[r]];
+      w[r] = cnwt[c[r]];
+      x[r] = cnfx[c[r]];
+      y[r] = cnfy[c[r]];
     }
-    a = a + cnwt[c];
-    fu = fu + cnfx[c];
-    fv = fv + cnfy[c];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (k + r < end) {
+        const int e = c[r] >> 2, j = c[r] & 3;
+        if (cm[r] > zerocut) {
+          m = m + cm[r];
+        } else {
+          const double cp = cnmass[4 * e + ((j + 3) & 3)];
+          if (cp > zerocut) m = m + cp;
+          else m = m + rho[e] * w[r];
+        }
+        a = a + w[r];
+        fu = fu + x[r];
+        fv = fv + y[r];
+      }
   }
   ndmass[n] = m;
   ndarea[n] = a;
@@ -496,6 +527,123 @@ __global__ void k_getdt_b(int nel, double zerocut, double cvisc1, double cvisc2,
   ellength[e] = zdtnotreg[ireg] ? DBL_MIN : minlength(x, y, zcut, zmidlength[ireg] != 0);
 }
 
+// (a) and (b) in one pass on a mesh with the limiter's outer-node table
+// (build_outer): the neighbour edges' velocity differences from the nodes
+// (the table's far node, and the element's own node at the other end), their
+// position differences from the neighbours' corners, so that nothing waits
+// for (a)'s arrays.  An element whose four nodes share one velocity has zero
+// own-edge differences: its ratios, viscosity and elvisc are zero whatever
+// the neighbours hold (finite states), and it reads none of them.  At 512^2
+// (Sedov) 26 us where (a) and (b) took 43: bound by what it writes (the
+// drivers' fields, 320 B an element).
+__global__ void __launch_bounds__(kBlock)
+k_getdt_ab(int nel, double zerocut, double cvisc1, double cvisc2, double zcut,
+           const int32_t* __restrict__ indtype, const int32_t* __restrict__ ielel,
+           const int32_t* __restrict__ ielnd, const int32_t* __restrict__ ielfc,
+           const int32_t* __restrict__ ielreg, const int32_t* __restrict__ outer,
+           const int32_t* __restrict__ zdtnotreg, const int32_t* __restrict__ zmidlength,
+           const double* __restrict__ ndu, const double* __restrict__ ndv,
+           const double* __restrict__ rho, const double* __restrict__ cs2,
+           const double* __restrict__ cnx, const double* __restrict__ cny,
+           const double* __restrict__ a1, const double* __restrict__ a3,
+           const double* __restrict__ b1, const double* __restrict__ b3,
+           const double* __restrict__ vol, double* __restrict__ cnu, double* __restrict__ cnv,
+           double* __restrict__ du, double* __restrict__ dv, double* __restrict__ dx,
+           double* __restrict__ dy, double* __restrict__ rs27, double* __restrict__ cnviscx,
+           double* __restrict__ cnviscy, double* __restrict__ elvisc,
+           double* __restrict__ ellength, double* __restrict__ part,
+           int32_t* __restrict__ parti) {
+  const int e = xcd_index();
+  double dval = -1.0;  // below TINY: never selected
+  if (e < nel) {
+    const int4 nd4 = reinterpret_cast<const int4*>(ielnd)[e];
+    const int4 nb4 = reinterpret_cast<const int4*>(ielel)[e];
+    const int ireg = ielreg[e] - 1;
+    const int nd[4] = {nd4.x - 1, nd4.y - 1, nd4.z - 1, nd4.w - 1};
+    const int nb[4] = {nb4.x - 1, nb4.y - 1, nb4.z - 1, nb4.w - 1};
+    const double u[4] = {ndu[nd[0]], ndu[nd[1]], ndu[nd[2]], ndu[nd[3]]};
+    const double v[4] = {ndv[nd[0]], ndv[nd[1]], ndv[nd[2]], ndv[nd[3]]};
+    const double4 X = reinterpret_cast<const double4*>(cnx)[e];
+    const double4 Y = reinterpret_cast<const double4*>(cny)[e];
+    const double x[4] = {X.x, X.y, X.z, X.w}, y[4] = {Y.x, Y.y, Y.z, Y.w};
+    dval = divterm(u, v, a1[e], a3[e], b1[e], b3[e], vol[e]);
+    double ou[4], ov[4], ox[4], oy[4];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      const int g = (f + 1) & 3;
+      ou[f] = u[g] - u[f]; ov[f] = v[g] - v[f]; ox[f] = x[g] - x[f]; oy[f] = y[g] - y[f];
+    }
+    const bool moving = !(u[0] == u[1] && u[0] == u[2] && u[0] == u[3] && v[0] == v[1] &&
+                          v[0] == v[2] && v[0] == v[3]);
+    double ev = 0.0, sc[4] = {0.0, 0.0, 0.0, 0.0};
+    double qx[4] = {0.0, 0.0, 0.0, 0.0}, qy[4] = {0.0, 0.0, 0.0, 0.0}, ed[4];
+    double cs2e = 0.0, rhoe = 0.0;
+    if (moving) { cs2e = cs2[e]; rhoe = rho[e]; }
+#pragma unroll
+    for (int iside = 0; iside < 2; ++iside) {
+      const int is1 = (iside + 3) & 3, is2 = iside + 1;
+      const int in1 = nb[iside], in2 = nb[iside + 2];
+      double s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
+      if (moving) {
+        const int4 o = reinterpret_cast<const int4*>(outer)[2 * e + iside];
+        const int f1 = ielfc[4 * e + iside] - 1, f2 = ielfc[4 * e + iside + 2] - 1;
+        const int n0 = o.x - 1, n1 = o.y - 1, n2 = o.z - 1, n3 = o.w - 1;
+        const double u0 = ndu[n0], v0 = ndv[n0], u1 = ndu[n1], v1 = ndv[n1];
+        const double u2 = ndu[n2], v2 = ndv[n2], u3 = ndu[n3], v3 = ndv[n3];
+        double xa[4], ya[4], xb[4], yb[4];  // the neighbours' corners from the shared face on
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int ca = 4 * in1 + ((f1 + k) & 3), cb = 4 * in2 + ((f2 + k) & 3);
+          xa[k] = cnx[ca]; ya[k] = cny[ca];
+          xb[k] = cnx[cb]; yb[k] = cny[cb];
+        }
+        const int j3 = (iside + 3) & 3;
+        // in1 edge f1+1, in2 edge f2+3
+        limiter_ratios(ou[is1], ov[is1], ox[is1], oy[is1], u0 - u[iside], v0 - v[iside],
+                       xa[2] - xa[1], ya[2] - ya[1], u[j3] - u2, v[j3] - v2, xb[0] - xb[3],
+                       yb[0] - yb[3], zerocut, s1, s2);
+        // in1 edge f1+3, in2 edge f2+1
+        limiter_ratios(ou[is2], ov[is2], ox[is2], oy[is2], u[iside + 1] - u1, v[iside + 1] - v1,
+                       xa[0] - xa[3], ya[0] - ya[3], u3 - u[iside + 2], v3 - v[iside + 2],
+                       xb[2] - xb[1], yb[2] - yb[1], zerocut, s3, s4);
+      }
+      // boundary override (hydro_kn_edgeviscosity.f90:148-178)
+      if (in1 == e) {
+        const int ic1 = nd[iside], ic2 = nd[(iside + 1) & 3];
+        if (indtype[ic1] < 0 && indtype[ic2] < 0 && in2 != e) { s1 = 1.0; s3 = 1.0; }
+        else { s1 = 0.0; s3 = 0.0; }
+      }
+      if (in2 == e) {
+        const int ic1 = nd[iside + 2], ic2 = nd[(iside + 3) & 3];
+        if (indtype[ic1] < 0 && indtype[ic2] < 0 && in1 != e) { s2 = 1.0; s4 = 1.0; }
+        else { s2 = 0.0; s4 = 0.0; }
+      }
+      if (moving) {
+        int ins = nb[is1];
+        ed[is1] = limiter_edge(s1, s2, ou[is1], ov[is1], cs2e, cs2[ins], rhoe, rho[ins], cvisc1,
+                               cvisc2, zerocut, ev);
+        ins = nb[is2];
+        ed[is2] = limiter_edge(s3, s4, ou[is2], ov[is2], cs2e, cs2[ins], rhoe, rho[ins], cvisc1,
+                               cvisc2, zerocut, ev);
+      }
+      sc[0] = s1; sc[1] = s2; sc[2] = s3; sc[3] = s4;
+    }
+    if (moving) geteviscosity(x, y, u, v, ed, ed, zerocut, qx, qy);
+    reinterpret_cast<double4*>(cnu)[e] = make_double4(u[0], u[1], u[2], u[3]);
+    reinterpret_cast<double4*>(cnv)[e] = make_double4(v[0], v[1], v[2], v[3]);
+    reinterpret_cast<double4*>(du)[e] = make_double4(ou[0], ou[1], ou[2], ou[3]);
+    reinterpret_cast<double4*>(dv)[e] = make_double4(ov[0], ov[1], ov[2], ov[3]);
+    reinterpret_cast<double4*>(dx)[e] = make_double4(ox[0], ox[1], ox[2], ox[3]);
+    reinterpret_cast<double4*>(dy)[e] = make_double4(oy[0], oy[1], oy[2], oy[3]);
+    reinterpret_cast<double4*>(rs27)[e] = make_double4(sc[0], sc[1], sc[2], sc[3]);
+    reinterpret_cast<double4*>(cnviscx)[e] = make_double4(qx[0], qx[1], qx[2], qx[3]);
+    reinterpret_cast<double4*>(cnviscy)[e] = make_double4(qy[0], qy[1], qy[2], qy[3]);
+    elvisc[e] = ev;
+    ellength[e] = zdtnotreg[ireg] ? DBL_MIN : minlength(x, y, zcut, zmidlength[ireg] != 0);
+  }
+  block_argmax_first(dval, e + 1, part, parti);
+}
+
 // (c) hydro_dr_getcs2 (cs2 += elvisc) and the CFL ratio with its min reduction
 //     (hydro_kn_getdt.f90:50-73)
 __global__ void k_getdt_c(int nel, const int32_t* __restrict__ ielreg,
@@ -520,9 +668,17 @@ __global__ void k_getdt_c(int nel, const int32_t* __restrict__ ielreg,
 // (d) one workgroup combines the per-workgroup partials of (a) and (c); a
 //     separate launch instead of a "last workgroup" ticket, which would need
 //     a device-scope fence in every workgroup (an L2 write-back per XCD)
+//     (host: the result for the host too, in pinned coherent memory: no copy
+//     follows)
 __global__ void k_dt_final(int nblk_a, int nblk_c, const double* __restrict__ part,
-                           const int32_t* __restrict__ parti, DtResult* __restrict__ res) {
+                           const int32_t* __restrict__ parti, DtResult* res, DtResult* host) {
   final_dt_reduce(nblk_a, nblk_c, part, parti, res);
+  if (threadIdx.x == 0) {
+    host->cfl_min = res->cfl_min;
+    host->div_max = res->div_max;
+    host->cfl_idx = res->cfl_idx;
+    host->div_idx = res->div_idx;
+  }
 }
 
 // --- the allocation-free timestep (bl_hydro_getdt_noalloc) ------------------
@@ -621,7 +777,7 @@ int bl_create(const bl_sizes_t* sizes, bl_handle_t** out) {
       hipMalloc(&h->d_parti, sizeof(int32_t) * 4 * h->npart) != hipSuccess ||
       hipMalloc(&h->d_ticket, sizeof(uint32_t) * 16) != hipSuccess ||
       hipMalloc(&h->d_state, 3 * sizeof(StepState)) != hipSuccess ||
-      hipHostMalloc(&h->h_dtres, sizeof(DtResult)) != hipSuccess ||
+      hipHostMalloc(&h->h_dtres, sizeof(DtResult), hipHostMallocCoherent) != hipSuccess ||
       hipHostMalloc(&h->h_ts, sizeof(DevTimestep)) != hipSuccess ||
       hipHostMalloc(&h->h_pub_ts, sizeof(DevTimestep), hipHostMallocCoherent) != hipSuccess) {
     set_error("bl_create: out of device memory"); bl_destroy(h); return BL_FAILURE;
@@ -977,20 +1133,18 @@ int bl_init_mesh(bl_handle_t* h) {
 }
 
 // --------------------------------------------------------------- utilities
-int bl_geometry_getgeometry(bl_handle_t* h, bl_error_t* err) {
-  bl_touch(h);
-  if (!h) return BL_FAILURE;
-  int nel = h->sz.nel;
-  BL_HIP(hipMemsetAsync(&h->d_dtres->negvol, 0, sizeof(int32_t), h->stream));
+// the geometry kernel (and a mixed cell's component geometry)
+static int launch_geometry(bl_handle_t* h) {
+  const int nel = h->sz.nel;
   BL_LAUNCH(h, "getgeometry", k_getgeometry, nblocks(nel), kBlock, nel, h->I(BL_IELND),
             h->R(BL_NDX), h->R(BL_NDY), h->R(BL_CNX), h->R(BL_CNY), h->R(BL_A1), h->R(BL_A2),
             h->R(BL_A3), h->R(BL_B1), h->R(BL_B2), h->R(BL_B3), h->R(BL_CNWT),
             h->R(BL_ELVOLUME), h->d_dtres);
-  if (mix_geometry(h, nullptr)) return BL_FAILURE;
-  BL_HIP(hipMemcpyAsync(&h->h_dtres->negvol, &h->d_dtres->negvol, sizeof(int32_t),
-                        hipMemcpyDeviceToHost, h->stream));
-  BL_HIP(hipStreamSynchronize(h->stream));
-  int bad = h->h_dtres->negvol;
+  return mix_geometry(h, nullptr);
+}
+
+// geometry_kn_checkvolume's outcome on the host: err, and the return code
+static int check_volume(int bad, bl_error_t* err) {
   if (bad > 0) {
     if (err) {
       err->ierr = -bad;
@@ -1004,6 +1158,30 @@ int bl_geometry_getgeometry(bl_handle_t* h, bl_error_t* err) {
   }
   if (err) { err->ierr = BL_SUCCESS; err->iout = 0; std::memset(err->serr, ' ', BL_SLEN); }
   return BL_SUCCESS;
+}
+
+// wait for the flag of the geometry queued before
+static int read_volume_flag(Handle* h, bl_error_t* err) {
+  BL_HIP(hipMemcpyAsync(&h->h_dtres->negvol, &h->d_dtres->negvol, sizeof(int32_t),
+                        hipMemcpyDeviceToHost, h->stream));
+  BL_HIP(hipStreamSynchronize(h->stream));
+  return check_volume(h->h_dtres->negvol, err);
+}
+
+}  // extern "C"
+
+namespace bl {
+int volume_flag(Handle* h, bl_error_t* err) { return read_volume_flag(h, err); }
+}  // namespace bl
+
+extern "C" {
+
+int bl_geometry_getgeometry(bl_handle_t* h, bl_error_t* err) {
+  bl_touch(h);
+  if (!h) return BL_FAILURE;
+  BL_HIP(hipMemsetAsync(&h->d_dtres->negvol, 0, sizeof(int32_t), h->stream));
+  if (launch_geometry(h)) return BL_FAILURE;
+  return read_volume_flag(h, err);
 }
 
 int bl_density_getdensity(bl_handle_t* h) {
@@ -1058,23 +1236,34 @@ static int getdt_with(bl_handle_t* h, double* part, int32_t* parti, DtResult* dr
   int nel = h->sz.nel;
   unsigned nb = nblocks(nel);
   const bl_config_t& c = h->cfg;
-  BL_LAUNCH(h, "getdt_a", k_getdt_a, nb, kBlock, nel, h->I(BL_IELND), h->R(BL_NDU),
-            h->R(BL_NDV), h->R(BL_CNX), h->R(BL_CNY), h->R(BL_A1), h->R(BL_A3), h->R(BL_B1),
-            h->R(BL_B3), h->R(BL_ELVOLUME), h->R(BL_RSCRATCH21), h->R(BL_RSCRATCH22),
-            h->R(BL_RSCRATCH23), h->R(BL_RSCRATCH24), h->R(BL_RSCRATCH25), h->R(BL_RSCRATCH26),
-            part, parti);
-  BL_LAUNCH(h, "getdt_b", k_getdt_b, nb, kBlock, nel, c.zerocut, c.cvisc1, c.cvisc2, c.zcut,
-            h->I(BL_INDTYPE), h->I(BL_IELEL), h->I(BL_IELND), h->I(BL_IELFC), h->I(BL_IELREG),
-            h->d_zdtnotreg, h->d_zmidlength, h->R(BL_ELDENSITY), h->R(BL_ELCS2),
-            h->R(BL_RSCRATCH23), h->R(BL_RSCRATCH24), h->R(BL_RSCRATCH25), h->R(BL_RSCRATCH26),
-            h->R(BL_CNX), h->R(BL_CNY), h->R(BL_RSCRATCH21), h->R(BL_RSCRATCH22),
-            h->R(BL_RSCRATCH27), h->R(BL_CNVISCX), h->R(BL_CNVISCY), h->R(BL_ELVISC),
-            h->R(BL_RSCRATCH12));
+  if (h->d_outer && h->maps_built) {
+    BL_LAUNCH(h, "getdt_ab", k_getdt_ab, nb, kBlock, nel, c.zerocut, c.cvisc1, c.cvisc2, c.zcut,
+              h->I(BL_INDTYPE), h->I(BL_IELEL), h->I(BL_IELND), h->I(BL_IELFC), h->I(BL_IELREG),
+              h->d_outer, h->d_zdtnotreg, h->d_zmidlength, h->R(BL_NDU), h->R(BL_NDV),
+              h->R(BL_ELDENSITY), h->R(BL_ELCS2), h->R(BL_CNX), h->R(BL_CNY), h->R(BL_A1),
+              h->R(BL_A3), h->R(BL_B1), h->R(BL_B3), h->R(BL_ELVOLUME), h->R(BL_RSCRATCH21),
+              h->R(BL_RSCRATCH22), h->R(BL_RSCRATCH23), h->R(BL_RSCRATCH24), h->R(BL_RSCRATCH25),
+              h->R(BL_RSCRATCH26), h->R(BL_RSCRATCH27), h->R(BL_CNVISCX), h->R(BL_CNVISCY),
+              h->R(BL_ELVISC), h->R(BL_RSCRATCH12), part, parti);
+  } else {
+    BL_LAUNCH(h, "getdt_a", k_getdt_a, nb, kBlock, nel, h->I(BL_IELND), h->R(BL_NDU),
+              h->R(BL_NDV), h->R(BL_CNX), h->R(BL_CNY), h->R(BL_A1), h->R(BL_A3), h->R(BL_B1),
+              h->R(BL_B3), h->R(BL_ELVOLUME), h->R(BL_RSCRATCH21), h->R(BL_RSCRATCH22),
+              h->R(BL_RSCRATCH23), h->R(BL_RSCRATCH24), h->R(BL_RSCRATCH25), h->R(BL_RSCRATCH26),
+              part, parti);
+    BL_LAUNCH(h, "getdt_b", k_getdt_b, nb, kBlock, nel, c.zerocut, c.cvisc1, c.cvisc2, c.zcut,
+              h->I(BL_INDTYPE), h->I(BL_IELEL), h->I(BL_IELND), h->I(BL_IELFC), h->I(BL_IELREG),
+              h->d_zdtnotreg, h->d_zmidlength, h->R(BL_ELDENSITY), h->R(BL_ELCS2),
+              h->R(BL_RSCRATCH23), h->R(BL_RSCRATCH24), h->R(BL_RSCRATCH25), h->R(BL_RSCRATCH26),
+              h->R(BL_CNX), h->R(BL_CNY), h->R(BL_RSCRATCH21), h->R(BL_RSCRATCH22),
+              h->R(BL_RSCRATCH27), h->R(BL_CNVISCX), h->R(BL_CNVISCY), h->R(BL_ELVISC),
+              h->R(BL_RSCRATCH12));
+  }
   BL_LAUNCH(h, "getdt_c", k_getdt_c, nb, kBlock, nel, h->I(BL_IELREG), h->d_zdtnotreg,
             h->R(BL_ELVISC), h->R(BL_ELCS2), h->R(BL_RSCRATCH12), h->R(BL_RSCRATCH11),
             part, parti, (int)nb, (const int32_t*)h->I(BL_IELMAT), make_mix(h));
-  BL_LAUNCH(h, "dt_final", k_dt_final, 1, kFinalBlock, (int)nb, (int)nb, part, parti, dres);
-  BL_HIP(hipMemcpyAsync(h->h_dtres, dres, sizeof(DtResult), hipMemcpyDeviceToHost, h->stream));
+  BL_LAUNCH(h, "dt_final", k_dt_final, 1, kFinalBlock, (int)nb, (int)nb, part, parti, dres,
+            h->h_dtres);
   BL_HIP(hipStreamSynchronize(h->stream));
   const DtResult& r = *h->h_dtres;
   if (r.cfl_min < 0.0) {
@@ -1158,9 +1347,18 @@ int bl_hydro_getstate(bl_handle_t* h, const bl_timestep_t* ts, bl_error_t* err) 
   if (!h || !ts) return BL_FAILURE;
   int nnd = h->sz.nnd;
   BL_LAUNCH(h, "getvertex", k_getvertex, nblocks(nnd), kBlock, nnd, 0.5 * ts->dt, h->R(BL_NDX),
-            h->R(BL_NDY), h->R(BL_NDU), h->R(BL_NDV));
-  if (bl_geometry_getgeometry(h, err) != BL_SUCCESS) return BL_FAILURE;
-  return bl_density_getdensity(h);
+            h->R(BL_NDY), h->R(BL_NDU), h->R(BL_NDV), &h->d_dtres->negvol);
+  if (launch_geometry(h)) return BL_FAILURE;
+  if (h->sz.ncp > 0) {
+    if (read_volume_flag(h, err) != BL_SUCCESS) return BL_FAILURE;
+    return bl_density_getdensity(h);
+  }
+  const int nel = h->sz.nel;
+  BL_LAUNCH(h, "getdensity", k_density_checked, nblocks(nel), kBlock, nel,
+            (const double*)h->R(BL_ELMASS), (const double*)h->R(BL_ELVOLUME), h->R(BL_ELDENSITY),
+            (const int32_t*)&h->d_dtres->negvol, &h->h_dtres->negvol);
+  BL_HIP(hipStreamSynchronize(h->stream));
+  return check_volume(h->h_dtres->negvol, err);
 }
 
 int bl_hydro_getenergy(bl_handle_t* h, const bl_timestep_t* ts) {

@@ -284,9 +284,9 @@ int timing_begin(Handle* h, const char* cls);
 void timing_end(Handle* h, int slot);
 // lazily allocated nsz-sized temporaries (bl_ale.hip)
 double* tmp_buffer(Handle* h, int k);
-// ALE step launches; with d_ts the kernels read dt, the step gate and
-// ale_on from the device timestep (bl_ale.hip)
-int ale_step_device(Handle* h, const DevTimestep* d_ts);
+// geometry_kn_checkvolume's outcome of the geometry queued on the stream
+// (d_dtres->negvol): waits for it, fills err (bl_api.hip)
+int volume_flag(Handle* h, bl_error_t* err);
 // the relaxation's ALE mesh velocity (x_R - x)/dt into (wu, wv), gated by
 // ts when given; the stencil table rebuilt from the connectivity
 int relax_velocity(Handle* h, const double* x, const double* y, double* wu, double* wv,

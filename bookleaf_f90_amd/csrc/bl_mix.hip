@@ -33,20 +33,6 @@ __global__ void k_mx_geometry(MixArgs M, const double* __restrict__ a1,
   }
 }
 
-// the component part of ale_dr_hydroupdate (ale_dr_update.f90:33-51):
-// geometry_dr_volume.f90:66-79, density_dr_getdensity.f90:40-43 and
-// eos_dr_geteos.f90:50-55 per mixed cell
-__global__ void k_mx_hydroupdate(MixArgs M, const int32_t* __restrict__ ielnd,
-                                 const double* __restrict__ ndx, const double* __restrict__ ndy,
-                                 const int32_t* __restrict__ eos_itype,
-                                 const double* __restrict__ eos_param, double pcut, double ccut,
-                                 const DevTimestep* ts) {
-  MIX_GATE(ts);
-  const int imx = xcd_index();
-  if (imx >= M.nmx) return;
-  mix_hydroupdate_cell(M, imx, ielnd, ndx, ndy, eos_itype, eos_param, pcut, ccut);
-}
-
 // density_dr_getdensity.f90:40-43
 __global__ void k_mx_density(MixArgs M, const DevTimestep* ts) {
   MIX_GATE(ts);
@@ -216,14 +202,6 @@ int mix_eos(Handle* h, const DevTimestep* ts) {
   BL_LAUNCH(h, "mx_eos", k_mx_eos, nblocks(h->sz.ncp), kBlock, make_mix(h),
             (const int32_t*)h->d_eos_itype, (const double*)h->d_eos_param, h->cfg.pcut,
             h->cfg.ccut, ts);
-  return BL_SUCCESS;
-}
-
-int mix_hydroupdate(Handle* h, const double* x, const double* y, const DevTimestep* ts) {
-  if (h->sz.ncp <= 0) return BL_SUCCESS;
-  BL_LAUNCH(h, "mx_hydroupdate", k_mx_hydroupdate, nblocks(h->sz.nmx), kBlock, make_mix(h),
-            (const int32_t*)h->I(BL_IELND), x, y, (const int32_t*)h->d_eos_itype,
-            (const double*)h->d_eos_param, h->cfg.pcut, h->cfg.ccut, ts);
   return BL_SUCCESS;
 }
 
