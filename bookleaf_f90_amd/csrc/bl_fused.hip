@@ -2641,10 +2641,7 @@ int launch_ale_step(bl_handle_t* h, int p, int stop_at_time_end) {
   else
     BL_LAUNCH(h, "remap_tile", k_remap_tile<false>, (unsigned)h->ntile, kBlock, B, R, H, W,
               cm[1 - p]);
-  if (!h->diag_on) return BL_SUCCESS;
-  // per-step diagnostics need the step's end first
-  BL_LAUNCH(h, "batch_end", k_batch_end, 1, 64, A.ts, (const DtResult*)A.dtres);
-  return launch_diag(h, W.x, W.y, W.u, W.v, R.rho_o, R.en_o, R.pre_o, A.ts);
+  return launch_diag(h, W.x, W.y, W.u, W.v, R.rho_o, R.en_o, R.pre_o, A.ts, A.dtres);
 }
 
 // one step (parity p: node set p -> node set 1-p), launched on h->stream
@@ -2665,11 +2662,9 @@ int launch_step(bl_handle_t* h, int p, int stop_at_time_end) {
     BL_LAUNCH(h, "f1_limiter", k_f1_limiter<true>, (unsigned)A.nlim, (unsigned)h->tune_lim_block,
               A, N, A.nseg);
     if (launch_lag_tile<false, false>(h, A, N, O)) return BL_FAILURE;
-    if (!h->diag_on) return BL_SUCCESS;
-    // per-step diagnostics: the step's end, then the record of the node and
-    // element sets the step wrote
-    BL_LAUNCH(h, "batch_end", k_batch_end, 1, 64, A.ts, (const DtResult*)A.dtres);
-    return launch_diag(h, O.x, O.y, O.u, O.v, A.rho_o, A.en_o, A.pre_o, A.ts);
+    // per-step diagnostics: the record of the node and element sets the step
+    // wrote
+    return launch_diag(h, O.x, O.y, O.u, O.v, A.rho_o, A.en_o, A.pre_o, A.ts, A.dtres);
   }
   const unsigned nbl = std::min(nbe, (unsigned)h->tune_lim_grid);
   A.end_in_f1b = end_in_f1b(h) ? 1 : 0;

@@ -254,7 +254,7 @@ struct Handle {
   double diag_x0 = 0.0, diag_scale = 1.0;
   int32_t diag_max = 0;
   double* d_diag_hist = nullptr;     // diag_max records of 2 + 9*nreg + 2
-  int32_t* d_diag_count = nullptr;   // records written
+  int32_t* d_diag_count = nullptr;   // records written, and the place of the step's
   double* d_diag_part = nullptr;     // per-workgroup partials
   size_t diag_part_n = 0;
   int graph_stop_at_end = -1;
@@ -307,7 +307,8 @@ int relax_rebuild(Handle* h);
 // element state it wrote: the registry's unless given)
 int launch_diag(Handle* h, const double* ndx, const double* ndy, const double* ndu,
                 const double* ndv, const double* rho = nullptr, const double* en = nullptr,
-                const double* pre = nullptr, const DevTimestep* ts = nullptr);
+                const double* pre = nullptr, const DevTimestep* ts = nullptr,
+                const DtResult* res = nullptr);
 // ensembles: the limiter pass's workgroups per instance for a chunk of
 // elements each (bl_ensemble.hip)
 int ens_set_chunk(Handle* h, int chunk);
