@@ -11,10 +11,6 @@
 namespace bl {
 
 constexpr int kBlock = 256;  // 4 wave64 per workgroup
-// workgroups of a grid-stride launch that usually exits at once (a gated
-// fallback): one per CU
-constexpr unsigned kGatedBlocks = 256;
-
 void set_error(const std::string& msg);
 
 #define BL_HIP(call)                                                              \
@@ -208,6 +204,7 @@ struct Handle {
   int32_t* d_zlist = nullptr;     // nodes that are not relaxed, ascending
   int32_t nzero = 0;
   int32_t* d_lflag = nullptr;     // learned-motion flags and counters
+  int32_t fallback_blocks = 0;    // workgroups of k_learned_fallback, all resident at once
   int32_t* d_lmark = nullptr;     // nnd: node marked by the check for the guard
   int32_t* d_nbfc = nullptr;      // (4, nel) ielel/ielfc packed for the fused remap
   // launch shape of the limiter pass, set by bl_autotune: threads per
@@ -290,7 +287,7 @@ int volume_flag(Handle* h, bl_error_t* err);
 // the relaxation's ALE mesh velocity (x_R - x)/dt into (wu, wv), gated by
 // ts when given; the stencil table rebuilt from the connectivity
 int relax_velocity(Handle* h, const double* x, const double* y, double* wu, double* wv,
-                   double dt, const DevTimestep* ts, const int32_t* only_if = nullptr);
+                   double dt, const DevTimestep* ts);
 // the learned relaxation's mesh velocity (bl_relax_learned), with the plain
 // relaxation as the fallback; and the training pairs of the plain relaxation
 // from x (Lagrangian) and its mesh velocity (bl_relax_collect)

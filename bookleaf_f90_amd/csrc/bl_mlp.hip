@@ -46,8 +46,9 @@ constexpr int kOffW1 = 0, kOffB1 = kOffW1 + kHid * kIn, kOffW2 = kOffB1 + kHid,
               kOffB3 = kOffW3 + kOut * kHid, kNParam = kOffB3 + kOut;
 constexpr int kTrainBlock = 64;  // samples per training workgroup
 // learned-motion flags: [0] this step falls back, [1] steps, [2] fallbacks,
-// [3] reasons seen, [4] this step used the guard, [5] guarded steps
-constexpr int kLFlags = 8;
+// [3] reasons seen, [4] this step used the guard, [5] guarded steps,
+// [kLBarrier] the arrivals at k_learned_fallback's barriers
+constexpr int kLFlags = 8, kLBarrier = 6;
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -350,6 +351,7 @@ __global__ void __launch_bounds__(256) k_mlp_nodes(MlpPacked W, const float* __r
     if (flag[4]) flag[5] = flag[5] + 1;
     flag[0] = 0;
     flag[4] = 0;
+    flag[kLBarrier] = 0;
     flag[1] = flag[1] + 1;
   }
   __shared__ MlpShared S;
@@ -469,7 +471,7 @@ __device__ __forceinline__ void check_element(int e, const int32_t* __restrict__
 // x + (d1/dt) dt (what the guard would give it), and an element also fails
 // when the proposal shrinks it below half its one-sweep area (bit 2).  stage 0: a counted element
 // marks its four nodes for the guard and sets flag[4]; stage 1 (only when
-// flag[4] is set, with the guard's velocities: k_learned_recheck): a counted
+// flag[4] is set, with the guard's velocities: k_learned_fallback): a counted
 // element sets the step's fallback flag[0].  flag[3] keeps every reason seen
 // since the network was attached.
 __global__ void k_learned_check(int nel, const int32_t* __restrict__ ielnd,
@@ -485,31 +487,80 @@ __global__ void k_learned_check(int nel, const int32_t* __restrict__ ielnd,
     check_element(e, ielnd, x, y, wu, wv, d1, dt, amax2, relative, stage, mark, flag);
 }
 
-// Stage 1 with the guard folded in (only when stage 0 marked nodes,
-// flag[4]): a relaxed node marked by stage 0 moves by one plain sweep
-// instead of the network's proposal (written here), and every element is
-// checked again with the guarded velocities, which it forms itself from the
-// marks, so that the check needs no pass of its own after the guard's
-__global__ void k_learned_recheck(int nel, const int32_t* __restrict__ ielnd,
-                                  const double* __restrict__ x, const double* __restrict__ y,
-                                  double* __restrict__ wu, double* __restrict__ wv,
-                                  const float2* __restrict__ d1, double dt, double amax2,
-                                  int relative, const int32_t* __restrict__ rlist, int nr,
-                                  int32_t* __restrict__ mark, int32_t* __restrict__ flag,
-                                  const DevTimestep* ts) {
+// A barrier of the whole grid, whose workgroups are all resident (the launch
+// is sized for it): count starts the launch at 0, target is the arrivals so
+// far and this barrier's.  Orders what the workgroups exchange at agent scope
+// (relaxed stores, loads and atomics): each thread waits for its own to
+// complete before its workgroup arrives.
+__device__ __forceinline__ void grid_barrier(int32_t* count, int32_t target) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    while (__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target)
+      __builtin_amdgcn_s_sleep(1);
+  }
+  __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// Stage 1 with the guard folded in, and the fallback, in one launch that
+// usually ends at once (stage 0 marked nothing: flag[4] is 0).  Every element
+// is checked again with the guarded velocities, which it forms itself from
+// the marks; after a barrier, when none failed, a relaxed node marked by
+// stage 0 takes one plain sweep's motion instead of the network's proposal.
+// When one failed (flag[0]) the plain relaxation's nsweep sweeps run with a
+// barrier between them; the workgroups exchange positions at agent scope, as
+// each XCD has its own L2.  As launches of their own, gated on the flag, the
+// recheck and eight sweeps cost 38 us a step of doing nothing on the
+// 512x256 problem.
+__global__ void __launch_bounds__(kBlock)
+k_learned_fallback(int nel, const int32_t* __restrict__ ielnd, const double* x, const double* y,
+                   double* wu, double* wv, const float2* __restrict__ d1, double dt, double amax2,
+                   int relative, const int32_t* __restrict__ rlist, int nr, int32_t* mark,
+                   int32_t* flag, RelaxArgs R, int nsweep, double* t0x, double* t0y, double* t1x,
+                   double* t1y, const DevTimestep* ts) {
   if (ts && (ts->skip || step_bad(ts) || !ts->ale_on)) return;
   if (flag[4] == 0) return;
   if (ts) dt = ts->dt;
   const int stride = gridDim.x * blockDim.x;
-  for (int i = xcd_index(); i < nr; i += stride) {
-    const int n = rlist[i];
-    if (!mark[n]) continue;
-    const float2 d = d1[n];
-    wu[n] = (double)d.x / dt;
-    wv[n] = (double)d.y / dt;
-  }
+  int32_t* count = flag + kLBarrier;
+  int32_t target = (int32_t)gridDim.x;
   for (int e = xcd_index(); e < nel; e += stride)
     check_element(e, ielnd, x, y, wu, wv, d1, dt, amax2, relative, 1, mark, flag, true);
+  grid_barrier(count, target);
+  if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
+    for (int i = xcd_index(); i < nr; i += stride) {
+      const int n = rlist[i];
+      if (!mark[n]) continue;
+      const float2 d = d1[n];
+      wu[n] = (double)d.x / dt;
+      wv[n] = (double)d.y / dt;
+    }
+    return;
+  }
+  for (int k = 0; k < nsweep; ++k) {
+    const bool last = k + 1 == nsweep;
+    const double* xi = k == 0 ? x : (k & 1) ? t0x : t1x;
+    const double* yi = k == 0 ? y : (k & 1) ? t0y : t1y;
+    double* xo = (k & 1) ? t1x : t0x;
+    double* yo = (k & 1) ? t1y : t0y;
+    for (int n = xcd_index(); n < R.nnd; n += stride) {
+      double a, b;
+      if (k == 0) relax_node(R, n, xi, yi, a, b);
+      else relax_node(R, n, xi, yi, a, b, AgentLoad());
+      if (last) {
+        wu[n] = (a - x[n]) / dt;
+        wv[n] = (b - y[n]) / dt;
+      } else {
+        __hip_atomic_store(xo + n, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(yo + n, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    target += (int32_t)gridDim.x;
+    if (!last) grid_barrier(count, target);
+  }
 }
 
 // per-column mean and standard deviation of the stored pairs (FP64 sums in
@@ -1003,7 +1054,7 @@ int learned_velocity(Handle* hh, const double* x, const double* y, double* wu, d
   const bl_mlp* m = h->mlp_infer;
   const int nel = h->sz.nel, nr = h->nrelaxed, nz = h->nzero;
   if (!m || !h->d_ring || !h->d_rlist || !h->d_zlist || !h->d_lflag || !h->d_lmark ||
-      !h->d_ld1) {
+      !h->d_ld1 || !h->relax_tmp[0] || h->fallback_blocks < 1) {
     set_error("learned relaxation: not set up (bl_relax_learned)");
     return BL_FAILURE;
   }
@@ -1022,12 +1073,13 @@ int learned_velocity(Handle* hh, const double* x, const double* y, double* wu, d
             (const int32_t*)h->I(BL_IELND), x, y, (const double*)wu, (const double*)wv,
             (const float2*)h->d_ld1, dt, amax2, h->learned_relative, 0, h->d_lmark,
             h->d_lflag, ts);
-  BL_LAUNCH(h, "learned_recheck", k_learned_recheck,
-            std::min(nblocks(std::max(nel, nr)), kGatedBlocks), kBlock, nel,
+  // the guard, and the plain relaxation when the check failed
+  double* const* t = h->relax_tmp;
+  BL_LAUNCH(h, "learned_fallback", k_learned_fallback, (unsigned)h->fallback_blocks, kBlock, nel,
             (const int32_t*)h->I(BL_IELND), x, y, wu, wv, (const float2*)h->d_ld1, dt, amax2,
-            h->learned_relative, (const int32_t*)h->d_rlist, nr, h->d_lmark, h->d_lflag, ts);
-  // the plain relaxation, whose kernels run only when the check failed
-  return relax_velocity(h, x, y, wu, wv, dt, ts, h->d_lflag);
+            h->learned_relative, (const int32_t*)h->d_rlist, nr, h->d_lmark, h->d_lflag,
+            relax_args(h), h->relax_nsweep, t[0], t[1], t[2], t[3], ts);
+  return BL_SUCCESS;
 }
 
 int collect_pairs(Handle* hh, const double* x, const double* y, const double* wu,
@@ -1286,6 +1338,18 @@ int bl_relax_learned(bl_handle_t* h, bl_mlp_t* m) {
   if (m && !h->d_lmark)
     BL_HIP(hipMalloc(&h->d_lmark, sizeof(int32_t) * std::max(h->sz.nnd, 1)));
   if (m && !h->d_ld1) BL_HIP(hipMalloc(&h->d_ld1, sizeof(float) * 2 * std::max(h->sz.nnd, 1)));
+  if (m && h->fallback_blocks < 1) {
+    // as many workgroups as the device holds at once, at most one per CU of
+    // an MI355X (a thread takes a few nodes when it runs at all)
+    int per_cu = 0, cus = 0;
+    BL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_learned_fallback, kBlock, 0));
+    BL_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device));
+    h->fallback_blocks = std::min(256, per_cu * cus);
+    if (h->fallback_blocks < 1) {
+      set_error("bl_relax_learned: the fallback kernel does not fit the device");
+      return BL_FAILURE;
+    }
+  }
   // the counters start again with every network attached
   if (m) BL_HIP(hipMemset(h->d_lflag, 0, sizeof(int32_t) * kLFlags));
   return BL_SUCCESS;

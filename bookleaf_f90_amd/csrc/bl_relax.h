@@ -12,15 +12,26 @@ struct RelaxArgs {
   int nnd, type;
   double om, tol, zerocut;
   const int32_t* ring;
-  const int32_t* only_if;  // non-null: the sweeps run only when *only_if != 0
+};
+
+// a position from memory, and one that another workgroup of the same launch
+// may have stored (agent scope: not from this XCD's L2)
+struct PlainLoad {
+  __device__ __forceinline__ double operator()(const double* p) const { return *p; }
+};
+struct AgentLoad {
+  __device__ __forceinline__ double operator()(const double* p) const {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 };
 
 // one node of one sweep (setup_mesh.F90:797-863); (xo, yo) the position
 // after it.  rr of the generator is y, ss is x.
-__device__ __forceinline__ void relax_node(const RelaxArgs& R, int n, const double* __restrict__ xi,
-                                           const double* __restrict__ yi, double& xo,
-                                           double& yo) {
-  const double xn = xi[n], yn = yi[n];
+template <typename LOAD = PlainLoad>
+__device__ __forceinline__ void relax_node(const RelaxArgs& R, int n, const double* xi,
+                                           const double* yi, double& xo, double& yo,
+                                           LOAD ld = LOAD()) {
+  const double xn = ld(xi + n), yn = ld(yi + n);
   xo = xn;
   yo = yn;
   const int4 qa = reinterpret_cast<const int4*>(R.ring)[2 * n];
@@ -30,8 +41,8 @@ __device__ __forceinline__ void relax_node(const RelaxArgs& R, int n, const doub
   double x[8], y[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    x[i] = xi[nb[i]];
-    y[i] = yi[nb[i]];
+    x[i] = ld(xi + nb[i]);
+    y[i] = ld(yi + nb[i]);
   }
   double r1, r2, r3, r4, r5, r6, r7, r8;
   if (R.type == BL_RELAX_EQUI) {

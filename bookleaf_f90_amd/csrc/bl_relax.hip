@@ -23,19 +23,18 @@
 namespace bl {
 
 #define RELAX_GATE(ts) \
-  if (((ts) && ((ts)->skip || step_bad(ts) || !(ts)->ale_on)) || (R.only_if && *R.only_if == 0)) return
+  if ((ts) && ((ts)->skip || step_bad(ts) || !(ts)->ale_on)) return
 
 __global__ void k_relax_sweep(RelaxArgs R, const double* __restrict__ xi,
                               const double* __restrict__ yi, double* __restrict__ xo,
                               double* __restrict__ yo, const DevTimestep* ts) {
   RELAX_GATE(ts);
-  const int stride = gridDim.x * blockDim.x;
-  for (int n = xcd_index(); n < R.nnd; n += stride) {
-    double a, b;
-    relax_node(R, n, xi, yi, a, b);
-    xo[n] = a;
-    yo[n] = b;
-  }
+  const int n = xcd_index();
+  if (n >= R.nnd) return;
+  double a, b;
+  relax_node(R, n, xi, yi, a, b);
+  xo[n] = a;
+  yo[n] = b;
 }
 
 // the last sweep of the ALE mesh motion: w = (x_R - x)/dt, x the Lagrangian
@@ -46,13 +45,12 @@ __global__ void k_relax_velocity(RelaxArgs R, const double* __restrict__ xl,
                                  double* __restrict__ wv, double dt, const DevTimestep* ts) {
   RELAX_GATE(ts);
   if (ts) dt = ts->dt;
-  const int stride = gridDim.x * blockDim.x;
-  for (int n = xcd_index(); n < R.nnd; n += stride) {
-    double a, b;
-    relax_node(R, n, xi, yi, a, b);
-    wu[n] = (a - xl[n]) / dt;
-    wv[n] = (b - yl[n]) / dt;
-  }
+  const int n = xcd_index();
+  if (n >= R.nnd) return;
+  double a, b;
+  relax_node(R, n, xi, yi, a, b);
+  wu[n] = (a - xl[n]) / dt;
+  wv[n] = (b - yl[n]) / dt;
 }
 
 }  // namespace bl
@@ -157,7 +155,6 @@ RelaxArgs make_relax(bl_handle_t* h, int type, double om, double tol) {
   R.tol = tol;
   R.zerocut = h->cfg.zerocut;
   R.ring = h->d_ring;
-  R.only_if = nullptr;
   return R;
 }
 
@@ -178,7 +175,7 @@ int relax_rebuild(Handle* h) {
 // (x, y); with ts the kernels are gated like the other ALE kernels and dt
 // is the device timestep's
 int relax_velocity(Handle* hh, const double* x, const double* y, double* wu, double* wv,
-                   double dt, const DevTimestep* ts, const int32_t* only_if) {
+                   double dt, const DevTimestep* ts) {
   bl_handle_t* h = static_cast<bl_handle_t*>(hh);
   const int nnd = h->sz.nnd;
   if (!h->d_ring || !h->relax_tmp[0]) {
@@ -186,10 +183,7 @@ int relax_velocity(Handle* hh, const double* x, const double* y, double* wu, dou
     return BL_FAILURE;
   }
   RelaxArgs R = make_relax(h, h->relax_type, h->relax_om, h->relax_tol);
-  R.only_if = only_if;
-  // a gated fallback mostly does nothing: a small grid (each thread a few
-  // nodes when it runs) keeps the empty launches cheap
-  const unsigned grid = only_if ? std::min(nblocks(nnd), kGatedBlocks) : nblocks(nnd);
+  const unsigned grid = nblocks(nnd);
   const double* xi = x;
   const double* yi = y;
   for (int k = 0; k + 1 < h->relax_nsweep; ++k) {
