@@ -22,12 +22,14 @@ __device__ __forceinline__ NbFc load_nbfc(int e, const int32_t* ielel, const int
 
 // the same from the packed table of the device-resident step: per face
 // (neighbour - 1) << 2 | (its face - 1), one int32 instead of two
-__device__ __forceinline__ NbFc load_nbfc_packed(int e, const int32_t* nbfc) {
-  const int4 a = reinterpret_cast<const int4*>(nbfc)[e];
+__device__ __forceinline__ NbFc unpack_nbfc(const int4 a) {
   NbFc r;
   r.nb[0] = a.x >> 2; r.nb[1] = a.y >> 2; r.nb[2] = a.z >> 2; r.nb[3] = a.w >> 2;
   r.fc[0] = a.x & 3; r.fc[1] = a.y & 3; r.fc[2] = a.z & 3; r.fc[3] = a.w & 3;
   return r;
+}
+__device__ __forceinline__ NbFc load_nbfc_packed(int e, const int32_t* nbfc) {
+  return unpack_nbfc(reinterpret_cast<const int4*>(nbfc)[e]);
 }
 
 // ale_kn_sumflux for one element (ale_kn_advectors.f90:216-244)
@@ -205,6 +207,24 @@ __device__ __forceinline__ double fluxnd_right(double cd, double rd, double w5, 
   const double w8 = (w1 * w6 * w6 + w2 * w5 * w5) / (w5 * w6 * (w5 + w6));
   double grad = -(w7 * dmin(dmin(fabs(w8), w3 / w5), w4 / w6));
   if (w1 * w2 <= 0.0) grad = 0.0;
+  return cd * (rv + grad * rd);
+}
+
+// fluxnd_left (left) or fluxnd_right in one form, so that the lanes of a wave
+// whose fluxes differ in sign share it: rv the upwind corner's value, vnb the
+// neighbour's corner beyond the face, vown the element's other corner.  Each
+// side's own difference pairs with w6^2 and w5, the neighbour's with w5^2 and
+// w6; the operations and their order are that side's.
+__device__ __forceinline__ double fluxnd_upwind(bool left, double cd, double rd, double w5,
+                                                double w6, double rv, double vnb, double vown) {
+  const double own = left ? vown - rv : rv - vown;
+  const double far = left ? rv - vnb : vnb - rv;
+  const double w8 = (own * w6 * w6 + far * w5 * w5) / (w5 * w6 * (w5 + w6));
+  const double q5 = fabs(own) / w5, q6 = fabs(far) / w6;
+  const double w7 = dsign(1.0, left ? own : far);
+  double grad = w7 * dmin(dmin(fabs(w8), left ? q6 : q5), left ? q5 : q6);
+  grad = left ? grad : -grad;
+  if (own * far <= 0.0) grad = 0.0;
   return cd * (rv + grad * rd);
 }
 

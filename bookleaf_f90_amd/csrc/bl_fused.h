@@ -153,7 +153,9 @@ struct FusedArgs {
   // corner in them (one byte each), and in y the corners in the order of the
   // ALE sums (2 bits each), in element order (2 bits each from bit 8), and
   // their count (from bit 16)
+  // tile_nbfc: the entry's packed neighbours and faces (load_nbfc_packed)
   const int32_t* tile_nbr;
+  const int4* tile_nbfc;
   const int2* tile_ninc;
   const uint8_t* rest8;
   const uint8_t* rest8_prev;

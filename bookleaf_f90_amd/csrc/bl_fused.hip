@@ -2033,15 +2033,30 @@ __global__ void __launch_bounds__(kBlock) k_r5(AleArgs B, DevTimestep* tsw) {
 // at most 168 VGPRs) of dependent gathers and divisions.  A tiling is used
 // wherever the mesh has one; the eleven kernels remain for meshes without.
 
-#define REMAP_TILE_GATE(T) \
-  if ((T)->skip || step_bad(T)) return
-
 // R1's face mass fluxes (and a negative volume of the moved mesh, which R3
-// finds in the five-kernel form)
-__global__ void __launch_bounds__(kBlock) k_remap_faces(AleArgs B) {
-  REMAP_TILE_GATE(B.ts);
-  if (!B.ts->ale_on) return;
-  const int e = xcd_index();
+// finds in the five-kernel form).  MIX: the first nbm8 workgroups (whole XCD
+// rounds) are F4m, one thread per mixed cell, on the node set H the tile step
+// wrote; a negative volume of the corrector leaves the components after the
+// predictor (of the predictor: before it).
+template <bool MIX>
+__global__ void __launch_bounds__(kBlock)
+k_remap_faces(AleArgs B, FusedArgs A, FusedNodes H, int nbm8) {
+  if (B.ts->skip) return;
+  if (MIX && (int)blockIdx.x < nbm8) {
+    const int imx = (int)blockIdx.x * kBlock + threadIdx.x;
+    if (imx >= A.mx.nmx || B.dtres->negvol) return;
+    if (!B.dtres->negvol2) {
+      f4_mix_cell(A, H, B.ts, imx, A.mx.cpe);
+      return;
+    }
+    for (int k = 0, icp = A.mx.imxfcp[imx] - 1; k < A.mx.imxncp[imx]; ++k, ++icp)
+      A.mx.cpenergy[icp] = A.mx.cpe[icp];
+    return;
+  }
+  if (step_bad(B.ts) || !B.ts->ale_on) return;
+  const int e = MIX ? xcd_block_of((int)blockIdx.x - nbm8, (int)gridDim.x - nbm8) * kBlock +
+                          (int)threadIdx.x
+                    : xcd_index();
   if (e >= B.nel) return;
   int nd[4];
   load_nd(B.ielnd, e, nd);
@@ -2089,21 +2104,19 @@ __device__ __forceinline__ void fluxndvl_outer(const FusedArgs& A, const FusedNo
       const double un[2] = {H.u[n0], H.u[n1]}, vn[2] = {H.v[n0], H.v[n1]};
       const double b0 = cb[4 * nb + f], b1 = cb[4 * nb + ((f + 1) & 3)],
                    b2 = cb[4 * nb + ((f + 2) & 3)], b3 = cb[4 * nb + ((f + 3) & 3)];
+      const double half = 0.5 * fabs(cd[l]);
 #pragma unroll
       for (int k = 0; k < 2; ++k) {  // icn = k + 1
         const int jl = l + k, jr = (lr + 1 - k) & 3;  // the two corners along the direction
+        // the upwind corner and the other one; the neighbour's two corners
+        // beyond the face
         const double w5 = cm[jl] + cm[jr];
-        if (left) {
-          const double rd = cm[jl] - 0.5 * cd[l];
-          const double w6 = k == 0 ? b2 + b1 : b3 + b0;
-          du[k] = fluxnd_left(cd[l], rd, w5, w6, u[jl], un[k], u[jr]);
-          dv[k] = fluxnd_left(cd[l], rd, w5, w6, v[jl], vn[k], v[jr]);
-        } else {
-          const double rd = cm[jr] + 0.5 * cd[l];
-          const double w6 = k == 0 ? b0 + b3 : b1 + b2;
-          du[k] = fluxnd_right(cd[l], rd, w5, w6, u[jr], u[jl], un[k]);
-          dv[k] = fluxnd_right(cd[l], rd, w5, w6, v[jr], v[jl], vn[k]);
-        }
+        const double w6 = left ? (k == 0 ? b2 + b1 : b3 + b0) : (k == 0 ? b0 + b3 : b1 + b2);
+        const double rd = (left ? cm[jl] : cm[jr]) - half;
+        du[k] = fluxnd_upwind(left, cd[l], rd, w5, w6, left ? u[jl] : u[jr], un[k],
+                              left ? u[jr] : u[jl]);
+        dv[k] = fluxnd_upwind(left, cd[l], rd, w5, w6, left ? v[jl] : v[jr], vn[k],
+                              left ? v[jr] : v[jl]);
       }
     }
 #pragma unroll
@@ -2124,15 +2137,17 @@ __device__ __forceinline__ void fluxndvl_outer(const FusedArgs& A, const FusedNo
 // (A.tile_ninc), the remapped velocity and position, to LDS and, by the one
 // tile that writes the node, to the home node set W.  Phase C, one thread per
 // own element: mass, energy, corner masses, then the hydro update on the
-// moved mesh, the components of a mixed cell and F1's terms.  H: the node set
+// moved mesh (of a mixed cell's components too) and F1's terms.  H: the node set
 // the tile step wrote.  A step outside the ALE time window copies the tile
 // step's state to the home sets and does F1's terms.
 template <bool MIX>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
 k_remap_tile(AleArgs B, FusedArgs A, FusedNodes H, FusedNodesOut W, double* cm_out) {
   __shared__ double s_cm[4][kTileEls], s_fu[4][kTileEls], s_fv[4][kTileEls], s_ef[4][kTileEls];
   __shared__ double s_v0[kTileEls], s_fl[kTileEls];
-  __shared__ double nout[4][kTileNodes + 1];  // x, y, u, v after the remap
+  // x, y, u, v after the remap, in the place of the u fluxes
+  static_assert(kTileNodes + 1 <= kTileEls, "a node's slot in an element array");
+  double (*nout)[kTileEls] = s_fu;
   const int t = xcd_block();
   const int tid = threadIdx.x;
   const int4 tb = A.tile_bounds[t];
@@ -2144,40 +2159,40 @@ k_remap_tile(AleArgs B, FusedArgs A, FusedNodes H, FusedNodesOut W, double* cm_o
   const int2 ent = A.tile_el[eb + min(tid, ne - 1)];
   const int4 q = A.tile_nd[eb + min(tid, ne - 1)];
   const uint32_t nbr = (uint32_t)A.tile_nbr[eb + min(tid, ne - 1)];
+  const int4 qn = A.tile_nbfc[eb + min(tid, ne - 1)];
   const DevTimestep* ts = A.ts;
   if (ts->skip) return;
   const int e = ent.x & 0x3fffffff;
   const bool own = active && (((uint32_t)ent.x >> 30) & kTileOwn);
   const uint32_t slots = (uint32_t)ent.y;
-  if (step_bad(ts)) {
-    // a negative volume of the corrector leaves the components after the
-    // predictor (of the predictor: before it)
-    if (MIX && own && !A.dtres->negvol && A.ielmat[e] < 0) {
-      const int imx = -A.ielmat[e] - 1;
-      for (int k = 0, icp = A.mx.imxfcp[imx] - 1; k < A.mx.imxncp[imx]; ++k, ++icp)
-        A.mx.cpenergy[icp] = A.mx.cpe[icp];
-    }
-    return;
-  }
+  if (step_bad(ts)) return;
   const bool on = ts->ale_on != 0;
   const double dt = ts->dt;
   const int nd[4] = {q.x, q.y, q.z, q.w};
-  const NbFc c = load_nbfc_packed(e, B.nbfc);
+  const NbFc c = unpack_nbfc(qn);
   // (every thread's entry names an element of the tile)
-  double cm[4], ef[4];
-  ld4(B.cnmass, e, cm);
-  const double en0 = B.en[e], v0 = B.vol[e];
-  double totm = 0.0, fl = 0.0;
+  const double en0 = B.en[e];
+  double totm = 0.0;
   if (on) {
-    double fm[4], wn[4];
+    double cm[4], fm[4], wn[4], cd[2];
+    ld4(B.cnmass, e, cm);
     ld4(B.fcdm, e, fm);
 #pragma unroll
     for (int i = 0; i < 4; ++i) wn[i] = B.fcdm[4 * c.nb[i] + c.fc[i]];
-    fluxelvl_own(c.nb, c.fc, cm, B.cnmass, fm, en0, B.en, ef);
+    s_v0[tid] = B.vol[e];
+    {
+      double ef[4];
+      fluxelvl_own(c.nb, c.fc, cm, B.cnmass, fm, en0, B.en, ef);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        s_cm[j][tid] = cm[j];
+        s_ef[j][tid] = ef[j];
+      }
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       if (c.nb[i] == e) wn[i] = 0.0;
-    double cd[2];
+    double fl = 0.0;
 #pragma unroll
     for (int i1 = 0; i1 < 2; ++i1) {
       const int i2 = i1 + 2;
@@ -2187,20 +2202,23 @@ k_remap_tile(AleArgs B, FusedArgs A, FusedNodes H, FusedNodesOut W, double* cm_o
       cd[i1] = 0.25 * (w1 - w2);
       fl = fl + 0.25 * (w1 + w2);
     }
+    s_fl[tid] = fl;
     double ou[4], ov[4];
     fluxndvl_outer(A, H, e, nd, c, B.cnmass, cm, cd, ou, ov);
-    if (active) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        s_cm[j][tid] = cm[j];
-        s_fu[j][tid] = ou[j];
-        s_fv[j][tid] = ov[j];
-        s_ef[j][tid] = ef[j];
-      }
-      s_v0[tid] = v0;
-      s_fl[tid] = fl;
+    for (int j = 0; j < 4; ++j) {
+      s_fu[j][tid] = ou[j];
+      s_fv[j][tid] = ov[j];
     }
   }
+  // what phase C needs of the faces in one word: per face its neighbour's face
+  // (2 bits) and whether it is a boundary (the bit above); its corner masses
+  // and fluxes come back from LDS (fewer registers over the barriers: four
+  // workgroups a CU)
+  uint32_t faces = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    faces |= ((uint32_t)c.fc[i] | (c.nb[i] == e ? 4u : 0u)) << (4 * i);
   // the node's values, and phase C's element inputs, before the barrier
   const int n = (int)(nv & 0x7fffffffu);
   const double x0 = H.x[n], y0 = H.y[n], u0 = H.u[n], v0n = H.v[n];
@@ -2208,9 +2226,16 @@ k_remap_tile(AleArgs B, FusedArgs A, FusedNodes H, FusedNodesOut W, double* cm_o
   const int ntype = A.indtype[n];
   const double m0 = B.mass[e];
   const int mat = A.ielmat[e];
+  const int ereg = (A.reg_tables ? A.ielreg : A.ielmat)[e];  // (used with reg_tables only)
   __syncthreads();
+  // the EOS and region tables, whose loads overlap the node sums
+  const int emat = mat > 0 ? mat : 0;
+  const int et = A.eos_itype[emat];
+  const double* ep = A.eos_param + BL_NEOSPARAM * emat;
+  const double ep0 = ep[0];
+  const CflIn cin = cfl_of_region(A, ereg - 1);
+  double x1 = x0, y1 = y0, u1 = u0, v1 = v0n;
   if (node) {
-    double x1 = x0, y1 = y0, u1 = u0, v1 = v0n;
     if (on) {
       // the entries around the node by corner; the two orders of its corners,
       // 2 bits a place, then the count
@@ -2247,6 +2272,9 @@ k_remap_tile(AleArgs B, FusedArgs A, FusedNodes H, FusedNodesOut W, double* cm_o
       W.u[n] = u1;
       W.v[n] = v1;
     }
+  }
+  __syncthreads();  // every thread has read its fluxes
+  if (node) {
     nout[0][tid] = x1;
     nout[1][tid] = y1;
     nout[2][tid] = u1;
@@ -2273,40 +2301,38 @@ k_remap_tile(AleArgs B, FusedArgs A, FusedNodes H, FusedNodesOut W, double* cm_o
 #pragma unroll
       for (int i1 = 0; i1 < 2; ++i1) {
         const int i2 = i1 + 2;
-        double w1 = s_ef[c.fc[i1]][(nbr >> (8 * i1)) & 0xffu];
-        double w2 = s_ef[c.fc[i2]][(nbr >> (8 * i2)) & 0xffu];
-        if (c.nb[i1] == e) w1 = 0.0;
-        if (c.nb[i2] == e) w2 = 0.0;
-        s = s - ef[i1] - ef[i2] + w1 + w2;
+        double w1 = s_ef[(faces >> (4 * i1)) & 3u][(nbr >> (8 * i1)) & 0xffu];
+        double w2 = s_ef[(faces >> (4 * i2)) & 3u][(nbr >> (8 * i2)) & 0xffu];
+        if ((faces >> (4 * i1)) & 4u) w1 = 0.0;
+        if ((faces >> (4 * i2)) & 4u) w2 = 0.0;
+        s = s - s_ef[i1][tid] - s_ef[i2][tid] + w1 + w2;
       }
-      const double m1 = m0 + totm;
+      const double m1 = m0 + totm, fl1 = s_fl[tid];
       double en = en0;
-      if (m1 > v0 * B.dencut) en = (en * m0 + s) / m1;
+      if (m1 > s_v0[tid] * B.dencut) en = (en * m0 + s) / m1;
       B.mass[e] = m1;
-      const double cm1[4] = {cm[0] + fl, cm[1] + fl, cm[2] + fl, cm[3] + fl};
+      const double cm1[4] = {s_cm[0][tid] + fl1, s_cm[1][tid] + fl1, s_cm[2][tid] + fl1,
+                             s_cm[3][tid] + fl1};
       st4(cm_out, e, cm1);
       const double r = m1 / g.vol;
-      ElIn ei;
-      el_eos(A, mat, ei);
       A.en_o[e] = en;
       A.rho_o[e] = r;
-      A.pre_o[e] = eos_pressure(ei.et, ei.p, r, en, B.pcut);
-      c2 = eos_cs2(ei.et, ei.p, r, en, B.pcut, B.ccut);
+      A.pre_o[e] = eos_pressure(et, ep0, ep, r, en, B.pcut);
+      c2 = eos_cs2(et, ep, r, en, B.pcut, B.ccut);
       A.cs2_o[e] = c2;
     } else {
-      st4(cm_out, e, cm);
+      double cm1[4];
+      ld4(B.cnmass, e, cm1);
+      st4(cm_out, e, cm1);
       A.en_o[e] = en0;
       A.rho_o[e] = A.rho[e];
       A.pre_o[e] = A.pre[e];
       c2 = A.cs2[e];
       A.cs2_o[e] = c2;
     }
-    if (MIX && mat < 0) {
-      f4_mix_cell(A, H, ts, -mat - 1, A.mx.cpe);
-      if (on && !A.dtres->negvol3)
-        mix_hydroupdate_iso(A.mx, -mat - 1, g, A.eos_itype, A.eos_param, A.pcut, A.ccut);
-    }
-    f1_terms(A, e, x, y, u, v, g, c2, moving, cflv, divv);
+    if (MIX && mat < 0 && on && !A.dtres->negvol3)
+      mix_hydroupdate_iso(A.mx, -mat - 1, g, A.eos_itype, A.eos_param, A.pcut, A.ccut);
+    f1_terms(A, e, x, y, u, v, g, c2, cin, moving, cflv, divv);
     A.rest8_next[e] = moving ? 0 : 1;
   }
   seg_collect(A, t, A.nseg, own, e, cflv, divv);
@@ -2518,6 +2544,7 @@ void tile_args(bl_handle_t* h, FusedArgs& A, int p, int s) {
   A.tile_el = h->d_tile_el;
   A.tile_nd = h->d_tile_nd;
   A.tile_nbr = h->d_tile_nbr;
+  A.tile_nbfc = h->d_tile_nbfc;
   A.tile_ninc = h->d_tile_ninc;
   A.rho = h->elset[s][0]; A.en = h->elset[s][1]; A.pre = h->elset[s][2]; A.cs2 = h->elset[s][3];
   A.rho_o = h->elset[1 - s][0]; A.en_o = h->elset[1 - s][1];
@@ -2634,7 +2661,13 @@ int launch_ale_step(bl_handle_t* h, int p, int stop_at_time_end) {
   B.cnmass = cm[p];
   FusedNodes H{O.x, O.y, O.u, O.v};
   FusedNodesOut W{h->nodeset[s][0], h->nodeset[s][1], h->nodeset[s][2], h->nodeset[s][3]};
-  BL_LAUNCH(h, "remap_faces", k_remap_faces, nblocks(h->sz.nel), kBlock, B);
+  const unsigned nbe = nblocks(h->sz.nel);
+  if (A.mx.ncp > 0) {
+    const unsigned nbm8 = (nblocks(A.mx.nmx) + kNumXcd - 1) / kNumXcd * kNumXcd;
+    BL_LAUNCH(h, "remap_faces", k_remap_faces<true>, nbm8 + nbe, kBlock, B, A, H, (int)nbm8);
+  } else {
+    BL_LAUNCH(h, "remap_faces", k_remap_faces<false>, nbe, kBlock, B, A, H, 0);
+  }
   if (A.mx.ncp > 0)
     BL_LAUNCH(h, "remap_tile", k_remap_tile<true>, (unsigned)h->ntile, kBlock, B, R, H, W,
               cm[1 - p]);

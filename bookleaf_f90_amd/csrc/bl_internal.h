@@ -240,6 +240,7 @@ struct Handle {
   // corner-mass array (the first is the registry's); the mesh velocity of
   // the node relaxation; the component energies after the predictor
   int32_t* d_tile_nbr = nullptr;
+  int4* d_tile_nbfc = nullptr;    // per tile entry: its packed ielel/ielfc
   int2* d_tile_ninc = nullptr;
   double* cm_other = nullptr;
   double* mesh_w[2] = {};

@@ -110,7 +110,7 @@ int upload_vec(T** d, const std::vector<T>& v) {
 
 void free_tiles(Handle* h) {
   void* bufs[] = {h->d_tile_eptr, h->d_tile_nptr, h->d_tile_bounds, h->d_tile_nodes, h->d_tile_ncm, h->d_tile_el,
-                  h->d_tile_nd, h->d_rest8, h->d_ens_toff, h->d_tile_nbr, h->d_tile_ninc};
+                  h->d_tile_nd, h->d_rest8, h->d_ens_toff, h->d_tile_nbr, h->d_tile_nbfc, h->d_tile_ninc};
   for (void* p : bufs)
     if (p) hipFree(p);
   h->d_tile_eptr = h->d_tile_nptr = h->d_tile_nodes = nullptr;
@@ -120,6 +120,7 @@ void free_tiles(Handle* h) {
   h->d_tile_nd = nullptr;
   h->d_ens_toff = nullptr;
   h->d_tile_nbr = nullptr;
+  h->d_tile_nbfc = nullptr;
   h->d_tile_ninc = nullptr;
   h->ale_tables = false;
   h->d_rest8 = nullptr;
@@ -293,8 +294,10 @@ int build_tiles(Handle* h) {
 
 int build_ale_tiles(Handle* h) {
   if (h->d_tile_nbr) hipFree(h->d_tile_nbr);
+  if (h->d_tile_nbfc) hipFree(h->d_tile_nbfc);
   if (h->d_tile_ninc) hipFree(h->d_tile_ninc);
   h->d_tile_nbr = nullptr;
+  h->d_tile_nbfc = nullptr;
   h->d_tile_ninc = nullptr;
   h->ale_tables = true;
   const int nel = h->sz.nel, ntile = h->ntile;
@@ -320,6 +323,10 @@ int build_ale_tiles(Handle* h) {
   }
   std::vector<int32_t> nbr(ents.size(), 0), local(nel, -1), stamp(nel, -1);
   std::vector<int2> ninc(nptr[ntile], make_int2(0, 0));
+  std::vector<int4> nbfc(ents.size());
+  auto packed = [&](int e, int i) {
+    return ((el[4 * (size_t)e + i] - 1) << 2) | ((fc[4 * (size_t)e + i] - 1) & 3);
+  };
   struct Inc { int32_t e, j; };
   std::vector<Inc> inc(4 * (kTileNodes + 1));
   std::vector<int> cnt(kTileNodes + 1);
@@ -330,6 +337,7 @@ int build_ale_tiles(Handle* h) {
       const int e = ents[eb + k].x & 0x3fffffff;
       local[e] = k;
       stamp[e] = t;
+      nbfc[eb + k] = make_int4(packed(e, 0), packed(e, 1), packed(e, 2), packed(e, 3));
       for (int j = 0; j < 4; ++j) {
         const uint32_t sl = ((uint32_t)ents[eb + k].y >> (8 * j)) & 0xFFu;
         if (sl == kNoSlot) continue;
@@ -368,7 +376,9 @@ int build_ale_tiles(Handle* h) {
       ninc[nb + v].y = (int)code;
     }
   }
-  if (upload_vec(&h->d_tile_ninc, ninc) || upload_vec(&h->d_tile_nbr, nbr)) return BL_FAILURE;
+  if (upload_vec(&h->d_tile_ninc, ninc) || upload_vec(&h->d_tile_nbfc, nbfc) ||
+      upload_vec(&h->d_tile_nbr, nbr))
+    return BL_FAILURE;
   return BL_SUCCESS;
 }
 
