@@ -721,8 +721,8 @@ __global__ void __launch_bounds__(kFinalBlock) k_f1b_select(FusedArgs A, int nb,
 // union of the instances' meshes, instance k owning elements [eoff[k],
 // eoff[k+1]).  Every instance has at least kBlock elements, so a workgroup
 // of F1 spans at most two instances (a and b); it keeps two partial slots of
-// each control.  F1L gives each instance one workgroup per chunk (4096 unless tuned) of its
-// elements, striding over the instance's own worklist segment, and E1b
+// each control.  F1L gives each instance one workgroup per piece of its
+// elements (ens_set_chunk), striding over the instance's own worklist segment, and E1b
 // selects each instance's dt in one workgroup per instance.  Each instance's selection is the first-index
 // extremum over its own (value, index) pairs, as a run of that instance
 // alone makes it.
@@ -795,7 +795,8 @@ k_e1_getdt(FusedArgs A, FusedNodes N, EnsArgs E) {
 }
 
 // E1L: instance k's workgroups lboff[k] .. lboff[k+1]-1 stride over its
-// worklist segment
+// worklist segment; a last round that fills at most a quarter of their lanes
+// takes a quad of lanes per element
 __global__ void __launch_bounds__(kBlock)
 k_e1_limiter(FusedArgs A, FusedNodes N, EnsArgs E) {
   if (step_skipped(A, A.ts)) return;
@@ -809,9 +810,22 @@ k_e1_limiter(FusedArgs A, FusedNodes N, EnsArgs E) {
   const uint32_t count = min(E.cnt[k], (uint32_t)(E.eoff[k + 1] - base));
   double best = DBL_MAX;
   int bi = 0x7fffffff;
-  for (uint32_t q = sub * blockDim.x + threadIdx.x; q < count; q += nbk * blockDim.x) {
-    const int e = A.work[base + q];
-    better_min(best, bi, f1_moving(A, N, e), e + 1);
+  const uint32_t round = nbk * blockDim.x;
+  uint32_t done = 0;
+  for (; 4 * (count - done) > round; done += min(count - done, round)) {
+    const uint32_t q = done + sub * blockDim.x + threadIdx.x;
+    if (q < count) {
+      const int e = A.work[base + q];
+      better_min(best, bi, f1_moving(A, N, e), e + 1);
+    }
+  }
+  // (whole waves: a quad past the end repeats the last element)
+  const uint32_t first = sub * blockDim.x + (threadIdx.x & ~63u);
+  if (done + first / 4 < count) {
+    const uint32_t q = done + (sub * blockDim.x + threadIdx.x) / 4;
+    const int e = A.work[base + min(q, count - 1)];
+    const double cfl = f1_moving_quad(A, N, e, threadIdx.x & 3, q < count);
+    better_min(best, bi, cfl, e + 1);
   }
   block_reduce_at<true>(best, bi, E.lpart + blockIdx.x, E.lparti + blockIdx.x);
 }
@@ -2025,12 +2039,14 @@ __global__ void __launch_bounds__(kBlock) k_r5(AleArgs B, DevTimestep* tsw) {
 // R5's, in their order.
 //
 // Against F1 to F4 and R1 to R5 in eleven kernels, per step: two-material
-// Eulerian Sod 2048x256 with mixed cells 240 -> 146 us, Eulerian Sedov 401^2
-// 105 -> 64 us, Eulerian Sod 100x25 58 -> 37 us, EQUI relaxation 1024x512
-// 309 -> 203 us: the corner terms, fluxes and corner masses that went through
+// Eulerian Sod 2048x256 with mixed cells 244 -> 128 us, Eulerian Sedov 401^2
+// 105 -> 56 us, Eulerian Sod 100x25 58 -> 31 us, EQUI relaxation 1024x512
+// 306 -> 185 us: the corner terms, fluxes and corner masses that went through
 // HBM between the kernels (about 900 B an element) stay in LDS, and F1 needs
-// no pass of its own.  Bound by latency: three workgroups a CU (45 KB of LDS,
-// at most 168 VGPRs) of dependent gathers and divisions.  A tiling is used
+// no pass of its own.  Bound by latency: four workgroups a CU (37 KB of LDS,
+// at most 128 VGPRs) of dependent gathers and divisions.  Three a CU (45 KB,
+// 167 VGPRs) took 57 us on the mixed Sod against 47 and 84 on the relaxation
+// against 72.  A tiling is used
 // wherever the mesh has one; the eleven kernels remain for meshes without.
 
 // R1's face mass fluxes (and a negative volume of the moved mesh, which R3

@@ -470,7 +470,7 @@ int bl_run_stats(bl_handle_t* h, int64_t* moving, int64_t* zeroed);
 typedef struct {
   int32_t limiter_block; /* threads per workgroup */
   int32_t limiter_grid;  /* workgroups launched */
-  int32_t ens_chunk;     /* ensemble: elements per workgroup and instance; 0 otherwise */
+  int32_t ens_chunk;     /* ensemble: most elements per workgroup and instance; 0 otherwise */
   int32_t trials;        /* shapes timed */
   double best_us;        /* median duration of the chosen shape, current worklist */
   double default_us;     /* the same for the shape in use before the call */
