@@ -26,7 +26,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
+#include <cstdlib>
+#include <exception>
+#include <memory>
+#include <new>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "bl_internal.h"
@@ -36,65 +43,144 @@ namespace bl {
 
 namespace {
 
+// The set-up is host work over every element, shared by up to kThreads
+// threads: a first run call of 524288 elements with mixed cells and the
+// remap took 110 ms with one and 44 with eight (10 of either are its steps).
+// The result does not depend on their number.
+constexpr int kThreads = 8;
+
+// a and b at once, each to its end; what either throws is thrown here
+template <typename F, typename G>
+void both(F&& a, G&& b) {
+  std::exception_ptr ea, eb;
+  auto run_b = [&] {
+    try { b(); } catch (...) { eb = std::current_exception(); }
+  };
+  std::thread t;
+  try {
+    t = std::thread(run_b);
+  } catch (const std::system_error&) {  // no thread to be had
+  }
+  try { a(); } catch (...) { ea = std::current_exception(); }
+  if (t.joinable()) t.join();
+  else run_b();
+  if (ea) std::rethrow_exception(ea);
+  if (eb) std::rethrow_exception(eb);
+}
+
+// f(p) for every part p in [lo, hi), each on a thread of its own
+template <typename F>
+void each_part(int lo, int hi, F& f) {
+  if (hi - lo < 2) {
+    if (lo < hi) f(lo);
+    return;
+  }
+  const int mid = (lo + hi) / 2;
+  both([&] { each_part(lo, mid, f); }, [&] { each_part(mid, hi, f); });
+}
+// the parts of n pieces of work, at least `least` each
+int parts_of(int64_t n, int64_t least) {
+  return (int)std::max<int64_t>(1, std::min<int64_t>(kThreads, n / least));
+}
+
+// zeros, whose pages a thread takes as it touches them
+struct Zeros {
+  std::unique_ptr<int32_t, void (*)(void*)> p;
+  explicit Zeros(size_t n)
+      : p(static_cast<int32_t*>(std::calloc(std::max<size_t>(n, 1), sizeof(int32_t))), std::free) {
+    if (!p) throw std::bad_alloc();
+  }
+  int32_t& operator[](size_t k) { return p.get()[k]; }
+};
+
 // Recursive coordinate bisection of the elements by their centroids: each
 // cut along the longer side of the element set's bounding box, at the share
 // that keeps the tile counts of the two sides proportional, down to about
 // kTileTarget elements; a leaf whose nodes or the elements around them do
 // not fit one workgroup is cut again.
+struct Centroid {
+  double x, y;
+  int32_t e;
+};
+using Leaves = std::vector<std::pair<int, int>>;
 struct Rcb {
-  const std::vector<double>& cx;
-  const std::vector<double>& cy;
-  const std::vector<int32_t>& ielnd;     // 4 per element, 1-based
-  const std::vector<int32_t>& adj_ptr;  // node -> incident elements
-  const std::vector<int32_t>& adj;
-  std::vector<int32_t> idx;              // element ids, cut in place
-  std::vector<int32_t> nstamp;           // per node: last count that saw it
-  std::vector<int32_t> estamp;           // per element: the same
-  std::vector<std::pair<int, int>> leaves;
-  int counter = 0;
+  const std::vector<int32_t>& ielnd;  // 4 per element, 1-based
+  const std::vector<int32_t>& inc;    // 4 per node: the element whose corner j it is, or -1
+  std::vector<Centroid>& el;          // cut in place
 
-  // the nodes of idx[lo, hi) fit the tile's node slots and the elements
+  struct Scratch {
+    Zeros nstamp, estamp;  // per node and element: the last count that saw it
+    int counter = 0;
+    Scratch(size_t nnd, size_t nel) : nstamp(nnd), estamp(nel) {}
+  };
+
+  // the nodes of el[lo, hi) fit the tile's node slots and the elements
   // around them one workgroup
-  bool fits(int lo, int hi) {
-    ++counter;
+  bool fits(int lo, int hi, Scratch& s) const {
+    ++s.counter;
     int nn = 0, ne = 0;
     for (int k = lo; k < hi; ++k)
       for (int j = 0; j < 4; ++j) {
-        const int v = ielnd[4 * (size_t)idx[k] + j] - 1;
-        if (nstamp[v] == counter) continue;
-        nstamp[v] = counter;
+        const int v = ielnd[4 * (size_t)el[k].e + j] - 1;
+        if (s.nstamp[v] == s.counter) continue;
+        s.nstamp[v] = s.counter;
         if (++nn > kTileNodes) return false;
-        for (int q = adj_ptr[v]; q < adj_ptr[v + 1]; ++q)
-          if (estamp[adj[q]] != counter) {
-            estamp[adj[q]] = counter;
-            if (++ne > kTileEls) return false;
-          }
+        for (int q = 0; q < 4; ++q) {
+          const int32_t b = inc[4 * (size_t)v + q];
+          if (b < 0 || s.estamp[b] == s.counter) continue;
+          s.estamp[b] = s.counter;
+          if (++ne > kTileEls) return false;
+        }
       }
     return true;
   }
 
-  void cut(int lo, int hi, int k) {
+  // cuts [lo, hi) at el[m]; returns m
+  int halve(int lo, int hi, int k, int k1) {
+    double x0 = el[lo].x, x1 = x0, y0 = el[lo].y, y1 = y0;
+    for (int q = lo + 1; q < hi; ++q) {
+      x0 = std::min(x0, el[q].x); x1 = std::max(x1, el[q].x);
+      y0 = std::min(y0, el[q].y); y1 = std::max(y1, el[q].y);
+    }
+    int m = lo + (int)((int64_t)(hi - lo) * k1 / k);
+    m = std::max(lo + 1, std::min(hi - 1, m));
+    auto at = [&](int q) { return el.begin() + q; };
+    if (x1 - x0 >= y1 - y0)
+      std::nth_element(at(lo), at(m), at(hi), [](const Centroid& a, const Centroid& b) {
+        return a.x < b.x || (a.x == b.x && a.e < b.e);
+      });
+    else
+      std::nth_element(at(lo), at(m), at(hi), [](const Centroid& a, const Centroid& b) {
+        return a.y < b.y || (a.y == b.y && a.e < b.e);
+      });
+    return m;
+  }
+
+  void cut(int lo, int hi, int k, Leaves& out, Scratch& s) {
     if (k <= 1) {
-      if (hi - lo < 2 || fits(lo, hi)) {
-        leaves.emplace_back(lo, hi);
+      if (hi - lo < 2 || fits(lo, hi, s)) {
+        out.emplace_back(lo, hi);
         return;
       }
       k = 2;
     }
-    double x0 = cx[idx[lo]], x1 = x0, y0 = cy[idx[lo]], y1 = y0;
-    for (int q = lo + 1; q < hi; ++q) {
-      const int e = idx[q];
-      x0 = std::min(x0, cx[e]); x1 = std::max(x1, cx[e]);
-      y0 = std::min(y0, cy[e]); y1 = std::max(y1, cy[e]);
+    const int k1 = k / 2, m = halve(lo, hi, k, k1);
+    cut(lo, m, k1, out, s);
+    cut(m, hi, k - k1, out, s);
+  }
+
+  // the same by `threads` threads
+  void cut_by(int threads, int lo, int hi, int k, Leaves& out) {
+    if (threads < 2 || k < 64) {
+      Scratch s(inc.size() / 4, el.size());
+      cut(lo, hi, k, out, s);
+      return;
     }
-    const std::vector<double>& c = (x1 - x0 >= y1 - y0) ? cx : cy;
-    const int k1 = k / 2;
-    int m = lo + (int)((int64_t)(hi - lo) * k1 / k);
-    m = std::max(lo + 1, std::min(hi - 1, m));
-    std::nth_element(idx.begin() + lo, idx.begin() + m, idx.begin() + hi,
-                     [&c](int32_t a, int32_t b) { return c[a] < c[b] || (c[a] == c[b] && a < b); });
-    cut(lo, m, k1);
-    cut(m, hi, k - k1);
+    const int k1 = k / 2, m = halve(lo, hi, k, k1);
+    Leaves right;
+    both([&] { cut_by(threads / 2, lo, m, k1, out); },
+         [&] { cut_by(threads - threads / 2, m, hi, k - k1, right); });
+    out.insert(out.end(), right.begin(), right.end());
   }
 };
 
@@ -109,8 +195,9 @@ int upload_vec(T** d, const std::vector<T>& v) {
 }  // namespace
 
 void free_tiles(Handle* h) {
-  void* bufs[] = {h->d_tile_eptr, h->d_tile_nptr, h->d_tile_bounds, h->d_tile_nodes, h->d_tile_ncm, h->d_tile_el,
-                  h->d_tile_nd, h->d_rest8, h->d_ens_toff, h->d_tile_nbr, h->d_tile_nbfc, h->d_tile_ninc};
+  void* bufs[] = {h->d_tile_eptr, h->d_tile_nptr, h->d_tile_bounds, h->d_tile_nodes,
+                  h->d_tile_ncm,  h->d_tile_el,   h->d_tile_nd,     h->d_rest8,
+                  h->d_ens_toff,  h->d_tile_nbr,  h->d_tile_nbfc,   h->d_tile_ninc};
   for (void* p : bufs)
     if (p) hipFree(p);
   h->d_tile_eptr = h->d_tile_nptr = h->d_tile_nodes = nullptr;
@@ -128,7 +215,35 @@ void free_tiles(Handle* h) {
   h->tile_state = 0;
 }
 
-int build_tiles(Handle* h) {
+namespace {
+
+// one thread's tiles
+struct TilePart {
+  std::vector<int32_t> nodes;
+  std::vector<uint8_t> ncm;
+  std::vector<int2> ents;
+  std::vector<int4> ent_nd;
+  bool fits = true;
+};
+
+// a table on the device from the parts' own, one after another
+template <typename T>
+int upload_parts(T** d, const std::vector<TilePart>& parts, std::vector<T> TilePart::*v) {
+  size_t n = 0;
+  for (const TilePart& p : parts) n += (p.*v).size();
+  if (*d) { hipFree(*d); *d = nullptr; }
+  BL_HIP(hipMalloc(d, sizeof(T) * std::max<size_t>(n, 1)));
+  size_t at = 0;
+  for (const TilePart& p : parts) {
+    const std::vector<T>& q = p.*v;
+    if (!q.empty())
+      BL_HIP(hipMemcpy(*d + at, q.data(), sizeof(T) * q.size(), hipMemcpyHostToDevice));
+    at += q.size();
+  }
+  return BL_SUCCESS;
+}
+
+int cut_tiles(Handle* h) {
   free_tiles(h);
   const int nel = h->sz.nel, nnd = h->sz.nnd;
   std::vector<int32_t> ielnd(4 * (size_t)nel);
@@ -137,137 +252,174 @@ int build_tiles(Handle* h) {
   if (bl_download(hh, BL_IELND, ielnd.data(), 4 * (int64_t)nel) ||
       bl_download(hh, BL_NDX, x.data(), nnd) || bl_download(hh, BL_NDY, y.data(), nnd))
     return BL_FAILURE;
-  // every node is corner jj of at most one element, for each jj
-  std::vector<uint8_t> seen(4 * (size_t)nnd, 0);
-  std::vector<int32_t> adj_ptr(nnd + 1, 0);
+  // every node is corner jj of at most one element, for each jj, and of one
+  // element at least (a node no element uses would be written by no tile);
+  // an element with a repeated node is there once per corner
+  std::vector<int32_t> inc(4 * (size_t)nnd, -1);
   for (int e = 0; e < nel; ++e)
     for (int j = 0; j < 4; ++j) {
       const int v = ielnd[4 * (size_t)e + j] - 1;
-      if (v < 0 || v >= nnd || seen[4 * (size_t)v + j]) {
+      if (v < 0 || v >= nnd || inc[4 * (size_t)v + j] >= 0) {
         h->tile_state = -1;  // not a tiling this step can use
         return BL_SUCCESS;
       }
-      seen[4 * (size_t)v + j] = 1;
-      ++adj_ptr[v + 1];
+      inc[4 * (size_t)v + j] = e;
     }
-  for (int v = 0; v < nnd; ++v) {
-    // a node no element uses would be written by no tile
-    if (adj_ptr[v + 1] == 0) {
+  // the node's first incident element
+  auto first_of = [&](int v) {
+    int e = nel;
+    for (int j = 0; j < 4; ++j)
+      if (inc[4 * (size_t)v + j] >= 0) e = std::min(e, inc[4 * (size_t)v + j]);
+    return e;
+  };
+  for (int v = 0; v < nnd; ++v)
+    if (first_of(v) == nel) {
       h->tile_state = -1;
       return BL_SUCCESS;
     }
-    adj_ptr[v + 1] += adj_ptr[v];
-  }
-  // (an element with a repeated node is listed once per corner: the counts
-  // below take each element once)
-  std::vector<int32_t> adj(adj_ptr[nnd]), fill(adj_ptr.begin(), adj_ptr.end() - 1);
-  for (int e = 0; e < nel; ++e)
-    for (int j = 0; j < 4; ++j) adj[fill[ielnd[4 * (size_t)e + j] - 1]++] = e;
   if (nel >= (1 << 30) || nnd >= (1 << 31) - 1) { h->tile_state = -1; return BL_SUCCESS; }
-  std::vector<double> cx(nel), cy(nel);
-  for (int e = 0; e < nel; ++e) {
-    const int32_t* q = &ielnd[4 * (size_t)e];
-    cx[e] = 0.25 * (x[q[0] - 1] + x[q[1] - 1] + x[q[2] - 1] + x[q[3] - 1]);
-    cy[e] = 0.25 * (y[q[0] - 1] + y[q[1] - 1] + y[q[2] - 1] + y[q[3] - 1]);
-  }
-  Rcb r{cx, cy, ielnd, adj_ptr, adj, {}, std::vector<int32_t>(nnd, 0),
-        std::vector<int32_t>(nel, 0), {}, 0};
-  r.idx.resize(nel);
-  for (int e = 0; e < nel; ++e) r.idx[e] = e;
+  std::vector<Centroid> el(nel);
+  const int npart = parts_of(nel, 16384);
+  auto share = [](int64_t n, int p, int np) { return (int)(n * p / np); };
+  auto centroids = [&](int p) {
+    for (int e = share(nel, p, npart), e1 = share(nel, p + 1, npart); e < e1; ++e) {
+      const int32_t* q = &ielnd[4 * (size_t)e];
+      el[e] = Centroid{0.25 * (x[q[0] - 1] + x[q[1] - 1] + x[q[2] - 1] + x[q[3] - 1]),
+                       0.25 * (y[q[0] - 1] + y[q[1] - 1] + y[q[2] - 1] + y[q[3] - 1]), e};
+    }
+  };
+  each_part(0, npart, centroids);
+  Rcb r{ielnd, inc, el};
+  Leaves leaves;
   // an ensemble's instances own contiguous element ranges: each is cut on
   // its own, so that a tile lies in one instance (one dt)
   std::vector<int32_t> toff;
+  auto tiles_for = [](int n) { return std::max(1, (n + kTileTarget - 1) / kTileTarget); };
   if (h->ens_n > 0) {
-    toff.assign(h->ens_n + 1, 0);
-    for (int k = 0; k < h->ens_n; ++k) {
-      const int lo = h->ens_eoff[k], hi = h->ens_eoff[k + 1];
-      toff[k] = (int)r.leaves.size();
-      r.cut(lo, hi, std::max(1, (hi - lo + kTileTarget - 1) / kTileTarget));
+    const int ninst = h->ens_n, np = parts_of(std::min<int64_t>(nel / 16384, ninst), 1);
+    std::vector<Leaves> out(ninst);
+    auto cut_some = [&](int p) {
+      Rcb::Scratch s(nnd, nel);
+      for (int k = share(ninst, p, np); k < share(ninst, p + 1, np); ++k) {
+        const int lo = h->ens_eoff[k], hi = h->ens_eoff[k + 1];
+        r.cut(lo, hi, tiles_for(hi - lo), out[k], s);
+      }
+    };
+    each_part(0, np, cut_some);
+    toff.push_back(0);
+    for (const Leaves& o : out) {
+      leaves.insert(leaves.end(), o.begin(), o.end());
+      toff.push_back((int)leaves.size());
     }
-    toff[h->ens_n] = (int)r.leaves.size();
   } else {
-    r.cut(0, nel, std::max(1, (nel + kTileTarget - 1) / kTileTarget));
+    r.cut_by(kThreads, 0, nel, tiles_for(nel), leaves);
   }
 
-  const int ntile = (int)r.leaves.size();
+  const int ntile = (int)leaves.size();
   std::vector<int32_t> tile_of(nel);
   for (int t = 0; t < ntile; ++t)
-    for (int k = r.leaves[t].first; k < r.leaves[t].second; ++k) tile_of[r.idx[k]] = t;
+    for (int k = leaves[t].first; k < leaves[t].second; ++k) tile_of[el[k].e] = t;
   // per tile: its nodes (ascending; the high bit marks the tile that writes
   // the node, the one holding the node's first incident element), then the
   // entries: its own elements ascending, then the ring around them
-  std::vector<int32_t> nptr(ntile + 1, 0), nodes, eptr(ntile + 1, 0);
-  std::vector<uint8_t> ncm;
-  std::vector<int2> ents;
-  std::vector<int4> ent_nd;
-  nodes.reserve((size_t)nnd + nnd / 4);
-  ncm.reserve((size_t)nnd + nnd / 4);
-  ents.reserve((size_t)nel + nel / 2);
-  ent_nd.reserve((size_t)nel + nel / 2);
-  std::vector<int32_t> nstamp(nnd, -1), slot_of(nnd, 0), estamp(nel, -1), tn, own, ring;
-  for (int t = 0; t < ntile; ++t) {
-    own.assign(r.idx.begin() + r.leaves[t].first, r.idx.begin() + r.leaves[t].second);
-    std::sort(own.begin(), own.end());
-    tn.clear();
-    for (int e : own) {
-      estamp[e] = t;
-      for (int j = 0; j < 4; ++j) {
-        const int v = ielnd[4 * (size_t)e + j] - 1;
-        if (nstamp[v] != t) { nstamp[v] = t; tn.push_back(v); }
-      }
+  const int nasm = parts_of(ntile, 64);
+  std::vector<TilePart> parts(nasm);
+  std::vector<int32_t> nptr(ntile + 1, 0), eptr(ntile + 1, 0);  // of the part, then of the whole
+  auto assemble = [&](int p) {
+    TilePart& o = parts[p];
+    Zeros nstamp(nnd), slot_of(nnd), estamp(nel);
+    std::vector<int32_t> tn, own, ring;
+    const int t0 = share(ntile, p, nasm), t1 = share(ntile, p + 1, nasm);
+    if (t0 < t1) {
+      const size_t n = (size_t)(leaves[t1 - 1].second - leaves[t0].first);
+      o.nodes.reserve(n + n / 3);
+      o.ncm.reserve(n + n / 3);
+      o.ents.reserve(n + n / 2);
+      o.ent_nd.reserve(n + n / 2);
     }
-    std::sort(tn.begin(), tn.end());
-    ring.clear();
-    for (int v : tn)
-      for (int q = adj_ptr[v]; q < adj_ptr[v + 1]; ++q)
-        if (estamp[adj[q]] != t) { estamp[adj[q]] = t; ring.push_back(adj[q]); }
-    std::sort(ring.begin(), ring.end());
-    if ((int)tn.size() > kTileNodes || own.size() + ring.size() > (size_t)kTileEls) {
+    for (int t = t0; t < t1; ++t) {
+      const int stamp = t - t0 + 1;
+      own.clear();
+      for (int k = leaves[t].first; k < leaves[t].second; ++k) own.push_back(el[k].e);
+      std::sort(own.begin(), own.end());
+      tn.clear();
+      for (int e : own) {
+        estamp[e] = stamp;
+        for (int j = 0; j < 4; ++j) {
+          const int v = ielnd[4 * (size_t)e + j] - 1;
+          if (nstamp[v] != stamp) { nstamp[v] = stamp; tn.push_back(v); }
+        }
+      }
+      std::sort(tn.begin(), tn.end());
+      ring.clear();
+      for (int v : tn)
+        for (int j = 0; j < 4; ++j) {
+          const int32_t e = inc[4 * (size_t)v + j];
+          if (e >= 0 && estamp[e] != stamp) { estamp[e] = stamp; ring.push_back(e); }
+        }
+      std::sort(ring.begin(), ring.end());
+      if ((int)tn.size() > kTileNodes || own.size() + ring.size() > (size_t)kTileEls) {
+        o.fits = false;
+        return;
+      }
+      nptr[t] = (int)o.nodes.size();
+      for (size_t k = 0; k < tn.size(); ++k) {
+        const int v = tn[k];
+        slot_of[v] = (int)k;
+        const bool writes = tile_of[first_of(v)] == t;
+        o.nodes.push_back((int32_t)((uint32_t)v | (writes ? 0x80000000u : 0u)));
+        // the corners jj the node is (every element around it is an entry
+        // of this tile, own or ring)
+        uint8_t cm = 0;
+        for (int j = 0; j < 4; ++j) cm |= inc[4 * (size_t)v + j] >= 0 ? (uint8_t)(1u << j) : 0u;
+        o.ncm.push_back(cm);
+      }
+      eptr[t] = (int)o.ents.size();
+      for (int pass = 0; pass < 2; ++pass)
+        for (int e : pass == 0 ? own : ring) {
+          uint32_t slots = 0;
+          for (int j = 0; j < 4; ++j) {
+            const int v = ielnd[4 * (size_t)e + j] - 1;
+            slots |= (uint32_t)(nstamp[v] == stamp ? (uint32_t)slot_of[v] : kNoSlot) << (8 * j);
+          }
+          // an own element: this tile completes and writes it
+          const uint32_t flags = pass == 0 ? kTileOwn : 0u;
+          o.ents.push_back(make_int2((int)((uint32_t)e | (flags << 30)), (int)slots));
+          const int32_t* q = &ielnd[4 * (size_t)e];
+          o.ent_nd.push_back(make_int4(q[0] - 1, q[1] - 1, q[2] - 1, q[3] - 1));
+        }
+    }
+  };
+  each_part(0, nasm, assemble);
+  int nn = 0, ne = 0;
+  for (int p = 0; p < nasm; ++p) {
+    if (!parts[p].fits) {
       h->tile_state = -1;
       return BL_SUCCESS;
     }
-    nptr[t] = (int)nodes.size();
-    for (size_t k = 0; k < tn.size(); ++k) {
-      const int v = tn[k];
-      slot_of[v] = (int)k;
-      const bool writes = tile_of[adj[adj_ptr[v]]] == t;
-      nodes.push_back((int32_t)((uint32_t)v | (writes ? 0x80000000u : 0u)));
-      // the corners jj the node is (every element around it is an entry
-      // of this tile, own or ring)
-      uint8_t cm = 0;
-      for (int j = 0; j < 4; ++j) cm |= seen[4 * (size_t)v + j] ? (uint8_t)(1u << j) : 0u;
-      ncm.push_back(cm);
+    for (int t = share(ntile, p, nasm); t < share(ntile, p + 1, nasm); ++t) {
+      nptr[t] += nn;
+      eptr[t] += ne;
     }
-    eptr[t] = (int)ents.size();
-    for (int pass = 0; pass < 2; ++pass)
-      for (int e : pass == 0 ? own : ring) {
-        uint32_t slots = 0;
-        for (int j = 0; j < 4; ++j) {
-          const int v = ielnd[4 * (size_t)e + j] - 1;
-          slots |= (uint32_t)(nstamp[v] == t ? slot_of[v] : kNoSlot) << (8 * j);
-        }
-        // an own element: this tile completes and writes it
-        const uint32_t flags = pass == 0 ? kTileOwn : 0u;
-        ents.push_back(make_int2((int)((uint32_t)e | (flags << 30)), (int)slots));
-        const int32_t* q = &ielnd[4 * (size_t)e];
-        ent_nd.push_back(make_int4(q[0] - 1, q[1] - 1, q[2] - 1, q[3] - 1));
-      }
+    nn += (int)parts[p].nodes.size();
+    ne += (int)parts[p].ents.size();
   }
-  nptr[ntile] = (int)nodes.size();
-  eptr[ntile] = (int)ents.size();
+  nptr[ntile] = nn;
+  eptr[ntile] = ne;
   std::vector<int4> bounds(ntile);
   for (int t = 0; t < ntile; ++t) bounds[t] = make_int4(eptr[t], eptr[t + 1], nptr[t], nptr[t + 1]);
   if (upload_vec(&h->d_tile_eptr, eptr) || upload_vec(&h->d_tile_nptr, nptr) ||
       upload_vec(&h->d_tile_bounds, bounds) ||
-      upload_vec(&h->d_tile_nodes, nodes) || upload_vec(&h->d_tile_ncm, ncm) ||
-      upload_vec(&h->d_tile_el, ents) ||
-      upload_vec(&h->d_tile_nd, ent_nd) ||
+      upload_parts(&h->d_tile_nodes, parts, &TilePart::nodes) ||
+      upload_parts(&h->d_tile_ncm, parts, &TilePart::ncm) ||
+      upload_parts(&h->d_tile_el, parts, &TilePart::ents) ||
+      upload_parts(&h->d_tile_nd, parts, &TilePart::ent_nd) ||
       (!toff.empty() && upload_vec(&h->d_ens_toff, toff)))
     return BL_FAILURE;
   BL_HIP(hipMalloc(&h->d_rest8, 2 * (size_t)std::max(nel, 1)));
   BL_HIP(hipMemset(h->d_rest8, 0, 2 * (size_t)std::max(nel, 1)));
   h->ntile = ntile;
-  h->nentries = (int32_t)ents.size();
+  h->nentries = ne;
   // the partial slots of the tile step: one per tile
   if (ntile + 16 > h->npart) {
     hipFree(h->d_part);
@@ -292,7 +444,7 @@ int build_tiles(Handle* h) {
   return BL_SUCCESS;
 }
 
-int build_ale_tiles(Handle* h) {
+int build_ale_tables(Handle* h) {
   if (h->d_tile_nbr) hipFree(h->d_tile_nbr);
   if (h->d_tile_nbfc) hipFree(h->d_tile_nbfc);
   if (h->d_tile_ninc) hipFree(h->d_tile_ninc);
@@ -321,65 +473,92 @@ int build_ale_tiles(Handle* h) {
     const int e = (sort2[k] < 1 || sort2[k] > nel) ? k : sort2[k] - 1;
     pos2[e] = k;
   }
-  std::vector<int32_t> nbr(ents.size(), 0), local(nel, -1), stamp(nel, -1);
+  std::vector<int32_t> nbr(ents.size(), 0);
   std::vector<int2> ninc(nptr[ntile], make_int2(0, 0));
   std::vector<int4> nbfc(ents.size());
   auto packed = [&](int e, int i) {
     return ((el[4 * (size_t)e + i] - 1) << 2) | ((fc[4 * (size_t)e + i] - 1) & 3);
   };
   struct Inc { int32_t e, j; };
-  std::vector<Inc> inc(4 * (kTileNodes + 1));
-  std::vector<int> cnt(kTileNodes + 1);
-  for (int t = 0; t < ntile; ++t) {
-    const int eb = eptr[t], ne = eptr[t + 1] - eb, nb = nptr[t], nn = nptr[t + 1] - nb;
-    std::fill(cnt.begin(), cnt.begin() + nn, 0);
-    for (int k = 0; k < ne; ++k) {
-      const int e = ents[eb + k].x & 0x3fffffff;
-      local[e] = k;
-      stamp[e] = t;
-      nbfc[eb + k] = make_int4(packed(e, 0), packed(e, 1), packed(e, 2), packed(e, 3));
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t sl = ((uint32_t)ents[eb + k].y >> (8 * j)) & 0xFFu;
-        if (sl == kNoSlot) continue;
-        // (at most four: no node is corner jj of two elements)
-        int2& q = ninc[nb + sl];
-        q.x = (int)((uint32_t)q.x | ((uint32_t)k << (8 * j)));
-        inc[4 * sl + cnt[sl]++] = Inc{e, j};
+  const int npart = parts_of(ntile, 64);
+  std::atomic<bool> runs{true};
+  auto some = [&](int p) {
+    Zeros local(nel), stamp(nel);
+    std::vector<Inc> inc(4 * (kTileNodes + 1));
+    std::vector<int> cnt(kTileNodes + 1);
+    const int t0 = (int)((int64_t)ntile * p / npart), t1 = (int)((int64_t)ntile * (p + 1) / npart);
+    for (int t = t0; t < t1; ++t) {
+      const int eb = eptr[t], ne = eptr[t + 1] - eb, nb = nptr[t], nn = nptr[t + 1] - nb;
+      std::fill(cnt.begin(), cnt.begin() + nn, 0);
+      for (int k = 0; k < ne; ++k) {
+        const int e = ents[eb + k].x & 0x3fffffff;
+        local[e] = k;
+        stamp[e] = t + 1;
+        nbfc[eb + k] = make_int4(packed(e, 0), packed(e, 1), packed(e, 2), packed(e, 3));
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t sl = ((uint32_t)ents[eb + k].y >> (8 * j)) & 0xFFu;
+          if (sl == kNoSlot) continue;
+          // (at most four: no node is corner jj of two elements)
+          int2& q = ninc[nb + sl];
+          q.x = (int)((uint32_t)q.x | ((uint32_t)k << (8 * j)));
+          inc[4 * sl + cnt[sl]++] = Inc{e, j};
+        }
+      }
+      for (int k = 0; k < ne; ++k) {
+        const uint32_t w = (uint32_t)ents[eb + k].x;
+        if (!((w >> 30) & kTileOwn)) continue;
+        const int e = (int)(w & 0x3fffffffu);
+        uint32_t bytes = 0;
+        for (int i = 0; i < 4; ++i) {
+          const int b = el[4 * (size_t)e + i] - 1, g = fc[4 * (size_t)e + i] - 1;
+          if (b < 0 || b >= nel || g < 0 || g > 3 || stamp[b] != t + 1 ||
+              (b == e && g != ((i + 2) & 3))) {
+            runs = false;  // not a mesh the tiled remap runs on
+            return;
+          }
+          bytes |= (uint32_t)local[b] << (8 * i);
+        }
+        nbr[eb + k] = (int32_t)bytes;
+      }
+      for (int v = 0; v < nn; ++v) {
+        Inc* q = &inc[4 * (size_t)v];
+        const int n = cnt[v];
+        uint32_t code = (uint32_t)n << 16;
+        std::sort(q, q + n, [&](const Inc& a, const Inc& b) {
+          return a.e != b.e ? pos2[a.e] < pos2[b.e] : a.j < b.j;
+        });
+        for (int k = 0; k < n; ++k) code |= (uint32_t)q[k].j << (2 * k);
+        std::sort(q, q + n, [](const Inc& a, const Inc& b) {
+          return a.e != b.e ? a.e < b.e : a.j < b.j;
+        });
+        for (int k = 0; k < n; ++k) code |= (uint32_t)q[k].j << (8 + 2 * k);
+        ninc[nb + v].y = (int)code;
       }
     }
-    for (int k = 0; k < ne; ++k) {
-      const uint32_t w = (uint32_t)ents[eb + k].x;
-      if (!((w >> 30) & kTileOwn)) continue;
-      const int e = (int)(w & 0x3fffffffu);
-      uint32_t bytes = 0;
-      for (int i = 0; i < 4; ++i) {
-        const int b = el[4 * (size_t)e + i] - 1, g = fc[4 * (size_t)e + i] - 1;
-        if (b < 0 || b >= nel || g < 0 || g > 3 || stamp[b] != t ||
-            (b == e && g != ((i + 2) & 3)))
-          return BL_SUCCESS;  // not a mesh the tiled remap runs on
-        bytes |= (uint32_t)local[b] << (8 * i);
-      }
-      nbr[eb + k] = (int32_t)bytes;
-    }
-    for (int v = 0; v < nn; ++v) {
-      Inc* q = &inc[4 * (size_t)v];
-      const int n = cnt[v];
-      uint32_t code = (uint32_t)n << 16;
-      std::sort(q, q + n, [&](const Inc& a, const Inc& b) {
-        return a.e != b.e ? pos2[a.e] < pos2[b.e] : a.j < b.j;
-      });
-      for (int k = 0; k < n; ++k) code |= (uint32_t)q[k].j << (2 * k);
-      std::sort(q, q + n, [](const Inc& a, const Inc& b) {
-        return a.e != b.e ? a.e < b.e : a.j < b.j;
-      });
-      for (int k = 0; k < n; ++k) code |= (uint32_t)q[k].j << (8 + 2 * k);
-      ninc[nb + v].y = (int)code;
-    }
-  }
+  };
+  each_part(0, npart, some);
+  if (!runs) return BL_SUCCESS;
   if (upload_vec(&h->d_tile_ninc, ninc) || upload_vec(&h->d_tile_nbfc, nbfc) ||
       upload_vec(&h->d_tile_nbr, nbr))
     return BL_FAILURE;
   return BL_SUCCESS;
 }
+
+// no exception passes the C entries
+template <typename F>
+int no_throw(F f, Handle* h) {
+  try {
+    return f(h);
+  } catch (const std::exception& e) {
+    set_error(std::string("tiles: ") + e.what());
+    return BL_FAILURE;
+  }
+}
+
+}  // namespace
+
+int build_tiles(Handle* h) { return no_throw(cut_tiles, h); }
+
+int build_ale_tiles(Handle* h) { return no_throw(build_ale_tables, h); }
 
 }  // namespace bl
