@@ -45,8 +45,11 @@ namespace {
 
 // The set-up is host work over every element, shared by up to kThreads
 // threads: a first run call of 524288 elements with mixed cells and the
-// remap took 110 ms with one and 44 with eight (10 of either are its steps).
-// The result does not depend on their number.
+// remap took 110 ms with one and 45 to 55 with eight (13 of either are its
+// steps).  A share is at least 32768 elements or 256 tiles: at 16384 and 64
+// the relaxation on 414x173 was ready after 93 ms, at these after 76, as a
+// thread that has to wait for a core costs more than it saves.  The result
+// does not depend on their number.
 constexpr int kThreads = 8;
 
 // a and b at once, each to its end; what either throws is thrown here
@@ -78,7 +81,7 @@ void each_part(int lo, int hi, F& f) {
   const int mid = (lo + hi) / 2;
   both([&] { each_part(lo, mid, f); }, [&] { each_part(mid, hi, f); });
 }
-// the parts of n pieces of work, at least `least` each
+// the shares of n pieces of work, at least `least` each
 int parts_of(int64_t n, int64_t least) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(kThreads, n / least));
 }
@@ -171,7 +174,7 @@ struct Rcb {
 
   // the same by `threads` threads
   void cut_by(int threads, int lo, int hi, int k, Leaves& out) {
-    if (threads < 2 || k < 64) {
+    if (threads < 2 || k < 256) {
       Scratch s(inc.size() / 4, el.size());
       cut(lo, hi, k, out, s);
       return;
@@ -279,7 +282,7 @@ int cut_tiles(Handle* h) {
     }
   if (nel >= (1 << 30) || nnd >= (1 << 31) - 1) { h->tile_state = -1; return BL_SUCCESS; }
   std::vector<Centroid> el(nel);
-  const int npart = parts_of(nel, 16384);
+  const int npart = parts_of(nel, 32768);
   auto share = [](int64_t n, int p, int np) { return (int)(n * p / np); };
   auto centroids = [&](int p) {
     for (int e = share(nel, p, npart), e1 = share(nel, p + 1, npart); e < e1; ++e) {
@@ -296,7 +299,7 @@ int cut_tiles(Handle* h) {
   std::vector<int32_t> toff;
   auto tiles_for = [](int n) { return std::max(1, (n + kTileTarget - 1) / kTileTarget); };
   if (h->ens_n > 0) {
-    const int ninst = h->ens_n, np = parts_of(std::min<int64_t>(nel / 16384, ninst), 1);
+    const int ninst = h->ens_n, np = parts_of(std::min<int64_t>(nel / 32768, ninst), 1);
     std::vector<Leaves> out(ninst);
     auto cut_some = [&](int p) {
       Rcb::Scratch s(nnd, nel);
@@ -322,7 +325,7 @@ int cut_tiles(Handle* h) {
   // per tile: its nodes (ascending; the high bit marks the tile that writes
   // the node, the one holding the node's first incident element), then the
   // entries: its own elements ascending, then the ring around them
-  const int nasm = parts_of(ntile, 64);
+  const int nasm = parts_of(ntile, 256);
   std::vector<TilePart> parts(nasm);
   std::vector<int32_t> nptr(ntile + 1, 0), eptr(ntile + 1, 0);  // of the part, then of the whole
   auto assemble = [&](int p) {
@@ -480,7 +483,7 @@ int build_ale_tables(Handle* h) {
     return ((el[4 * (size_t)e + i] - 1) << 2) | ((fc[4 * (size_t)e + i] - 1) & 3);
   };
   struct Inc { int32_t e, j; };
-  const int npart = parts_of(ntile, 64);
+  const int npart = parts_of(ntile, 256);
   std::atomic<bool> runs{true};
   auto some = [&](int p) {
     Zeros local(nel), stamp(nel);

@@ -33,7 +33,7 @@ def _neighbours(p):
 
 
 @pytest.mark.parametrize("nx,ny,turn", [(2, 1, 0), (19, 1, 1), (37, 29, 2), (190, 61, 3),
-                                        (300, 170, 1)])
+                                        (300, 170, 1), (430, 250, 2)])
 def test_tables(nx, ny, turn):
     from bookleaf_f90_amd.device import BookLeaf
     p = _renumbered(_stirred(P.sod(nx=nx, ny=ny, height=ny / nx, eulerian=True,
