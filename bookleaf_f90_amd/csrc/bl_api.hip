@@ -527,8 +527,8 @@ __global__ void k_getdt_b(int nel, double zerocut, double cvisc1, double cvisc2,
   ellength[e] = zdtnotreg[ireg] ? DBL_MIN : minlength(x, y, zcut, zmidlength[ireg] != 0);
 }
 
-// (a) and (b) in one pass on a mesh with the limiter's outer-node table
-// (build_outer): the neighbour edges' velocity differences from the nodes
+// (a) and (b) in one pass on a mesh whose outer-node table (build_outer)
+// follows its present connectivity: the neighbour edges' velocity differences from the nodes
 // (the table's far node, and the element's own node at the other end), their
 // position differences from the neighbours' corners, so that nothing waits
 // for (a)'s arrays.  An element whose four nodes share one velocity has zero
@@ -916,6 +916,7 @@ void* bl_field_device_ptr(bl_handle_t* h, int32_t id) {
   // stores through it are not seen here: no run call resumes after this
   h->ptr_out = true;
   h->resumable = false;
+  if (id == BL_IELND || id == BL_IELEL || id == BL_IELFC) h->conn_out = true;
   return h->f[id];
 }
 
@@ -927,7 +928,10 @@ int bl_upload(bl_handle_t* h, int32_t id, const void* host, int64_t count) {
   BL_HIP(hipMemcpyAsync(h->f[id], host, count * kind_bytes(h->kind[id]), hipMemcpyHostToDevice, h->stream));
   BL_HIP(hipStreamSynchronize(h->stream));
   if (id == BL_IELND || id == BL_IELSORT1 || id == BL_IELSORT2) { h->maps_built = false; invalidate_graph(h); }
-  if (id == BL_IELEL || id == BL_IELFC) { h->nbfc_stale = true; invalidate_graph(h); }
+  if (id == BL_IELEL || id == BL_IELFC) {
+    h->nbfc_stale = h->outer_stale = true;
+    invalidate_graph(h);
+  }
   return BL_SUCCESS;
 }
 
@@ -982,6 +986,7 @@ static int build_csr(bl_handle_t* h, const std::vector<int32_t>& nodes,
 static int build_outer(bl_handle_t* h, const std::vector<int32_t>& ielnd) {
   if (h->d_outer) hipFree(h->d_outer);
   h->d_outer = nullptr;
+  h->outer_stale = false;
   const int nel = h->sz.nel;
   std::vector<int32_t> ielel(4 * (size_t)nel), ielfc(4 * (size_t)nel);
   if (bl_download(h, BL_IELEL, ielel.data(), 4 * (int64_t)nel) ||
@@ -1015,6 +1020,20 @@ static int build_outer(bl_handle_t* h, const std::vector<int32_t>& ielnd) {
   }
   return upload_table(h, &h->d_outer, outer);
 }
+
+}  // extern "C"
+
+namespace bl {
+int refresh_outer(Handle* hh) {
+  if (!hh->outer_stale) return BL_SUCCESS;
+  bl_handle_t* h = static_cast<bl_handle_t*>(hh);
+  std::vector<int32_t> ielnd(4 * (size_t)h->sz.nel);
+  if (bl_download(h, BL_IELND, ielnd.data(), 4 * (int64_t)h->sz.nel)) return BL_FAILURE;
+  return build_outer(h, ielnd);
+}
+}  // namespace bl
+
+extern "C" {
 
 int bl_build_maps(bl_handle_t* h) {
   bl_touch(h);
@@ -1253,7 +1272,8 @@ static int getdt_with(bl_handle_t* h, double* part, int32_t* parti, DtResult* dr
   int nel = h->sz.nel;
   unsigned nb = nblocks(nel);
   const bl_config_t& c = h->cfg;
-  if (h->d_outer && h->maps_built) {
+  // (a stale table is not rebuilt here: bl_hydro_getdt_noalloc may not allocate)
+  if (h->d_outer && h->maps_built && !h->outer_stale && !h->conn_out) {
     BL_LAUNCH(h, "getdt_ab", k_getdt_ab, nb, kBlock, nel, c.zerocut, c.cvisc1, c.cvisc2, c.zcut,
               h->I(BL_INDTYPE), h->I(BL_IELEL), h->I(BL_IELND), h->I(BL_IELFC), h->I(BL_IELREG),
               h->d_outer, h->d_zdtnotreg, h->d_zmidlength, h->R(BL_NDU), h->R(BL_NDV),

@@ -3212,6 +3212,11 @@ int bl_ensemble_run(bl_handle_t* h, int32_t nsteps, double* dt_hist, int32_t* id
   }
   fill_err(err, BL_SUCCESS, 0, "");
   if (nsteps <= 0) { if (steps_taken) *steps_taken = 0; return BL_SUCCESS; }
+  if (refresh_outer(h)) return BL_FAILURE;
+  if (!h->d_outer) {
+    set_error("bl_ensemble_run: the neighbours uploaded do not meet face to face");
+    return BL_FAILURE;
+  }
   if (ensure_nodesets(h) || prepare_tiles(h) || ensure_step_buffers(h) || clear_rest(h))
     return BL_FAILURE;
   if (h->ehist_cap < nsteps) {
@@ -3341,7 +3346,8 @@ int bl_autotune(bl_handle_t* h, int32_t reps, bl_tuning_t* out) {
     return BL_FAILURE;
   }
   const bool ens = h->ens_n > 0;
-  if (!ens && (!h->maps_built || !h->d_eos_itype || !h->d_zdtnotreg || !h->d_outer)) {
+  if (refresh_outer(h)) return BL_FAILURE;
+  if (!h->d_outer || (!ens && (!h->maps_built || !h->d_eos_itype || !h->d_zdtnotreg))) {
     set_error("bl_autotune: mesh maps, regions or EOS not set");
     return BL_FAILURE;
   }
@@ -3594,6 +3600,7 @@ int bl_run_graph(bl_handle_t* h, int32_t nsteps, int32_t stop_at_time_end, bl_ti
     set_error("bl_run_graph: mesh maps, regions or EOS not set");
     return BL_FAILURE;
   }
+  if (refresh_outer(h)) return BL_FAILURE;
   // split advection, ALE with neither Eulerian nor relaxation mesh motion, or
   // a mesh without the limiter stencil table: host-driven
   if ((h->cfg.zexist &&

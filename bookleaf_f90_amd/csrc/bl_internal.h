@@ -128,8 +128,14 @@ struct Handle {
   int32_t* d_el_idx = nullptr;
   // limiter stencil of a consistently oriented conforming quad mesh: per
   // element, the far node of each of the 8 neighbour edges the Christensen
-  // limiter reads (null when some element breaks that pattern)
+  // limiter reads (null when some element breaks that pattern).  Made from
+  // ielnd, ielel and ielfc: stale after an upload of the last two, until
+  // refresh_outer
   int32_t* d_outer = nullptr;
+  bool outer_stale = false;
+  // a pointer to ielnd, ielel or ielfc was handed out: stores through it are
+  // not seen here, so the drivers read the connectivity itself
+  bool conn_out = false;
   bool maps_built = false;
   // reductions
   double* d_part = nullptr;  // 4 doubles per workgroup
@@ -282,6 +288,9 @@ int timing_begin(Handle* h, const char* cls);
 void timing_end(Handle* h, int slot);
 // lazily allocated nsz-sized temporaries (bl_ale.hip)
 double* tmp_buffer(Handle* h, int k);
+// d_outer again from the connectivity if the neighbours were uploaded since
+// (bl_api.hip); it allocates, so never inside a capture
+int refresh_outer(Handle* h);
 // geometry_kn_checkvolume's outcome of the geometry queued on the stream
 // (d_dtres->negvol): waits for it, fills err (bl_api.hip)
 int volume_flag(Handle* h, bl_error_t* err);
