@@ -930,6 +930,7 @@ int bl_upload(bl_handle_t* h, int32_t id, const void* host, int64_t count) {
   if (id == BL_IELND || id == BL_IELSORT1 || id == BL_IELSORT2) { h->maps_built = false; invalidate_graph(h); }
   if (id == BL_IELEL || id == BL_IELFC) {
     h->nbfc_stale = h->outer_stale = true;
+    h->ale_tables = false;
     invalidate_graph(h);
   }
   return BL_SUCCESS;

@@ -2902,7 +2902,7 @@ int prepare_tiles(bl_handle_t* h) {
   }
   if (h->tile_state != 1) return BL_SUCCESS;
   // the remap's tables follow the neighbours (ielel, ielfc) too
-  if (ale && (!h->ale_tables || h->nbfc_stale)) {
+  if (ale && !h->ale_tables) {
     if (build_ale_tiles(h)) return BL_FAILURE;
     invalidate_graph(h);
   }

@@ -251,7 +251,9 @@ struct Handle {
   double* cm_other = nullptr;
   double* mesh_w[2] = {};
   double* d_cpe = nullptr;
-  bool ale_tables = false;        // built, or found that the mesh has none (both null)
+  // built (or found that the mesh has none: all null) on the present tiling and
+  // neighbours
+  bool ale_tables = false;
   int ale_home = -1;              // the node set the captured remap steps start from
   // per-step diagnostics of the fused step: region table + Sod L1 records
   bool diag_on = false;

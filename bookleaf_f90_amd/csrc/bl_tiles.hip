@@ -454,7 +454,6 @@ int build_ale_tables(Handle* h) {
   h->d_tile_nbr = nullptr;
   h->d_tile_nbfc = nullptr;
   h->d_tile_ninc = nullptr;
-  h->ale_tables = true;
   const int nel = h->sz.nel, ntile = h->ntile;
   bl_handle_t* hh = static_cast<bl_handle_t*>(h);
   std::vector<int32_t> el(4 * (size_t)nel), fc(4 * (size_t)nel), sort2(nel), pos2(nel);
@@ -540,10 +539,10 @@ int build_ale_tables(Handle* h) {
     }
   };
   each_part(0, npart, some);
-  if (!runs) return BL_SUCCESS;
-  if (upload_vec(&h->d_tile_ninc, ninc) || upload_vec(&h->d_tile_nbfc, nbfc) ||
-      upload_vec(&h->d_tile_nbr, nbr))
+  if (runs && (upload_vec(&h->d_tile_ninc, ninc) || upload_vec(&h->d_tile_nbfc, nbfc) ||
+               upload_vec(&h->d_tile_nbr, nbr)))
     return BL_FAILURE;
+  h->ale_tables = true;
   return BL_SUCCESS;
 }
 

@@ -98,3 +98,20 @@ def test_steps_after_an_upload(eulerian, tiles, oracle_lib):
             assert np.array_equal(a, b)
         assert diff_fields(g.state(), o.state(), compared(p)) == [], k
     assert bool(g.get_tiling()[0]) == tiles
+
+
+def test_tiled_remap_after_an_upload_the_other_form_ran_on(oracle_lib):
+    """The neighbours change while the tiling is off and a run of the other
+    form rebuilds its own table: the tiled remap's tables follow too."""
+    p = _problem(True)
+    print("switched", flush=True)
+    g, o, whole = _pair(p, None)
+    for tiles, tables in ((True, None), (False, _cut(g, p, 0.5)), (True, None), (False, whole),
+                          (True, None)):
+        g.set_tiling(tiles)
+        if tables is not None:
+            _give(g, o, tables)
+        for a, b in zip(g.run(4, runner="run_graph"), o.run(4)):
+            assert np.array_equal(a, b)
+        assert bool(g.get_tiling()[0]) == tiles
+        assert diff_fields(g.state(), o.state(), compared(p)) == []
