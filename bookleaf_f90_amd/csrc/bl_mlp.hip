@@ -32,6 +32,7 @@
 #include <random>
 #include <vector>
 
+#include "bl_grow.h"
 #include "bl_internal.h"
 #include "bl_math.h"
 #include "bl_relax.h"
@@ -1275,15 +1276,15 @@ int bl_mlp_train(bl_mlp_t* m, int32_t iters, int32_t batch, float lr, uint64_t s
   BL_HIP(hipMemcpy(&c, m->count, sizeof(int32_t), hipMemcpyDeviceToHost));
   if (c <= 0) { set_error("bl_mlp_train: no training pairs"); return BL_FAILURE; }
   if (!m->norm_set && mlp_normalize(m)) return BL_FAILURE;
-  if (iters > m->loss_cap) {
-    hipFree(m->loss);
-    m->loss = nullptr;
-    m->loss_cap = 0;
-    if (hipMalloc(&m->loss, sizeof(float) * (size_t)iters) != hipSuccess) {
-      set_error("mlp: out of device memory");
-      return BL_FAILURE;
-    }
-    m->loss_cap = iters;
+  auto take = [](int32_t n) -> float* {
+    float* p = nullptr;
+    if (hipMalloc(&p, sizeof(float) * (size_t)n) == hipSuccess) return p;
+    (void)hipGetLastError();  // (the next launch's check is not to find it)
+    return nullptr;
+  };
+  if (!grow(&m->loss, &m->loss_cap, std::max(iters, 1), take, hipFree)) {
+    set_error("mlp: out of device memory");
+    return BL_FAILURE;
   }
   // the losses stay on the device until the call's end: no host round trip
   // between the steps (a copy of each one took a third of a step)
