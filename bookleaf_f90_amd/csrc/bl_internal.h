@@ -210,7 +210,6 @@ struct Handle {
   int32_t* d_zlist = nullptr;     // nodes that are not relaxed, ascending
   int32_t nzero = 0;
   int32_t* d_lflag = nullptr;     // learned-motion flags and counters
-  int32_t fallback_blocks = 0;    // workgroups of k_learned_fallback, all resident at once
   int32_t* d_lmark = nullptr;     // nnd: node marked by the check for the guard
   int32_t* d_nbfc = nullptr;      // (4, nel) ielel/ielfc packed for the fused remap
   // launch shape of the limiter pass, set by bl_autotune: threads per

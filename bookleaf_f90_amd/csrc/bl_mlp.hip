@@ -34,6 +34,7 @@
 
 #include "bl_grow.h"
 #include "bl_internal.h"
+#include "bl_ordered.h"
 #include "bl_math.h"
 #include "bl_relax.h"
 
@@ -48,8 +49,16 @@ constexpr int kOffW1 = 0, kOffB1 = kOffW1 + kHid * kIn, kOffW2 = kOffB1 + kHid,
 constexpr int kTrainBlock = 64;  // samples per training workgroup
 // learned-motion flags: [0] this step falls back, [1] steps, [2] fallbacks,
 // [3] reasons seen, [4] this step used the guard, [5] guarded steps,
-// [kLBarrier] the arrivals at k_learned_fallback's barriers
-constexpr int kLFlags = 8, kLBarrier = 6;
+// [kLTaken] and [kLDone] the shares of k_learned_fallback taken and done (a
+// cache line each)
+constexpr int kLTaken = 32, kLDone = 64, kLFlags = 96;
+// its workgroups, one per CU of an MI355X: a launch that mostly ends at once
+// costs less with fewer, and a thread takes a few nodes when it runs at all
+constexpr unsigned kFallbackShares = 256;
+// looks at a counter (about a microsecond each) before a workgroup takes a
+// share that no other has started on: all of a launch that has the device
+// have started by then
+constexpr int kPatience = 64;
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -352,7 +361,8 @@ __global__ void __launch_bounds__(256) k_mlp_nodes(MlpPacked W, const float* __r
     if (flag[4]) flag[5] = flag[5] + 1;
     flag[0] = 0;
     flag[4] = 0;
-    flag[kLBarrier] = 0;
+    flag[kLTaken] = 0;
+    flag[kLDone] = 0;
     flag[1] = flag[1] + 1;
   }
   __shared__ MlpShared S;
@@ -488,34 +498,71 @@ __global__ void k_learned_check(int nel, const int32_t* __restrict__ ielnd,
     check_element(e, ielnd, x, y, wu, wv, d1, dt, amax2, relative, stage, mark, flag);
 }
 
-// A barrier of the whole grid, whose workgroups are all resident (the launch
-// is sized for it): count starts the launch at 0, target is the arrivals so
-// far and this barrier's.  Orders what the workgroups exchange at agent scope
-// (relaxed stores, loads and atomics): each thread waits for its own to
-// complete before its workgroup arrives.
-__device__ __forceinline__ void grid_barrier(int32_t* count, int32_t target) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    while (__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target)
-      __builtin_amdgcn_s_sleep(1);
+// The workgroups' part of ordered_phases.  What they exchange is ordered at
+// agent scope (relaxed stores, loads and atomics): each thread waits for its
+// own to complete before its workgroup's share counts as done.
+struct AgentCounter {
+  int32_t* p;
+  __device__ __forceinline__ int add(int n) const {
+    return __hip_atomic_fetch_add(p, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  __syncthreads();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
+  __device__ __forceinline__ int value() const {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ __forceinline__ void pause() const { __builtin_amdgcn_s_sleep(1); }
+};
+// Each of its calls ends in a barrier, after the one thread's branch: a branch
+// of one lane at the end of a loop would meet the one at its start, and the
+// compiler may then send the wave's other lanes round the loop, through its
+// barriers, without that lane (it did: a hang).
+struct Workgroup {
+  ShareCounters<AgentCounter> counters;
+  int32_t *word, *shares;  // in LDS: a value for every thread, the shares held
+  __device__ __forceinline__ int everyones() {
+    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    return __builtin_amdgcn_readfirstlane(*word);
+  }
+  __device__ __forceinline__ void settle() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();  // (and *word is read by all)
+  }
+  __device__ __forceinline__ int take() {
+    if (threadIdx.x == 0) *word = counters.taken.add(1);
+    return everyones();
+  }
+  __device__ __forceinline__ int another(int all) {
+    settle();
+    if (threadIdx.x == 0) *word = counters.another(all);
+    return everyones();
+  }
+  __device__ __forceinline__ void wait(int n, int all) {
+    settle();
+    if (threadIdx.x == 0) counters.wait(n, all);
+    (void)everyones();
+  }
+  // (the same value from every thread)
+  __device__ __forceinline__ void keep(int i, int v) { shares[i] = v; }
+  __device__ __forceinline__ int kept(int i) {
+    return __builtin_amdgcn_readfirstlane(shares[i]);
+  }
+};
 
 // Stage 1 with the guard folded in, and the fallback, in one launch that
-// usually ends at once (stage 0 marked nothing: flag[4] is 0).  Every element
-// is checked again with the guarded velocities, which it forms itself from
-// the marks; after a barrier, when none failed, a relaxed node marked by
-// stage 0 takes one plain sweep's motion instead of the network's proposal.
-// When one failed (flag[0]) the plain relaxation's nsweep sweeps run with a
-// barrier between them; the workgroups exchange positions at agent scope, as
-// each XCD has its own L2.  As launches of their own, gated on the flag, the
-// recheck and eight sweeps cost 38 us a step of doing nothing on the
-// 512x256 problem.
+// usually ends at once (stage 0 marked nothing: flag[4] is 0).  Phase 0 checks
+// every element again with the guarded velocities, which it forms itself from
+// the marks.  When none failed, phase 1 gives a relaxed node marked by stage 0
+// one plain sweep's motion instead of the network's proposal.  When one failed
+// (flag[0]) the phases from 1 on are the plain relaxation's nsweep sweeps; the
+// workgroups exchange positions at agent scope, as each XCD has its own L2.
+// Between the phases bl_ordered.h's waits, which end however many of the
+// workgroups run at once.  On the 512x256 problem with eight sweeps 4.5 us
+// when nothing is marked, 107 us when the step falls back; as launches of
+// their own, gated on the flag, the recheck and the sweeps cost 38 us a step
+// of doing nothing.  (With the shares of every phase taken from a counter, an
+// atomic more per workgroup and phase and the captures in scratch memory, 320
+// us a fallback.)
 __global__ void __launch_bounds__(kBlock)
 k_learned_fallback(int nel, const int32_t* __restrict__ ielnd, const double* x, const double* y,
                    double* wu, double* wv, const float2* __restrict__ d1, double dt, double amax2,
@@ -525,33 +572,46 @@ k_learned_fallback(int nel, const int32_t* __restrict__ ielnd, const double* x, 
   if (ts && (ts->skip || step_bad(ts) || !ts->ale_on)) return;
   if (flag[4] == 0) return;
   if (ts) dt = ts->dt;
-  const int stride = gridDim.x * blockDim.x;
-  int32_t* count = flag + kLBarrier;
-  int32_t target = (int32_t)gridDim.x;
-  for (int e = xcd_index(); e < nel; e += stride)
-    check_element(e, ielnd, x, y, wu, wv, d1, dt, amax2, relative, 1, mark, flag, true);
-  grid_barrier(count, target);
-  if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
-    for (int i = xcd_index(); i < nr; i += stride) {
-      const int n = rlist[i];
-      if (!mark[n]) continue;
-      const float2 d = d1[n];
-      wu[n] = (double)d.x / dt;
-      wv[n] = (double)d.y / dt;
+  __shared__ int32_t word, held[kFallbackShares];
+  Workgroup group{{{flag + kLTaken}, {flag + kLDone}, kPatience}, &word, held};
+  const int shares = (int)gridDim.x, stride = shares * kBlock;
+  bool sweeps = false;
+  // (inlined: called otherwise, each has what it captures in scratch memory)
+  auto recheck = [&](int share) __attribute__((always_inline)) {
+    for (int e = share * kBlock + (int)threadIdx.x; e < nel; e += stride)
+      check_element(e, ielnd, x, y, wu, wv, d1, dt, amax2, relative, 1, mark, flag, true);
+  };
+  auto phases = [&]() __attribute__((always_inline)) {
+    sweeps = __builtin_amdgcn_readfirstlane(__hip_atomic_load(
+                 flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
+    return sweeps ? nsweep : 1;
+  };
+  auto move = [&](int phase, int share) __attribute__((always_inline)) {
+    const int i0 = share * kBlock + (int)threadIdx.x;
+    if (!sweeps) {
+      for (int i = i0; i < nr; i += stride) {
+        const int n = rlist[i];
+        if (!mark[n]) continue;
+        const float2 d = d1[n];
+        wu[n] = (double)d.x / dt;
+        wv[n] = (double)d.y / dt;
+      }
+      return;
     }
-    return;
-  }
-  for (int k = 0; k < nsweep; ++k) {
-    const bool last = k + 1 == nsweep;
-    const double* xi = k == 0 ? x : (k & 1) ? t0x : t1x;
-    const double* yi = k == 0 ? y : (k & 1) ? t0y : t1y;
-    double* xo = (k & 1) ? t1x : t0x;
-    double* yo = (k & 1) ? t1y : t0y;
-    for (int n = xcd_index(); n < R.nnd; n += stride) {
+    const int k = phase - 1;
+    // (a choice between the captured variables themselves would keep them in
+    // scratch memory)
+    double *const ax = t0x, *const ay = t0y, *const bx = t1x, *const by = t1y;
+    const bool odd = (k & 1) != 0;
+    double* const xo = odd ? bx : ax;
+    double* const yo = odd ? by : ay;
+    const double* const xi = k == 0 ? x : odd ? ax : bx;
+    const double* const yi = k == 0 ? y : odd ? ay : by;
+    for (int n = i0; n < R.nnd; n += stride) {
       double a, b;
       if (k == 0) relax_node(R, n, xi, yi, a, b);
       else relax_node(R, n, xi, yi, a, b, AgentLoad());
-      if (last) {
+      if (phase == nsweep) {
         wu[n] = (a - x[n]) / dt;
         wv[n] = (b - y[n]) / dt;
       } else {
@@ -559,9 +619,8 @@ k_learned_fallback(int nel, const int32_t* __restrict__ ielnd, const double* x, 
         __hip_atomic_store(yo + n, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
-    target += (int32_t)gridDim.x;
-    if (!last) grid_barrier(count, target);
-  }
+  };
+  ordered_phases(group, shares, recheck, phases, move);
 }
 
 // per-column mean and standard deviation of the stored pairs (FP64 sums in
@@ -1055,7 +1114,7 @@ int learned_velocity(Handle* hh, const double* x, const double* y, double* wu, d
   const bl_mlp* m = h->mlp_infer;
   const int nel = h->sz.nel, nr = h->nrelaxed, nz = h->nzero;
   if (!m || !h->d_ring || !h->d_rlist || !h->d_zlist || !h->d_lflag || !h->d_lmark ||
-      !h->d_ld1 || !h->relax_tmp[0] || h->fallback_blocks < 1) {
+      !h->d_ld1 || !h->relax_tmp[0]) {
     set_error("learned relaxation: not set up (bl_relax_learned)");
     return BL_FAILURE;
   }
@@ -1076,7 +1135,8 @@ int learned_velocity(Handle* hh, const double* x, const double* y, double* wu, d
             h->d_lflag, ts);
   // the guard, and the plain relaxation when the check failed
   double* const* t = h->relax_tmp;
-  BL_LAUNCH(h, "learned_fallback", k_learned_fallback, (unsigned)h->fallback_blocks, kBlock, nel,
+  const unsigned shares = std::min(nblocks(std::max(nel, h->sz.nnd)), kFallbackShares);
+  BL_LAUNCH(h, "learned_fallback", k_learned_fallback, shares, kBlock, nel,
             (const int32_t*)h->I(BL_IELND), x, y, wu, wv, (const float2*)h->d_ld1, dt, amax2,
             h->learned_relative, (const int32_t*)h->d_rlist, nr, h->d_lmark, h->d_lflag,
             relax_args(h), h->relax_nsweep, t[0], t[1], t[2], t[3], ts);
@@ -1339,18 +1399,6 @@ int bl_relax_learned(bl_handle_t* h, bl_mlp_t* m) {
   if (m && !h->d_lmark)
     BL_HIP(hipMalloc(&h->d_lmark, sizeof(int32_t) * std::max(h->sz.nnd, 1)));
   if (m && !h->d_ld1) BL_HIP(hipMalloc(&h->d_ld1, sizeof(float) * 2 * std::max(h->sz.nnd, 1)));
-  if (m && h->fallback_blocks < 1) {
-    // as many workgroups as the device holds at once, at most one per CU of
-    // an MI355X (a thread takes a few nodes when it runs at all)
-    int per_cu = 0, cus = 0;
-    BL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_learned_fallback, kBlock, 0));
-    BL_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device));
-    h->fallback_blocks = std::min(256, per_cu * cus);
-    if (h->fallback_blocks < 1) {
-      set_error("bl_relax_learned: the fallback kernel does not fit the device");
-      return BL_FAILURE;
-    }
-  }
   // the counters start again with every network attached
   if (m) BL_HIP(hipMemset(h->d_lflag, 0, sizeof(int32_t) * kLFlags));
   return BL_SUCCESS;

@@ -227,6 +227,42 @@ def test_fallback_is_the_plain_relaxation_bitexact(runner, oracle_lib):
     assert diff_fields(g.state(), o.state(), names, ncp=p.ncp or None) == []
 
 
+def test_fallbacks_of_several_handles_at_once(oracle_lib):
+    """Handles that fall back at every step, each on a stream and a thread of
+    its own: every launch takes its phases through whatever share of the
+    device it gets.  A mesh of more nodes than one round of the launch's
+    workgroups, several sweeps: each handle ends where the plain relaxation
+    does."""
+    import threading
+
+    from bookleaf_f90_amd.device import BookLeaf
+    p = _relaxed(420, 180, nsweep=5, om=0.25, nsteps=6)
+    print("fallbacks at once", p.nnd, flush=True)
+    plain = BookLeaf(p)
+    plain.run(1, runner="run_graph")
+    want = plain.run(6, runner="run_graph")
+    handles = [BookLeaf(p) for _ in range(3)]
+    nets = [_far_net() for _ in handles]
+    got = [None] * len(handles)
+
+    def run(k):
+        got[k] = handles[k].run(6, runner="run_graph")
+
+    for g, net in zip(handles, nets):
+        g.relax_learned(net)
+        g.run(1, runner="run_graph")  # the tables and graphs, one handle at a time
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(len(handles))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for g, h in zip(handles, got):
+        for a, b in zip(h, want):
+            assert np.array_equal(a, b)
+        assert g.learned_stats() == (7, 7)
+        assert diff_fields(g.state(), plain.state(), compared(p)) == []
+
+
 def test_learned_motion_is_applied(oracle_lib):
     """A network adding +0.01 h in x to one sweep everywhere: after one ALE
     step every relaxed node sits h (f24 + 0.01, f25) from its Lagrangian
