@@ -2572,17 +2572,24 @@ void tile_args(bl_handle_t* h, FusedArgs& A, int p, int s) {
   A.end_in_f1b = 1;
 }
 
+// the limiter pass's workgroups on a tiling, with the launch shape `grid`: one
+// per 64 elements at least (a small mesh's elements in motion then spread over
+// the chip), kLimParts at most; a shape of a workgroup per 256 elements, the
+// most of the three-kernel step, or more is no limit
+int tile_limiter_grid(const bl_handle_t* h, int grid) {
+  const int most = std::min((int)nblocks(h->sz.nel, 64), kLimParts);
+  return std::max(1, grid >= (int)nblocks(h->sz.nel) ? most : std::min(grid, most));
+}
+
 // a step on a tiling of parity p: its states, and the limiter pass's
-// workgroups (one per 64 elements at least: a small mesh's elements in motion
-// then spread over the chip)
+// workgroups
 void select_args(bl_handle_t* h, FusedArgs& A, int p) {
   A.before = h->d_state + p;
   A.mid = &h->d_state[2].ts;
   A.ts = &h->d_state[1 - p].ts;
   A.dtres = &h->d_state[1 - p].res;
   A.lim = static_cast<LimPart*>(h->d_lim);
-  A.nlim = std::max(1, std::min((int)nblocks(h->sz.nel, 64),
-                                std::min(h->tune_lim_grid, kLimParts)));
+  A.nlim = tile_limiter_grid(h, h->tune_lim_grid);
 }
 
 // The tilings whose tiles select dt themselves: at most two rounds of
@@ -3329,13 +3336,21 @@ int bl_ensemble_run(bl_handle_t* h, int32_t nsteps, double* dt_hist, int32_t* id
   }
 }
 
+// the launch shape as bl_autotune and bl_get_tuning report it: no more than a
+// workgroup per 256 elements, nor than a tiling's limiter pass takes
+int reported_grid(const bl_handle_t* h, int grid) {
+  const int g = std::min((int)nblocks(h->sz.nel), grid);
+  return use_tiles(h) || ale_tiles(h) ? std::min(g, kLimParts) : g;
+}
+
 // The launch-shape autotuner: times the limiter pass (F1L, or E1L for an
 // ensemble) of the current state under each candidate shape -- threads per
-// workgroup 64/128/256 and workgroups 128..2048 (single problem) or
-// elements per workgroup and instance 1024..16384 (ensemble) -- and keeps
-// the fastest.  Each trial runs the viscosity pass (F1/E1) that writes the
-// at-rest mask (an ensemble's worklists), then the limiter pass between two
-// events; neither touches the state a step carries over (the viscosity
+// workgroup 64/128/256 and workgroups 128..2048 (the three-kernel step),
+// 32..512 (a step on a tiling) or elements per workgroup and instance
+// 1024..16384 (ensemble) -- and keeps the fastest.  Each trial runs the
+// viscosity pass (F1/E1) that writes the at-rest mask (a tiling's bytes, an
+// ensemble's worklists), then the limiter pass of the handle's next run
+// between two events; neither touches the state a step carries over (the viscosity
 // fields they write are saved and restored, the masks and worklist counters
 // reset).  The choice changes no result: the limiter's CFL selection is a
 // first-index minimum whatever the split.
@@ -3351,19 +3366,23 @@ int bl_autotune(bl_handle_t* h, int32_t reps, bl_tuning_t* out) {
     set_error("bl_autotune: mesh maps, regions or EOS not set");
     return BL_FAILURE;
   }
-  if (ensure_nodesets(h)) return BL_FAILURE;
+  if (ensure_nodesets(h) || (!ens && prepare_tiles(h))) return BL_FAILURE;
+  const bool ale = ale_tiles(h), tiled = !ens && (use_tiles(h) || ale);
+  if (tiled && ensure_step_buffers(h)) return BL_FAILURE;
   // the device timestep as the last run left it (done set after an error or
   // time_end), put back at the end; the trials run with done and skip clear,
   // as the next run starts
-  DevTimestep ts_saved, ts_trial;
-  BL_HIP(hipMemcpyAsync(&ts_saved, h->d_ts, sizeof(DevTimestep), hipMemcpyDeviceToHost,
-                        h->stream));
+  const int p0 = ale ? 0 : h->cur_set;  // the next run's first parity
+  StepState saved[3], trial;
+  BL_HIP(hipMemcpyAsync(saved, h->d_state, sizeof(saved), hipMemcpyDeviceToHost, h->stream));
   BL_HIP(hipStreamSynchronize(h->stream));
-  ts_trial = ts_saved;
-  ts_trial.done = 0;
-  ts_trial.skip = 0;
-  BL_HIP(hipMemcpyAsync(h->d_ts, &ts_trial, sizeof(DevTimestep), hipMemcpyHostToDevice,
-                        h->stream));
+  trial.ts = saved[0].ts;
+  trial.ts.done = 0;
+  trial.ts.skip = 0;
+  trial.ts.open = 0;
+  trial.res = DtResult{};
+  BL_HIP(hipMemcpyAsync(h->d_state + (tiled ? p0 : 0), &trial, sizeof(trial),
+                        hipMemcpyHostToDevice, h->stream));
   const int nel = h->sz.nel;
   const unsigned nbe = nblocks(nel);
   // save the viscosity outputs the trials overwrite
@@ -3379,6 +3398,15 @@ int bl_autotune(bl_handle_t* h, int32_t reps, bl_tuning_t* out) {
   const int p = h->cur_set;
   FusedNodes N{h->nodeset[p][0], h->nodeset[p][1], h->nodeset[p][2], h->nodeset[p][3]};
   EnsArgs E{};
+  if (tiled) {
+    tile_args(h, A, p0, p);
+    select_args(h, A, p0);
+  }
+  FusedArgs first = A;  // of the first viscosity pass of a run on the tiling
+  if (tiled) {
+    first.rest8_next = h->d_rest8 + (size_t)p0 * h->sz.nel;
+    first.ts = &h->d_state[p0].ts;
+  }
   if (ens) {
     A.einst = h->d_einst;
     A.ninst = h->d_ninst;
@@ -3393,7 +3421,7 @@ int bl_autotune(bl_handle_t* h, int32_t reps, bl_tuning_t* out) {
   BL_HIP(hipEventCreate(&e0));
   BL_HIP(hipEventCreate(&e1));
   const int blocks[3] = {64, 128, 256};
-  const int grids[5] = {128, 256, 512, 1024, 2048};
+  const int grids[5] = {128, 256, 512, 1024, 2048}, tile_grids[5] = {32, 64, 128, 256, kLimParts};
   const int chunks[5] = {1024, 2048, 4096, 8192, 16384};
   const int def_block = h->tune_lim_block, def_second = ens ? h->tune_ens_chunk : h->tune_lim_grid;
   double tcur[15], tfull[15];
@@ -3401,16 +3429,19 @@ int bl_autotune(bl_handle_t* h, int32_t reps, bl_tuning_t* out) {
   int rc = BL_SUCCESS;
   for (int b = 0; b < 3 && rc == BL_SUCCESS; ++b)
     for (int g = 0; g < 5 && rc == BL_SUCCESS; ++g) {
-      const int block = blocks[b], second = ens ? chunks[g] : grids[g];
+      const int block = blocks[b], second = ens ? chunks[g] : tiled ? tile_grids[g] : grids[g];
+      if (tiled) A.nlim = tile_limiter_grid(h, second);
       if (ens && ens_set_chunk(h, second)) { rc = BL_FAILURE; break; }
       if (ens) E = make_ens(h);
       // pass 0: the elements in motion in the current state; pass 1: every
       // element in motion (the flow spread everywhere)
       for (int pass = 0; pass < 2 && rc == BL_SUCCESS; ++pass) {
         std::vector<float> t;
-        // every element in motion: the single problem's mask all zero, an
-        // ensemble's worklist every element (and its counts below)
-        if (pass == 1 && !ens)
+        // every element in motion: the single problem's mask or bytes all
+        // zero, an ensemble's worklist every element (and its counts below)
+        if (pass == 1 && tiled)
+          hipMemsetAsync(first.rest8_next, 0, (size_t)nel, h->stream);
+        else if (pass == 1 && !ens)
           hipMemsetAsync(h->d_rest, 0, sizeof(uint64_t) * 4 * (size_t)nbe, h->stream);
         if (pass == 1 && ens)
           hipLaunchKernelGGL(k_work_all, dim3(nbe), dim3(kBlock), 0, h->stream, h->d_work, nel);
@@ -3420,6 +3451,9 @@ int bl_autotune(bl_handle_t* h, int32_t reps, bl_tuning_t* out) {
             if (ens) hipMemsetAsync(cnt, 0, sizeof(uint32_t) * full.size(), h->stream);
             if (ens)
               hipLaunchKernelGGL(k_e1_getdt, dim3(nbe), dim3(kBlock), 0, h->stream, A, N, E);
+            else if (tiled)
+              hipLaunchKernelGGL(k_f1_seg, dim3(h->ntile), dim3(kBlock), 0, h->stream, first, N,
+                                 EnsArgs{});
             else
               hipLaunchKernelGGL(k_f1_getdt, dim3(nbe), dim3(kBlock), 0, h->stream, A, N);
           } else if (ens) {
@@ -3430,6 +3464,9 @@ int bl_autotune(bl_handle_t* h, int32_t reps, bl_tuning_t* out) {
           if (ens)
             hipLaunchKernelGGL(k_e1_limiter, dim3(h->ens_lblocks), dim3(block), 0, h->stream, A,
                                N, E);
+          else if (tiled)
+            hipLaunchKernelGGL(k_f1_limiter<true>, dim3(A.nlim), dim3(block), 0, h->stream, A, N,
+                               A.nseg);
           else
             hipLaunchKernelGGL(k_f1_limiter<false>, dim3(std::min(nbe, (unsigned)second)), dim3(block),
                                0, h->stream, A, N, (int)nbe);
@@ -3456,8 +3493,8 @@ int bl_autotune(bl_handle_t* h, int32_t reps, bl_tuning_t* out) {
   hipMemcpyAsync(h->R(BL_CNVISCY), save + 4 * (size_t)nel, c4, hipMemcpyDeviceToDevice, h->stream);
   hipMemcpyAsync(h->R(BL_ELVISC), save + 8 * (size_t)nel, c1, hipMemcpyDeviceToDevice, h->stream);
   if (ens) hipMemsetAsync(h->d_cnt, 0, sizeof(uint32_t) * h->ens_n, h->stream);
-  hipMemcpyAsync(h->d_ts, &ts_saved, sizeof(DevTimestep), hipMemcpyHostToDevice, h->stream);
   clear_rest(h);
+  hipMemcpyAsync(h->d_state, saved, sizeof(saved), hipMemcpyHostToDevice, h->stream);
   hipStreamSynchronize(h->stream);
   hipFree(save);
   hipEventDestroy(e0);
@@ -3475,7 +3512,9 @@ int bl_autotune(bl_handle_t* h, int32_t reps, bl_tuning_t* out) {
   for (int k = 0; k < trials; ++k) {
     const double sk = std::max(tcur[k] / bc, tfull[k] / bf);
     if (sk < score) { score = sk; pick = k; }
-    if (cblock[k] == def_block && csecond[k] == def_second) idef = k;
+    const bool same = tiled ? tile_limiter_grid(h, csecond[k]) == tile_limiter_grid(h, def_second)
+                            : csecond[k] == def_second;
+    if (cblock[k] == def_block && same) idef = k;
   }
   h->tune_lim_block = cblock[pick];
   if (ens) {
@@ -3486,8 +3525,7 @@ int bl_autotune(bl_handle_t* h, int32_t reps, bl_tuning_t* out) {
   invalidate_graph(h);
   if (out) {
     out->limiter_block = cblock[pick];
-    out->limiter_grid = ens ? (int32_t)h->ens_lblocks
-                            : (int32_t)std::min(nbe, (unsigned)csecond[pick]);
+    out->limiter_grid = ens ? (int32_t)h->ens_lblocks : reported_grid(h, csecond[pick]);
     out->ens_chunk = ens ? csecond[pick] : 0;
     out->trials = trials;
     out->best_us = tcur[pick];
@@ -3574,8 +3612,7 @@ int bl_get_tuning(bl_handle_t* h, bl_tuning_t* t) {
   }
   const bool ens = h->ens_n > 0;
   t->limiter_block = h->tune_lim_block;
-  t->limiter_grid = ens ? (int32_t)h->ens_lblocks
-                        : (int32_t)std::min(nblocks(h->sz.nel), (unsigned)h->tune_lim_grid);
+  t->limiter_grid = ens ? (int32_t)h->ens_lblocks : reported_grid(h, h->tune_lim_grid);
   t->ens_chunk = ens ? h->tune_ens_chunk : 0;
   t->trials = 0;
   t->best_us = 0.0;

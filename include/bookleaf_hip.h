@@ -455,8 +455,9 @@ int bl_run_stats(bl_handle_t* h, int64_t* moving, int64_t* zeroed);
  * no launch shape).  Times the limiter pass -- the viscosity and CFL of the
  * elements with moving nodes, the step's one worklist-driven kernel -- under
  * 15 shapes: 64, 128 or 256 threads per workgroup times 128..2048
- * workgroups (a single problem) or 1024..16384 elements per workgroup and
- * instance (an ensemble).  Each shape is timed twice, on the worklist of the
+ * workgroups (the three-kernel step), 32..512 (a step on a tiling) or
+ * 1024..16384 elements per workgroup and instance (an ensemble): the kernel
+ * and the shapes of the handle's next run.  Each shape is timed twice, on the worklist of the
  * handle's current state and with every element listed (the worklist as the
  * flow spreads), each the median of reps launches after one warm-up; the
  * shape kept for every later step is the one whose worse ratio to the best
@@ -469,7 +470,8 @@ int bl_run_stats(bl_handle_t* h, int64_t* moving, int64_t* zeroed);
  * number of shapes timed, and the chosen and the default shape's times. */
 typedef struct {
   int32_t limiter_block; /* threads per workgroup */
-  int32_t limiter_grid;  /* workgroups launched */
+  int32_t limiter_grid;  /* most workgroups, as reported no more than one per 256 elements
+                          * (an ensemble: workgroups launched) */
   int32_t ens_chunk;     /* ensemble: most elements per workgroup and instance; 0 otherwise */
   int32_t trials;        /* shapes timed */
   double best_us;        /* median duration of the chosen shape, current worklist */
@@ -483,8 +485,11 @@ int bl_autotune(bl_handle_t* h, int32_t reps, bl_tuning_t* out);
  * limiter_grid (>= 1, a single problem) or ens_chunk (>= 64, an ensemble);
  * the other fields are ignored.  No result depends on it. */
 int bl_set_tuning(bl_handle_t* h, const bl_tuning_t* t);
-/* the shape in use: limiter_grid is the number of workgroups launched;
- * trials and the four times are zero */
+/* the shape in use.  limiter_grid: the three-kernel step launches that many
+ * workgroups; a step on a tiling (which the handle is known to take once it
+ * has run) at most that many and never more than 512, or, where it is one per
+ * 256 elements and so no limit, one per 64.  trials and the four times are
+ * zero */
 int bl_get_tuning(bl_handle_t* h, bl_tuning_t* t);
 
 /* The tile step (no counterpart in the reference, which has no kernels to

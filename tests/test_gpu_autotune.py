@@ -134,3 +134,31 @@ def test_autotune_after_time_end_and_errors():
     assert g.get_tuning() == shape
     with pytest.raises(BookLeafError):
         g.autotune(reps=0)
+
+
+def test_reported_shapes_are_those_of_the_next_run(oracle_lib):
+    """A mesh of more blocks than a tiling's limiter pass takes workgroups:
+    the shape reported and the shapes tuned are the three-kernel step's without
+    the tiling, the tile step's on it; nothing depends on them."""
+    from bookleaf_f90_amd.device import BookLeaf
+    p = P.sedov(n=400, nsteps=6, kappa=0.01)
+    blocks = -(-p.nel // 256)
+    print("reported", p.nel, blocks, flush=True)
+    g, other = BookLeaf(p), BookLeaf(p)
+    g.set_tuning(limiter_block=128, limiter_grid=2048)
+    assert g.get_tuning()["limiter_grid"] == blocks
+    g.run(2, runner="run_graph")
+    assert g.get_tiling()[0] and g.get_tuning()["limiter_grid"] == 512
+    t = g.autotune(reps=1)
+    assert t["limiter_grid"] in (32, 64, 128, 256, 512)
+    assert g.get_tuning()["limiter_grid"] == t["limiter_grid"]
+    g.set_tiling(False)
+    t = g.autotune(reps=1)
+    assert t["limiter_grid"] in (128, 256, 512, blocks)
+    g.run(2, runner="run_graph")
+    g.set_tuning(limiter_block=256, limiter_grid=100)
+    g.set_tiling(True)
+    assert g.get_tuning()["limiter_grid"] == 100
+    g.run(2, runner="run_graph")
+    other.run(6, runner="run_graph")
+    assert diff_fields(g.state(), other.state(), compared(p)) == []
