@@ -189,13 +189,13 @@ namespace bl {
 
 // the limiter pass's workgroups per instance, ceil(nel_k / piece), their
 // offsets lboff on the device, and room for their partials.  A workgroup's
-// piece is the chunk, halved while the launch would have fewer than
-// kEnsWorkgroups workgroups (two rounds of the 512 that are resident at
-// two waves a SIMD) and a lane its own element at least: the limiter of an
-// element is one long chain, and a piece runs its elements one round after
-// another.  Step of an ensemble at a piece of 256 / 1024 / 4096: 8 instances
-// of 32^2..64^2 36 / 45 / 83 us, 48 of 64^2..256^2 215 / 205 / 235, 96 of
-// 64^2..512^2 1088 / 986 / 1008.
+// piece is the chunk, if one was chosen; the default's is halved while the
+// launch would have fewer than kEnsWorkgroups workgroups (two rounds of the
+// 512 that are resident at two waves a SIMD) and a lane its own element at
+// least: the limiter of an element is one long chain, and a piece runs its
+// elements one round after another.  Step of an ensemble at a piece of 256 /
+// 1024 / 4096: 8 instances of 32^2..64^2 36 / 45 / 83 us, 48 of 64^2..256^2
+// 215 / 205 / 235, 96 of 64^2..512^2 1088 / 986 / 1008.
 int ens_set_chunk(Handle* hh, int chunk) {
   bl_handle_t* h = static_cast<bl_handle_t*>(hh);
   const int ninst = h->ens_n;
@@ -205,7 +205,8 @@ int ens_set_chunk(Handle* hh, int chunk) {
   }
   constexpr long long kEnsWorkgroups = 1024;
   int piece = chunk;
-  while (piece / 2 >= kBlock && h->sz.nel < kEnsWorkgroups * piece) piece /= 2;
+  if (chunk == kEnsChunk)
+    while (piece / 2 >= kBlock && h->sz.nel < kEnsWorkgroups * piece) piece /= 2;
   std::vector<int32_t> lboff(ninst + 1, 0);
   for (int k = 0; k < ninst; ++k)
     lboff[k + 1] = lboff[k] + (h->ens_eoff[k + 1] - h->ens_eoff[k] + piece - 1) / piece;

@@ -11,6 +11,8 @@
 namespace bl {
 
 constexpr int kBlock = 256;  // 4 wave64 per workgroup
+// elements per limiter workgroup and instance of an ensemble, unless tuned
+constexpr int kEnsChunk = 4096;
 void set_error(const std::string& msg);
 
 #define BL_HIP(call)                                                              \
@@ -215,7 +217,7 @@ struct Handle {
   // launch shape of the limiter pass, set by bl_autotune: threads per
   // workgroup, workgroups (single problem), elements per workgroup and
   // instance (ensembles)
-  int32_t tune_lim_block = 256, tune_lim_grid = 512, tune_ens_chunk = 4096;
+  int32_t tune_lim_block = 256, tune_lim_grid = 512, tune_ens_chunk = kEnsChunk;
   int32_t ens_lblocks_cap = 0;    // limiter partial slots allocated
   bool nbfc_stale = true;         // rebuild it before the next capture
   // the tile step of a pure-cell Lagrangian problem (bl_tiles.hip): the

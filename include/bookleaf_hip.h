@@ -472,7 +472,7 @@ typedef struct {
   int32_t limiter_block; /* threads per workgroup */
   int32_t limiter_grid;  /* most workgroups, as reported no more than one per 256 elements
                           * (an ensemble: workgroups launched) */
-  int32_t ens_chunk;     /* ensemble: most elements per workgroup and instance; 0 otherwise */
+  int32_t ens_chunk;     /* ensemble: elements per workgroup and instance; 0 otherwise */
   int32_t trials;        /* shapes timed */
   double best_us;        /* median duration of the chosen shape, current worklist */
   double default_us;     /* the same for the shape in use before the call */
@@ -483,7 +483,10 @@ int bl_autotune(bl_handle_t* h, int32_t reps, bl_tuning_t* out);
 /* Apply a launch shape without timing (one bl_autotune chose for the same
  * problem before, say): limiter_block (a multiple of 64 up to 256) and
  * limiter_grid (>= 1, a single problem) or ens_chunk (>= 64, an ensemble);
- * the other fields are ignored.  No result depends on it. */
+ * the other fields are ignored.  ens_chunk 4096 is the default and leaves the
+ * split to the ensemble's size (4096 elements, halved while that makes fewer
+ * than 1024 workgroups); any other is taken as it is.  No result depends on
+ * it. */
 int bl_set_tuning(bl_handle_t* h, const bl_tuning_t* t);
 /* the shape in use.  limiter_grid: the three-kernel step launches that many
  * workgroups; a step on a tiling (which the handle is known to take once it

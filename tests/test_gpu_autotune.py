@@ -162,3 +162,25 @@ def test_reported_shapes_are_those_of_the_next_run(oracle_lib):
     g.run(2, runner="run_graph")
     other.run(6, runner="run_graph")
     assert diff_fields(g.state(), other.state(), compared(p)) == []
+
+
+def test_a_chosen_chunk_is_taken_as_it_is():
+    from bookleaf_f90_amd.device import Ensemble
+    params = P.ensemble_params(4, seed=3, nmin=30, nmax=60)
+    sizes = [q["nx"] * q["ny"] for q in params]
+    print("chunks", sizes, flush=True)
+    ens = Ensemble(params)
+
+    def grid(chunk):
+        return sum(-(-n // chunk) for n in sizes)
+
+    assert ens.get_tuning()["limiter_grid"] == grid(256)  # the default, halved
+    for chunk in (300, 1024, 2048, 8192, 16384):
+        ens.set_tuning(ens_chunk=chunk)
+        t = ens.get_tuning()
+        assert (t["ens_chunk"], t["limiter_grid"]) == (chunk, grid(chunk))
+    ens.set_tuning()
+    assert ens.get_tuning()["limiter_grid"] == grid(256)
+    # the five chunks tuned are five launches
+    assert len({grid(c) for c in (1024, 2048, 256, 8192)}) >= 3
+    ens.close()
