@@ -133,3 +133,140 @@ def test_negative_volume_stops_both_forms_alike(where):
     names = ["ndx", "ndy", "ndu", "ndv", "eldensity", "elenergy", "elpressure", "elcs2",
              "elmass", "cnmass", "cnviscx", "cnviscy", "elvisc"]
     assert diff_fields(seen[0][3], seen[1][3], names) == []
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_summation_orders_of_the_sorted_elements(mixed, oracle_lib):
+    """ielsort1 and ielsort2 two permutations: a node's remap sums run in the
+    order of ielsort2, then in element order, and the two differ."""
+    from bookleaf_f90_amd.device import BookLeaf
+    from oracle.pyoracle import Oracle
+    p = _stirred((P.sod2mat_mixed if mixed else P.sod2mat)(nx=33, ny=18), u=0.05)
+    if not mixed:  # (the components' lists name elements)
+        p = _renumbered(p, 7, 1)
+    print("sorted", p.nel, mixed, flush=True)
+    rng = np.random.default_rng(8)
+    sorts = {k: (rng.permutation(p.nel) + 1).astype(np.int32) for k in ("ielsort1", "ielsort2")}
+    tiled, other, o, plain = BookLeaf(p), BookLeaf(p), Oracle(p), Oracle(p)
+    other.set_tiling(False)
+    for s in (tiled, other, o):
+        for k, v in sorts.items():
+            s.set(k, v)
+    for s in (tiled, other):
+        assert s.lib.bl_build_maps(s.h) == 0
+    for n in (3, 6):
+        ho = o.run(n)
+        for s in (tiled, other):
+            for x, y in zip(s.run(n, runner="run_graph"), ho):
+                assert np.array_equal(x, y)
+            assert diff_fields(s.state(), o.state(), compared(p)) == []
+    assert tiled.get_tiling()[0] and not other.get_tiling()[0]
+    plain.run(9)
+    assert not np.array_equal(plain.get("ndu"), o.get("ndu"))  # the order shows
+
+
+@pytest.mark.parametrize("kind", ["boundary_face", "wrapped"])
+def test_meshes_the_tiled_remap_refuses(kind, oracle_lib):
+    """A boundary face whose ielfc is not the opposite face: the remap's grid
+    form runs.  Neighbours across the ends of the tube, which share no nodes
+    (outside a tile's entries): the drivers run.  Both match the oracle."""
+    from bookleaf_f90_amd.device import BookLeaf
+    from oracle.pyoracle import Oracle
+    nx, ny = 24, 9
+    p = _stirred(P.sod(nx=nx, ny=ny, height=0.4, eulerian=True, dt_initial=1e-3))
+    print("refused", kind, flush=True)
+    g, o = BookLeaf(p), Oracle(p)
+    g.run(2, runner="run_graph")
+    o.run(2)
+    assert g.get_tiling()[0]
+    el, fc = g.get("ielel"), g.get("ielfc")
+    x = g.get("ndx")[p.ielnd.reshape(-1, 4) - 1].mean(axis=1)
+    y = g.get("ndy")[p.ielnd.reshape(-1, 4) - 1].mean(axis=1)
+    own = np.arange(p.nel).repeat(4) + 1 == el[:4 * p.nel]
+    if kind == "boundary_face":
+        k = np.nonzero(own)[0][7]
+        fc[k] = k % 4 + 1
+    else:
+        rows = np.argsort(y, kind="stable").reshape(ny, nx)
+        for row in rows:
+            a, b = row[np.argmin(x[row])], row[np.argmax(x[row])]
+            # the boundary face towards the end of the tube: opposite the
+            # neighbour inside the row
+            f = [i for i in range(4) if el[4 * a + i] == a + 1 and
+                 el[4 * a + (i + 2) % 4] - 1 in row and el[4 * a + (i + 2) % 4] != a + 1][0]
+            h = [i for i in range(4) if el[4 * b + i] == b + 1 and
+                 el[4 * b + (i + 2) % 4] - 1 in row and el[4 * b + (i + 2) % 4] != b + 1][0]
+            el[4 * a + f], fc[4 * a + f] = b + 1, h + 1
+            el[4 * b + h], fc[4 * b + h] = a + 1, f + 1
+    for s in (g, o):
+        s.set("ielel", el)
+        s.set("ielfc", fc)
+    for n in (3, 4):
+        for a, b in zip(g.run(n, runner="run_graph"), o.run(n)):
+            assert np.array_equal(a, b)
+        assert diff_fields(g.state(), o.state(), compared(p)) == []
+    if kind == "boundary_face":
+        assert not g.get_tiling()[0]
+
+
+STAGES = ("predictor", "corrector", "remap")
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("stage", STAGES)
+def test_negative_volume_of_each_stage(stage, mixed, oracle_lib):
+    """A volume negative at the half step, at the full step (a node carried two
+    and a half cells, one at the half step) or after the moved mesh: both
+    forms stop there alike, with the oracle's error, and the fields show the
+    stage: nodes not moved, nodes moved and no mass advected, mass advected.
+    Component energies are the reference's: before the predictor, after it,
+    after the corrector."""
+    from bookleaf_f90_amd.device import BookLeaf, BookLeafError
+    from oracle.pyoracle import Oracle
+    nx, ny = 24, 9
+    make = P.sod2mat_mixed if mixed else P.sod2mat
+    p = make(nx=nx, ny=ny, eulerian=stage != "remap", dt_initial=1.0e-3)
+    inner = np.nonzero(p.indtype > 0)[0]
+    width = (p.ndx.max() - p.ndx.min()) / nx
+    if stage == "remap":
+        p = P.with_relaxation(p, abi.RELAX_LIN1, nsweep=1, om=3.0)
+        rng = np.random.default_rng(1)
+        p.ndx[inner] += rng.uniform(-0.4, 0.4, inner.size) * width
+    else:
+        # a node of the column at the interface (the mixed cells')
+        xm = 0.5 * (p.ndx.max() + p.ndx.min())
+        n = inner[np.argmin(np.abs(p.ndx[inner] - xm) + 1e-6 * np.abs(p.ndy[inner] - 0.5))]
+        cells = {"predictor": 100.0, "corrector": 2.5}[stage]
+        p.ndu[n] = cells * width / 1.0e-3
+    p.config.update(cvisc1=0.0, cvisc2=0.0, div_sf=1.0e30, dt_max=1.0e-3, cfl_sf=1.0e10)
+    print("stage", stage, mixed, flush=True)
+    o = Oracle(p)
+    with pytest.raises(BookLeafError) as e:
+        o.run(6)
+    want = (e.value.ierr, o.ts.nstep)
+    seen = []
+    for tiles in (True, False):
+        g = BookLeaf(p)
+        g.set_tiling(tiles)
+        if want[1] > 1:  # to the step that fails
+            g.run(want[1] - 1, runner="run_graph")
+        before = g.state()
+        with pytest.raises(BookLeafError) as e:
+            g.run(6, runner="run_graph")
+        assert "negative volume" in str(e.value)
+        assert (e.value.ierr, g.ts.nstep) == want
+        after = g.state()
+        assert bool(g.get_tiling()[0]) == tiles
+        same = {k: np.array_equal(before[k], after[k]) for k in ("ndx", "elmass", "cnmass")}
+        assert same == {"predictor": dict(ndx=True, elmass=True, cnmass=True),
+                        "corrector": dict(ndx=False, elmass=True, cnmass=True),
+                        "remap": dict(ndx=False, elmass=False, cnmass=False)}[stage]
+        seen.append(after)
+    names = ["ndx", "ndy", "ndu", "ndv", "eldensity", "elenergy", "elpressure", "elcs2",
+             "elmass", "cnmass", "cnviscx", "cnviscy", "elvisc"]
+    names += ["cpdensity", "cppressure", "cpcs2", "cpvolume", "cpmass"]
+    if stage != "predictor":  # (without tiles they are already the predictor's)
+        names.append("cpenergy")
+    assert diff_fields(seen[0], seen[1], names) == []
+    if mixed:
+        assert np.array_equal(seen[0]["cpenergy"][:p.ncp], o.get("cpenergy")[:p.ncp])
