@@ -1093,7 +1093,7 @@ int bl_init_mesh(bl_handle_t* h) {
     return BL_FAILURE;
   std::vector<int32_t> ielel(4 * (size_t)nel, 0), ielfc(4 * (size_t)nel, 0);
   for (int32_t n : ielnd)
-    if (n < 1 || n > nnd) { set_error("bl_build_maps: ielnd entry out of range"); return BL_FAILURE; }
+    if (n < 1 || n > nnd) { set_error("bl_init_mesh: ielnd entry out of range"); return BL_FAILURE; }
   // face f of element e joins corners f and f+1.  The faces by their smaller
   // node (counted, in (e, f) order), a node's few by the other node: two
   // faces in a row with both nodes alike are neighbours.  (Set-up of 524288

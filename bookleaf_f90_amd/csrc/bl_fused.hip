@@ -27,9 +27,11 @@
 //   F5 end     : errors and the node-set flip, when no later kernel of the
 //                step or the next F1b can record them; F2m, F4m: the mixed
 //                cells' component terms, in F2's and F5's extra workgroups
-//   tile step  : in a Lagrangian step of pure cells, F2, F3 and F4 in one
-//                kernel per tile of elements and the ring around them
-//                (k_lag_tile, bl_tiles.hip)
+//   tile step  : in a Lagrangian step of pure cells and an ALE step with
+//                unsplit advection, F2, F3 and F4 in one kernel per tile of
+//                elements and the ring around them (k_lag_tile,
+//                bl_tiles.hip); the step before's end is recorded by F1L and
+//                dt selected by the tiles or k_select, without F1b and F5
 //   R1..R5     : the remap (ale_dr_*), after the Lagrangian step when ALE is
 //                active; on a tiling the Lagrangian part is the tile step and
 //                the remap two kernels (k_remap_faces, k_remap_tile)
@@ -358,8 +360,7 @@ __device__ __forceinline__ void select_dt(const FusedArgs& A, double dt_prev, in
 // negative volume of the predictor (F2: the nodes were not moved) or of the
 // corrector (F4: they were) stops the batch at that step, as
 // geometry_kn_checkvolume's error halts the reference; a step that moved
-// the nodes wrote the other node set.  Host and device form of the same
-// record (the host runs it for a batch's last step).
+// the nodes wrote the other node set (unless the tiled remap ran after it).
 template <typename TS>
 __device__ __forceinline__ void step_end(TS* ts, const DtResult* res) {
   if (!ts->open) return;
@@ -2044,10 +2045,12 @@ __global__ void __launch_bounds__(kBlock) k_r5(AleArgs B, DevTimestep* tsw) {
 // 306 -> 185 us: the corner terms, fluxes and corner masses that went through
 // HBM between the kernels (about 900 B an element) stay in LDS, and F1 needs
 // no pass of its own.  Bound by latency: four workgroups a CU (37 KB of LDS,
-// at most 128 VGPRs) of dependent gathers and divisions.  Three a CU (45 KB,
-// 167 VGPRs) took 57 us on the mixed Sod against 47 and 84 on the relaxation
-// against 72.  A tiling is used
-// wherever the mesh has one; the eleven kernels remain for meshes without.
+// at most 128 VGPRs: 120 for pure cells; with mixed cells 128 and 8 spilled)
+// of dependent gathers and divisions.  Three a CU (45 KB, 167 VGPRs, none
+// spilled) took 57 us on the mixed Sod against 47 and 84 on the relaxation
+// against 72.  (k_lag_tile before it spills 11 of its 168 with mixed cells, 6
+// when dt is selected in a launch of its own.)  A tiling is used wherever the
+// mesh has one; the eleven kernels remain for meshes without.
 
 // R1's face mass fluxes (and a negative volume of the moved mesh, which R3
 // finds in the five-kernel form).  MIX: the first nbm8 workgroups (whole XCD
@@ -2518,8 +2521,8 @@ bool end_in_f1b(const bl_handle_t* h) {
 }
 
 // the tile step runs a folded Lagrangian step when the mesh has a tiling
-// (bl_tiles.hip) and tiling is on; with per-step diagnostics F5 ends each
-// step and the records follow it
+// (bl_tiles.hip) and tiling is on, also with per-step diagnostics (the
+// record's kernels follow it)
 bool use_tiles(const bl_handle_t* h) {
   return fold_f1(h) && h->tiles_on && h->tile_state == 1;
 }

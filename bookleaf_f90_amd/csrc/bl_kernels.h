@@ -5,8 +5,9 @@
 // picks the FIRST element attaining the maximum, and only if it exceeds TINY
 // (strict '>' scan from TINY, hydro_kn_getdt.f90:104-117).  Both are total
 // orders on (value, index), so a tree reduction in any order returns the
-// same element as the serial scan: wave64 shuffles, then LDS across the
-// waves of the workgroup, then the last workgroup over the partials.
+// same element as the serial scan: register moves across a wave, LDS across
+// the waves of the workgroup, then one workgroup over the partials (a step on
+// a small tiling: every tile).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cfloat>

@@ -811,7 +811,7 @@ k_mlp_train(const float* __restrict__ wr, const float* __restrict__ norm,
   if (live)
     src = drawn ? (int)(mix64(seed ^ mix64(((uint64_t)it << 32) | (uint32_t)s)) % (uint64_t)npairs)
                 : s;
-  // the inputs: a wave loads every fourth column of its lanes' samples
+  // the inputs: a wave loads every eighth column of its lanes' samples
   for (int k = wave; k < kIn; k += kTrainThreads / 64)
     sx[lane][k] = live ? bfr(norm_in(norm, k, feat[(size_t)src * kIn + k])) : 0.0f;
   __syncthreads();
@@ -944,7 +944,7 @@ __device__ __forceinline__ float sum_parts(int nblk, const float* __restrict__ p
   for (; b < nblk; ++b) g = g + part[(size_t)b * stride];
   return g;
 }
-constexpr int kSumBlock = 64;  // a wave a workgroup: 94 workgroups
+constexpr int kSumBlock = 64;  // a wave a workgroup: 95 workgroups
 
 __global__ void __launch_bounds__(kSumBlock)
 k_mlp_reduce(int nblk, const float* __restrict__ part, const float* __restrict__ lpart,

@@ -1,7 +1,9 @@
 // bl_tiles.hip -- the element tiling of the tile step (host side).
 //
-// The tile step fuses the fused step's F2, F3 and F4 for a pure-cell
-// Lagrangian problem: one workgroup owns a tile of elements.  It computes
+// The tile step fuses the fused step's F2, F3 and F4, for a Lagrangian step
+// of pure cells and for the Lagrangian part of an ALE step with unsplit
+// advection, mixed cells included (whose remap then runs on the same tiles,
+// k_remap_tile in bl_fused.hip): one workgroup owns a tile of elements.  It computes
 // the predictor and the corrector corner terms (F2's work, kept in LDS) of
 // its own elements and of the ring of elements around their nodes, sums
 // them for every node of its own elements in the reference's scatter order

@@ -160,7 +160,8 @@ int bl_download(bl_handle_t* h, int32_t id, void* host, int64_t count);
 /* Build the node->corner CSR maps from ielnd, ielsort1, ielsort2 (upload
  * those first).  Two orderings: hydro (corner jj, then element in ielsort1
  * order, hydro_kn_getacceleration.f90:53-72) and ALE (element in ielsort2
- * order, then corner, ale_kn_advect.f90:96-124). */
+ * order, then corner, ale_kn_advect.f90:96-124).  ielel and ielfc may be
+ * uploaded before or after: every table made from them follows an upload. */
 int bl_build_maps(bl_handle_t* h);
 /* Host-side mesh initialisation for hosts that do not run the reference's
  * own init: ielel/ielfc from ielnd (init_kn_connectivity, init_kn.f90:82-91,
@@ -496,17 +497,20 @@ int bl_set_tuning(bl_handle_t* h, const bl_tuning_t* t);
 int bl_get_tuning(bl_handle_t* h, bl_tuning_t* t);
 
 /* The tile step (no counterpart in the reference, which has no kernels to
- * fuse).  A Lagrangian step of a problem with pure cells only and no
- * per-step diagnostics can run its predictor, node update and corrector
- * (the work of hydro_dr_getforce, getstate, getenergy, geteos and the
- * acceleration drivers) as one kernel per tile of about 180 elements and
- * the ring of elements around their nodes, keeping the corner forces and
- * node results in LDS: tiles come from recursive coordinate bisection of
+ * fuse).  A Lagrangian step of a problem with pure cells only, and an ALE step
+ * with unsplit advection (Eulerian or node relaxation, mixed cells included),
+ * can run the predictor, node update and corrector (the work of
+ * hydro_dr_getforce, getstate, getenergy, geteos and the acceleration
+ * drivers) as one kernel per tile of about 180 elements and the ring of
+ * elements around their nodes, keeping the corner forces and node results in
+ * LDS, and the remap (ale_dr_advect, ale_dr_hydroupdate) as a pass of face
+ * fluxes and one more kernel per tile: tiles come from recursive coordinate bisection of
  * the element centroids the first time bl_run_graph needs them after the
  * connectivity was built (bl_build_maps).  The mesh
- * must have no node that is the same corner (1..4) of two elements; a mesh
- * that does runs the three-kernel step.  on = 0 keeps the three-kernel step
- * for every problem.  No result depends on the choice: the sums over a
+ * must have no node that is the same corner (1..4) of two elements, for ALE
+ * also face neighbours that share the face's nodes and boundary faces whose
+ * ielfc is the opposite face; another runs the three-kernel step and the
+ * remap's grid kernels.  on = 0 keeps those for every problem.  No result depends on the choice: the sums over a
  * node's corners stay in the reference's order. */
 int bl_set_tiling(bl_handle_t* h, int32_t on);
 /* whether the next run uses the tile step (as far as known: the tiling is
