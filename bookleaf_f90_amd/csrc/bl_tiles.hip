@@ -38,6 +38,7 @@
 #include <thread>
 #include <vector>
 
+#include "bl_grow.h"
 #include "bl_internal.h"
 #include "bl_tiles.h"
 
@@ -195,6 +196,15 @@ int upload_vec(T** d, const std::vector<T>& v) {
   BL_HIP(hipMalloc(d, sizeof(T) * std::max<size_t>(v.size(), 1)));
   if (!v.empty()) BL_HIP(hipMemcpy(*d, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
   return BL_SUCCESS;
+}
+
+// four partials for each of n workgroups
+template <typename T>
+T* slots_of(int64_t n) {
+  T* p = nullptr;
+  if (hipMalloc(&p, sizeof(T) * 4 * (size_t)n) == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
 }
 
 }  // namespace
@@ -426,15 +436,14 @@ int cut_tiles(Handle* h) {
   h->ntile = ntile;
   h->nentries = ne;
   // the partial slots of the tile step: one per tile
-  if (ntile + 16 > h->npart) {
-    hipFree(h->d_part);
-    hipFree(h->d_parti);
-    h->d_part = nullptr;
-    h->d_parti = nullptr;
-    h->npart = ntile + 16;
-    BL_HIP(hipMalloc(&h->d_part, sizeof(double) * 4 * h->npart));
-    BL_HIP(hipMalloc(&h->d_parti, sizeof(int32_t) * 4 * h->npart));
+  const int64_t need = ntile + 16;
+  int64_t have = h->npart, have_i = h->npart;
+  if (!grow(&h->d_part, &have, need, slots_of<double>, hipFree) ||
+      !grow(&h->d_parti, &have_i, need, slots_of<int32_t>, hipFree)) {
+    set_error("tiles: out of device memory");
+    return BL_FAILURE;
   }
+  h->npart = std::max(h->npart, need);
   // the second element set
   if (!h->elset[0][0]) {
     const int ids[4] = {BL_ELDENSITY, BL_ELENERGY, BL_ELPRESSURE, BL_ELCS2};

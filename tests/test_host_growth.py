@@ -59,3 +59,11 @@ def test_training_grows_its_losses_this_way():
         text = f.read()
     assert "grow(&m->loss" in text
     assert "hipFree(m->loss)" not in text
+
+
+def test_the_tiles_grow_the_partials_this_way():
+    """The drivers' dt reductions write to the partials a tiling may grow."""
+    with open(os.path.join(ROOT, "bookleaf_f90_amd", "csrc", "bl_tiles.hip")) as f:
+        text = f.read()
+    assert "grow(&h->d_part," in text and "grow(&h->d_parti," in text
+    assert "hipFree(h->d_part" not in text
